@@ -6,7 +6,7 @@ disabled (-packed-fp32-ops) for gfx950.
 
 The kernels are templates with many variants, so the library is built from
 several translation units compiled in parallel: the step launches once per
-storage type and dynamics (csrc/step.hip), the other typed operations once
+storage type and dynamics (csrc/step.hip, csrc/fused.hip), the other typed operations once
 per storage type (csrc/storage_ops.hip), the adjoint (csrc/adjoint.hip), the
 allocation-free moments entry point (csrc/noalloc.hip) and the set-up and C ABI
 (csrc/engine.hip). Objects go to palabos_amd/_build/.
@@ -41,6 +41,7 @@ def units():
         out.append((f"ops_{s}", "storage_ops.hip", [f"-DPLBAMD_S={s}"]))
         for dyn in (0, 1):
             out.append((f"step_{s}_{dyn}", "step.hip", [f"-DPLBAMD_S={s}", f"-DPLBAMD_DYN={dyn}"]))
+            out.append((f"fused_{s}_{dyn}", "fused.hip", [f"-DPLBAMD_S={s}", f"-DPLBAMD_DYN={dyn}"]))
     return out
 
 

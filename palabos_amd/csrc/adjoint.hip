@@ -88,19 +88,19 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
         hipFree(gS); hipFree(acc); hipFree(sum); hipFree(dAdjBlock); hipFree(dAdjBegin);
     };
     const uint64_t nAcc = (uint64_t)adjWGs + planeWGs;   // J accumulators: bulk workgroups, then plane ones
-    hipError_t err = hipMalloc(&ck, stateBytes * nCk);
-    if (err == hipSuccess) err = hipMalloc(&work, stateBytes);
-    if (err == hipSuccess) err = hipMalloc(&mom, momElems * (K + 1) * lamSize);
-    if (err == hipSuccess) err = hipMalloc(&pf, pfElems * (K + 1) * sizeof(double));
-    if (err == hipSuccess) err = hipMalloc(&lamA, arenaElems * lamSize);
-    if (err == hipSuccess) err = hipMalloc(&lamB, arenaElems * lamSize);
-    if (err == hipSuccess) err = hipMalloc(&gA, cells * sizeof(double));
-    if (err == hipSuccess && !lam64) err = hipMalloc(&gA32, cells * sizeof(float));
-    if (err == hipSuccess) err = hipMalloc(&gS, std::max<uint32_t>(1, L.nSpecial) * sizeof(double));
-    if (err == hipSuccess) err = hipMalloc(&acc, nAcc * sizeof(double));
-    if (err == hipSuccess) err = hipMalloc(&sum, 8 * sizeof(double));
-    if (err == hipSuccess) err = hipMalloc(&dAdjBlock, adjBlock.size() * sizeof(uint16_t));
-    if (err == hipSuccess) err = hipMalloc(&dAdjBegin, adjBegin.size() * sizeof(uint32_t));
+    hipError_t err = deviceAlloc((void**)&ck, stateBytes * nCk);
+    if (err == hipSuccess) err = deviceAlloc((void**)&work, stateBytes);
+    if (err == hipSuccess) err = deviceAlloc((void**)&mom, momElems * (K + 1) * lamSize);
+    if (err == hipSuccess) err = deviceAlloc((void**)&pf, pfElems * (K + 1) * sizeof(double));
+    if (err == hipSuccess) err = deviceAlloc((void**)&lamA, arenaElems * lamSize);
+    if (err == hipSuccess) err = deviceAlloc((void**)&lamB, arenaElems * lamSize);
+    if (err == hipSuccess) err = deviceAlloc((void**)&gA, cells * sizeof(double));
+    if (err == hipSuccess && !lam64) err = deviceAlloc((void**)&gA32, cells * sizeof(float));
+    if (err == hipSuccess) err = deviceAlloc((void**)&gS, std::max<uint32_t>(1, L.nSpecial) * sizeof(double));
+    if (err == hipSuccess) err = deviceAlloc((void**)&acc, nAcc * sizeof(double));
+    if (err == hipSuccess) err = deviceAlloc((void**)&sum, 8 * sizeof(double));
+    if (err == hipSuccess) err = deviceAlloc((void**)&dAdjBlock, adjBlock.size() * sizeof(uint16_t));
+    if (err == hipSuccess) err = deviceAlloc((void**)&dAdjBegin, adjBegin.size() * sizeof(uint32_t));
     if (err == hipSuccess)
         err = hipMemcpy(dAdjBlock, adjBlock.data(), adjBlock.size() * sizeof(uint16_t), hipMemcpyHostToDevice);
     if (err == hipSuccess)
@@ -136,8 +136,8 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
         ++nKeep;
     }
     if (nKeep > 0) {
-        if (hipMalloc(&keepMom, keepRecs * momElems * lamSize) != hipSuccess ||
-            hipMalloc(&keepPf, keepRecs * pfElems * sizeof(double)) != hipSuccess) {
+        if (deviceAlloc((void**)&keepMom, keepRecs * momElems * lamSize) != hipSuccess ||
+            deviceAlloc((void**)&keepPf, keepRecs * pfElems * sizeof(double)) != hipSuccess) {
             // the budget was not there after all: recompute everything
             (void)hipGetLastError();
             hipFree(keepMom);

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cctype>
 #include <cstdio>
 #include <cstdlib>
@@ -142,7 +143,30 @@ struct Lattice {
     dim3 bulkBlock;
     int zChunk = 0;
 
+    // two steps per launch (fused.h): a second population array that changes
+    // places with the first, the per-cell words and the special cells' records
+    // and first-step outputs. Allocated by the first call that takes the path,
+    // given back when device memory runs short (releaseSpares); spareMutex is held
+    // while a call uses them.
+    struct FusedPlan {
+        int rows = 0, cols = 0, tilesY = 0, tilesZ = 0, len = 0;
+    } fused;
+    std::mutex spareMutex;
+    void* spare = nullptr;
+    uint32_t* dInfo = nullptr;
+    uint32_t* dIndex = nullptr;
+    void* dPre = nullptr;
+    bool anySolid = false;         // link-wall solids
+    bool nodeBesideWall = false;   // and nodes or boundary objects: single steps
+
+    void releaseSpare() {
+        hipFree(spare); hipFree(dInfo); hipFree(dIndex); hipFree(dPre);
+        spare = dPre = nullptr;
+        dInfo = dIndex = nullptr;
+    }
+
     ~Lattice() {
+        releaseSpare();
         hipFree(arena); hipFree(dGeom); hipFree(dTags); hipFree(dSpecial); hipFree(dValues); hipFree(dAlpha);
         hipFree(dBulkPartials); hipFree(dBulkLevel1); hipFree(dSpecialPartials); hipFree(dStats); hipFree(dSegs); hipFree(dSegs1); hipFree(dTasks1);
         hipFree(dWgBlock); hipFree(dTasks); hipFree(dWalls); hipFree(dEvenBlock); hipFree(dProc); hipFree(dExtField);
@@ -161,12 +185,17 @@ struct Recording {
     double* specialF = nullptr;
 };
 
+// hipMalloc that, short of memory, takes back the second arrays of the lattices
+// that no call is using and tries again.
+hipError_t deviceAlloc(void** p, size_t bytes);
+void releaseSpares();
+
 // Device buffers of one call, freed on every return path.
 struct DeviceBuffers {
     std::vector<void*> p;
     void* get(size_t bytes) {
         void* q = nullptr;
-        if (hipMalloc(&q, bytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+        if (deviceAlloc(&q, bytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
         p.push_back(q);
         return q;
     }
@@ -194,6 +223,11 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
 // DYN) in their own translation units.
 template<typename S, int DYN>
 int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record = nullptr);
+// Two fused steps from an odd time on; before them the set-up of L.dInfo (when
+// it is new) and the begin of a call's run of fused steps.
+enum FusedOp { FUSED_PREPARE, FUSED_BEGIN, FUSED_STEPS };
+template<typename S, int DYN>
+int launchFused(Lattice& L, FusedOp op);
 template<typename S>
 int exchange(Lattice& L);
 template<typename S>

@@ -5,6 +5,8 @@
 
 #include <unordered_map>
 
+#include "fused.h"
+
 namespace plbamd {
 
 // Cells up to which the odd steps write their z-moving outputs with ordinary
@@ -32,6 +34,25 @@ Lattice* find(int handle) {
     std::lock_guard<std::mutex> lock(g_mutex);
     auto it = g_lattices.find(handle);
     return it == g_lattices.end() ? nullptr : it->second.get();
+}
+
+void releaseSpares() {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    for (auto& e : g_lattices) {
+        Lattice& L = *e.second;
+        std::unique_lock<std::mutex> use(L.spareMutex, std::try_to_lock);
+        if (!use.owns_lock() || !L.spare) continue;
+        (void)hipStreamSynchronize(L.stream);
+        L.releaseSpare();
+    }
+}
+
+hipError_t deviceAlloc(void** p, size_t bytes) {
+    hipError_t err = hipMalloc(p, bytes);
+    if (err == hipSuccess) return err;
+    (void)hipGetLastError();
+    releaseSpares();
+    return hipMalloc(p, bytes);
 }
 
 bool boxValid(const Lattice& L, const plbamd_box& b) {
@@ -212,7 +233,12 @@ int setup(Lattice& L) {
     for (BlockGeom& g : L.geom) {
         const uint64_t cells = (uint64_t)g.nx * g.ny * g.nz;
         if (cells >= (1ull << 32)) return fail(PLBAMD_EINVAL, "lattice_create: at most 2^32 - 1 cells per block");
-        g.slot = (cells + 63) / 64 * 64;
+        // Slots start an odd number of 64-element runs apart, so that the 19 streams
+        // of a launch do not all start on the same memory channels where the cell
+        // count is a multiple of a large power of two (fused steps, us a step:
+        // FP64 256^3 670 -> 645, FP32 320^3 758 -> 717, FP16 320^3 493 -> 469; single
+        // steps within 1 %).
+        g.slot = (cells + 511) / 512 * 512 + 64;
         g.offset = offset;
         g.cellOffset = cellOffset;
         g.nzChunks = (g.nz + L.zChunk - 1) / L.zChunk;
@@ -250,12 +276,12 @@ int setup(Lattice& L) {
     // kCachedZCells cells (PLBAMD_CACHED_Z=0/1 overrides)
     L.cachedZ = cellOffset <= kCachedZCells;
     if (const char* e = getenv("PLBAMD_CACHED_Z")) L.cachedZ = atoi(e) != 0;
-    if (hipMalloc(&L.arena, bytes) != hipSuccess) {
+    if (deviceAlloc(&L.arena, bytes) != hipSuccess) {
         (void)hipGetLastError();
         return fail(PLBAMD_ENOMEM, "lattice_create: cannot allocate " + std::to_string(bytes) + " bytes");
     }
     PLBAMD_HIP(hipMemset(L.arena, 0, bytes));
-    PLBAMD_HIP(hipMalloc(&L.dGeom, L.geom.size() * sizeof(BlockGeom)));
+    PLBAMD_HIP(deviceAlloc((void**)&L.dGeom, L.geom.size() * sizeof(BlockGeom)));
     PLBAMD_HIP(hipMemcpy(L.dGeom, L.geom.data(), L.geom.size() * sizeof(BlockGeom), hipMemcpyHostToDevice));
     if (L.multi) {
         std::vector<uint16_t> wgBlock(L.nBulkPartials);
@@ -263,21 +289,21 @@ int setup(Lattice& L) {
             const uint64_t end = b + 1 < L.geom.size() ? L.geom[b + 1].wgBegin : L.nBulkPartials;
             std::fill(wgBlock.begin() + L.geom[b].wgBegin, wgBlock.begin() + end, (uint16_t)b);
         }
-        PLBAMD_HIP(hipMalloc(&L.dWgBlock, wgBlock.size() * sizeof(uint16_t)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dWgBlock, wgBlock.size() * sizeof(uint16_t)));
         PLBAMD_HIP(hipMemcpy(L.dWgBlock, wgBlock.data(), wgBlock.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
     }
-    PLBAMD_HIP(hipMalloc(&L.dBulkPartials, std::max(L.nBulkPartials, L.nEven) * 16 * sizeof(double)));
-    PLBAMD_HIP(hipMalloc(&L.dBulkLevel1, kStatsLevel1 * 16 * sizeof(double)));
+    PLBAMD_HIP(deviceAlloc((void**)&L.dBulkPartials, std::max(L.nBulkPartials, L.nEven) * 16 * sizeof(double)));
+    PLBAMD_HIP(deviceAlloc((void**)&L.dBulkLevel1, kStatsLevel1 * 16 * sizeof(double)));
     if (L.multi && L.linearEven) {
         std::vector<uint16_t> eb(L.nEven);
         for (size_t b = 0; b < L.geom.size(); ++b) {
             const uint64_t end = b + 1 < L.geom.size() ? L.geom[b + 1].evenBegin : L.nEven;
             std::fill(eb.begin() + L.geom[b].evenBegin, eb.begin() + end, (uint16_t)b);
         }
-        PLBAMD_HIP(hipMalloc(&L.dEvenBlock, eb.size() * sizeof(uint16_t)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dEvenBlock, eb.size() * sizeof(uint16_t)));
         PLBAMD_HIP(hipMemcpy(L.dEvenBlock, eb.data(), eb.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
     }
-    PLBAMD_HIP(hipMalloc(&L.dStats, 16 * sizeof(double)));
+    PLBAMD_HIP(deviceAlloc((void**)&L.dStats, 16 * sizeof(double)));
     PLBAMD_HIP(hipMemset(L.dStats, 0, 16 * sizeof(double)));
 
     // Envelope segments: the allocated box of block b (or its bulk widened by
@@ -642,7 +668,7 @@ int rebuild(Lattice& L) {
     PLBAMD_TRY(buildProcessors(L, planeOf, boxIndex, special, procs));
     hipFree(L.dProc); L.dProc = nullptr;
     if (!procs.empty()) {
-        PLBAMD_HIP(hipMalloc(&L.dProc, procs.size() * sizeof(ProcCell)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dProc, procs.size() * sizeof(ProcCell)));
         PLBAMD_HIP(hipMemcpy(L.dProc, procs.data(), procs.size() * sizeof(ProcCell), hipMemcpyHostToDevice));
     }
     hipFree(L.dTags); L.dTags = nullptr;
@@ -653,37 +679,160 @@ int rebuild(Lattice& L) {
     hipFree(L.dWalls); L.dWalls = nullptr;
     L.nSpecial = (uint32_t)special.size();
     if (anyNonBulk) {
-        PLBAMD_HIP(hipMalloc(&L.dTags, L.allocCells));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dTags, L.allocCells));
         PLBAMD_HIP(hipMemcpy(L.dTags, dev.data(), L.allocCells, hipMemcpyHostToDevice));
     }
     if (!walls.empty()) {
-        PLBAMD_HIP(hipMalloc(&L.dWalls, walls.size() * sizeof(uint32_t)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dWalls, walls.size() * sizeof(uint32_t)));
         PLBAMD_HIP(hipMemcpy(L.dWalls, walls.data(), walls.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
     if (!special.empty()) {
-        PLBAMD_HIP(hipMalloc(&L.dSpecial, special.size() * sizeof(SpecialCell)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dSpecial, special.size() * sizeof(SpecialCell)));
         PLBAMD_HIP(hipMemcpy(L.dSpecial, special.data(), special.size() * sizeof(SpecialCell), hipMemcpyHostToDevice));
         L.nSpecialPartials = (special.size() + 255) / 256;
-        PLBAMD_HIP(hipMalloc(&L.dSpecialPartials, L.nSpecialPartials * 16 * sizeof(double)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dSpecialPartials, L.nSpecialPartials * 16 * sizeof(double)));
     }
     if (!values.empty()) {
-        PLBAMD_HIP(hipMalloc(&L.dValues, values.size() * sizeof(double)));
+        PLBAMD_HIP(deviceAlloc((void**)&L.dValues, values.size() * sizeof(double)));
         PLBAMD_HIP(hipMemcpy(L.dValues, values.data(), values.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     if (!alpha.empty()) {
         // in the arithmetic type of the storage (FP32 below FP64 storage): the
         // kernels use the porosity converted to it, so the values are the same
         if (L.desc.storage == PLBAMD_F64) {
-            PLBAMD_HIP(hipMalloc(&L.dAlpha, alpha.size() * sizeof(double)));
+            PLBAMD_HIP(deviceAlloc((void**)&L.dAlpha, alpha.size() * sizeof(double)));
             PLBAMD_HIP(hipMemcpy(L.dAlpha, alpha.data(), alpha.size() * sizeof(double), hipMemcpyHostToDevice));
         } else {
             std::vector<float> a32(alpha.begin(), alpha.end());
-            PLBAMD_HIP(hipMalloc(&L.dAlpha, a32.size() * sizeof(float)));
+            PLBAMD_HIP(deviceAlloc((void**)&L.dAlpha, a32.size() * sizeof(float)));
             PLBAMD_HIP(hipMemcpy(L.dAlpha, a32.data(), a32.size() * sizeof(float), hipMemcpyHostToDevice));
         }
     }
+    {
+        // the words of the fused steps follow the tags: built anew by the next call
+        std::lock_guard<std::mutex> use(L.spareMutex);
+        hipFree(L.dInfo); hipFree(L.dIndex); hipFree(L.dPre);
+        L.dInfo = L.dIndex = nullptr;
+        L.dPre = nullptr;
+        bool solid = false, other = L.nSpecial > 0;
+        for (uint8_t t : dev) {
+            solid = solid || t == BT_WALL_NEAR;
+            other = other || t == BT_BOUNCE_BACK || t == BT_NO_DYNAMICS;
+        }
+        for (uint8_t t : L.hostTags) solid = solid || t == PLBAMD_TAG_WALL_LINK;
+        L.anySolid = solid;
+        L.nodeBesideWall = solid && other;
+    }
     L.dirty = false;
     return PLBAMD_OK;
+}
+
+// Tile and chunk of the fused steps: the least of
+//   rounds of workgroups * (planes per workgroup + 2.5) * bytes per plane of a tile.
+// The 2.5 planes are the two that a chunk's ends repeat and the pipeline's start;
+// the bytes are the lines a row of the tile reads, its rim counted at `rim` (most
+// of it hits in L2), and those it writes; rows that do not start on 64-byte
+// boundaries write lines in parts. Against 900 timed combinations of tile and
+// chunk on eleven lattices (64^3 to 384x256x256, 191x203x197 among them) the
+// choice is 0.4 % (FP64) and 4 % (FP32) from the fastest on average, 5 % and
+// 19 % at worst; the fewest tiles alone chose 18x23 cells at 160^3 (FP64 218 us a
+// step; with 10x40 144 us).
+static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size) {
+    const int wgsPerCU = size == 8 ? 1 : 2;     // by registers
+    const double rim = size == 8 ? 0.3 : 0.5, slots = 256.0 * wgsPerCU;
+    const bool rowLines = g.nz * size % 128 == 0;
+    Lattice::FusedPlan best;
+    double least = 1e300;
+    for (int width = 8; width <= 128; width += 2) {
+        const int w = std::min(width, g.nz), tz = (g.nz + w - 1) / w;
+        int rows = kFusedThreads / (w + 2) - 2;
+        const int ty = (g.ny + rows - 1) / rows;
+        rows = (g.ny + ty - 1) / ty;
+        const bool aligned = rowLines && w * size % 64 == 0, lines = rowLines && w * size % 128 == 0;
+        const double row = w * (double)size / 128.0;
+        const double bytes = (rows + 2) * (row + 2 * rim + (aligned ? 0.0 : 0.5)) +
+                             rows * (row + (lines ? 0.0 : aligned ? 0.5 : 1.0) * rim);
+        for (int chunks = 1; chunks <= g.nx; ++chunks) {
+            const int len = (g.nx + chunks - 1) / chunks;
+            const double wgs = (double)ty * tz * ((g.nx + len - 1) / len);
+            const double cost = std::ceil(wgs / slots) * (len + 2.5) * bytes;
+            if (cost >= least) continue;
+            least = cost;
+            best.rows = rows + 2; best.cols = w + 2; best.tilesY = ty; best.tilesZ = tz; best.len = len;
+        }
+        if (w < width) break;
+    }
+    return best;
+}
+
+// Whether the next steps may be taken two at a time (fused.h), with the second
+// array allocated: one block, no boundary processors, no link walls together
+// with nodes, a second array of at most an eighth of the free device memory, and
+// a lattice on which it is the faster way (us a step on periodic n^3 lattices,
+// single -> fused):
+//   FP64 from 64^3 on     64^3 14.4 -> 12.7, 96^3 48.9 -> 31.1, 128^3 97.8 -> 82.6,
+//                         256^3 903 -> 642, 512^3 7357 -> 5325 (48^3 and below: equal)
+//   FP32 from 64^3 on     64^3 9.1 -> 8.0, 128^3 52.4 -> 50.8, 200^3 277 -> 185,
+//                         256^3 445 -> 352, 512^3 3737 -> 2831; not with link walls (their
+//                         reflections cost a tile's workgroup more than the second pass
+//                         over memory: 256x160x128 171 -> 193; FP64 323 -> 270)
+//   16 bits               bound by the arithmetic of two collisions where the pair kernel
+//                         is not (256^3 206 -> 239): below 96^3, in the last-level cache
+//                         (64^3 9.5 -> 7.4, 96^3 16.0 -> 14.4, 112^3 22.2 -> 24.4), and for odd
+//                         nz, which has no pair kernel (191x203x197 225 -> 136); bulk
+//                         cells only
+// Planes and momentum-exchange nodes bring two more small launches: from a
+// million cells on (FP64 channel 192x96x96 108 -> 101, 128x64x64 equal).
+// PLBAMD_FUSED=0/1 overrides the choice.
+static bool fusedReady(Lattice& L) {
+    if (L.multi || L.dProc || L.nodeBesideWall) return false;
+    const BlockGeom& g = L.geom[0];
+    bool wanted = L.cells >= 200000;
+    if (L.nSpecial) wanted = L.cells >= 1000000;
+    if (L.elemSize == 4) wanted = wanted && !L.anySolid;
+    if (L.elemSize == 2) wanted = !L.nSpecial && !L.anySolid && (!L.pairs || L.cells <= 1000000);
+    if (const char* e = getenv("PLBAMD_FUSED")) wanted = atoi(e) != 0;
+    const bool needInfo = L.dTags || !(g.px && g.py && g.pz);
+    // 32-bit lane offsets: within a plane, or (reflections) over ten slots
+    const uint64_t span = (needInfo ? 10 * g.slot : (uint64_t)g.ny * g.nz) * L.elemSize;
+    if (!wanted || span > 0xffffffffull) return false;
+    if (!L.spare) {
+        const uint64_t bytes = 19 * g.slot * L.elemSize;
+        size_t freeB = 0, totalB = 0;
+        if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || bytes > freeB / 8 || hipMalloc(&L.spare, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            L.spare = nullptr;
+            return false;
+        }
+        L.fused = planFused(g, L.elemSize);
+    }
+    if (needInfo && !L.dInfo) {
+        bool ok = hipMalloc(&L.dInfo, L.cells * sizeof(uint32_t)) == hipSuccess;
+        if (ok && L.nSpecial) {
+            ok = hipMalloc(&L.dIndex, L.cells * sizeof(uint32_t)) == hipSuccess &&
+                 hipMalloc(&L.dPre, 19 * (size_t)L.nSpecial * L.elemSize) == hipSuccess;
+        }
+        if (!ok) {
+            (void)hipGetLastError();
+            L.releaseSpare();
+            return false;
+        }
+    }
+    return true;
+}
+
+template<typename S>
+static int fusedStep(Lattice& L, FusedOp op) {
+    return L.desc.dynamics == PLBAMD_BGK ? launchFused<S, 0>(L, op) : launchFused<S, 1>(L, op);
+}
+
+static int fusedDispatch(Lattice& L, FusedOp op) {
+    switch (L.desc.storage) {
+    case PLBAMD_F64: return fusedStep<double>(L, op);
+    case PLBAMD_F32: return fusedStep<float>(L, op);
+    case PLBAMD_F16: return fusedStep<f16s>(L, op);
+    default: return fusedStep<bf16s>(L, op);
+    }
 }
 
 template<typename S>
@@ -694,8 +843,24 @@ int launchStep(Lattice& L, bool odd, bool stats) {
 
 int step(Lattice& L, int nsteps) {
     PLBAMD_TRY(rebuild(L));
+    // steps that need not report statistics, from an odd time on, two at a time
+    std::unique_lock<std::mutex> use(L.spareMutex, std::defer_lock);
+    bool fused = false;
+    if (nsteps - (L.statsOn ? 1 : 0) - (L.time & 1 ? 0 : 1) >= 2) {
+        use.lock();
+        const bool had = L.spare && (L.dInfo || !(L.dTags || !(L.geom[0].px && L.geom[0].py && L.geom[0].pz)));
+        fused = fusedReady(L);
+        if (fused && !had) PLBAMD_TRY(fusedDispatch(L, FUSED_PREPARE));
+        if (fused) PLBAMD_TRY(fusedDispatch(L, FUSED_BEGIN));
+    }
     for (int s = 0; s < nsteps; ++s) {
         const bool odd = (L.time & 1) != 0;
+        if (fused && odd && nsteps - s - (L.statsOn ? 1 : 0) >= 2) {
+            PLBAMD_TRY(fusedDispatch(L, FUSED_STEPS));
+            L.time += 2;
+            ++s;
+            continue;
+        }
         const bool stats = L.statsOn && s == nsteps - 1;
         int rc;
         switch (L.desc.storage) {

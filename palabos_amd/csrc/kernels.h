@@ -1321,6 +1321,8 @@ struct SpecialArgs {
     void* moments;        // or null: pre-collision moments (layout and type of StepArgs::moments)
     uint64_t momStride;
     double* dumpF;        // or null: pre-completion populations, 19 per record
+    void* pre;            // odd steps, or null: the outputs go here ([19][count], storage type) instead of
+                          // streaming (the first of two fused steps, fused.h)
 };
 
 template<typename S, int DYN, bool ODD, bool STATS, bool FORCED>
@@ -1399,6 +1401,10 @@ __global__ void __launch_bounds__(256) special_step(SpecialArgs a) {
         if constexpr (!ODD) {
 #pragma unroll
             for (int i = 0; i < 19; ++i) Store<S>::store(f + (uint64_t)opp(i) * g.slot + cell, fc[i]);
+        } else if (a.pre) {
+            typename Store<S>::R* out = reinterpret_cast<typename Store<S>::R*>(a.pre);
+#pragma unroll
+            for (int i = 0; i < 19; ++i) out[(uint64_t)i * a.count + k] = Store<S>::to_raw(fc[i]);
         } else {
             Store<S>::store(f + cell, fc[0]);
 #pragma unroll

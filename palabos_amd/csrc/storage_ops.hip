@@ -64,7 +64,7 @@ int transfer(Lattice& L, const plbamd_box& b, int elem, void* data, size_t bytes
         return fail(PLBAMD_ESTATE, "upload: a multi-block lattice accepts populations after an even number of steps");
     PLBAMD_TRY(rebuild(L));
     void* staging = nullptr;
-    PLBAMD_HIP(hipMalloc(&staging, bytes));
+    PLBAMD_HIP(deviceAlloc(&staging, bytes));
     hipError_t err = hipSuccess;
     if (up) err = hipMemcpyAsync(staging, data, bytes, hipMemcpyHostToDevice, L.stream);
     if (err == hipSuccess) err = transferDevice<S>(L, b, elem, staging, up);
@@ -184,7 +184,7 @@ int equilibrium(Lattice& L, const plbamd_box& b, const double* rho, const double
         return fail(PLBAMD_ESTATE, "initialize_at_equilibrium: a multi-block lattice accepts populations after an even number of steps");
     PLBAMD_TRY(rebuild(L));
     double* d = nullptr;
-    PLBAMD_HIP(hipMalloc(&d, n * 4 * sizeof(double)));
+    PLBAMD_HIP(deviceAlloc((void**)&d, n * 4 * sizeof(double)));
     hipError_t err = hipMemcpyAsync(d, rho, n * sizeof(double), hipMemcpyHostToDevice, L.stream);
     if (err == hipSuccess) err = hipMemcpyAsync(d + n, u, 3 * n * sizeof(double), hipMemcpyHostToDevice, L.stream);
     for (size_t bi = 0; bi < L.geom.size() && err == hipSuccess; ++bi) {
@@ -235,7 +235,7 @@ int moments(Lattice& L, const plbamd_box& b, double* rho, double* u, double* sum
         dPart = scratch->base;
         dLevel1 = dPart + 8 * scratch->maxRecords;
     } else {
-        PLBAMD_HIP(hipMalloc(&d, (fieldDoubles + analysisDoubles + nRecords * 8 + 8 * level1 + 8) * sizeof(double)));
+        PLBAMD_HIP(deviceAlloc((void**)&d, (fieldDoubles + analysisDoubles + nRecords * 8 + 8 * level1 + 8) * sizeof(double)));
         dPart = d + fieldDoubles + analysisDoubles;
         dLevel1 = dPart + nRecords * 8;
     }
@@ -331,7 +331,7 @@ int externalField(Lattice& L, const plbamd_box& b, double* rhoBar, double* j, in
     using T = typename Store<S>::T;
     PLBAMD_TRY(rebuild(L));
     if (!L.dExtField) {
-        PLBAMD_HIP(hipMalloc(&L.dExtField, 4 * L.allocCells * sizeof(T)));
+        PLBAMD_HIP(deviceAlloc(&L.dExtField, 4 * L.allocCells * sizeof(T)));
         PLBAMD_HIP(hipMemsetAsync(L.dExtField, 0, 4 * L.allocCells * sizeof(T), L.stream));
     }
     T* field = static_cast<T*>(L.dExtField);
