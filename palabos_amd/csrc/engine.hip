@@ -411,7 +411,7 @@ static int copyOp(const Plane& P) {
 // read in the phase that writes it and every pair of touching objects was added
 // in phase order (faces, edges, corners), which this checks.
 int buildProcessors(Lattice& L, const std::vector<int>& planeOf, const std::vector<uint32_t>& boxIndex,
-                    const std::vector<SpecialCell>& special, std::vector<ProcCell>& out) {
+                    const std::vector<SpecialCell>& special, const std::vector<uint32_t>& walls, std::vector<ProcCell>& out) {
     out.clear();
     L.anyCopy = false;
     bool any = false;
@@ -436,12 +436,15 @@ int buildProcessors(Lattice& L, const std::vector<int>& planeOf, const std::vect
         if (P.shape == SHAPE_CORNER) return 3;
         return P.wrapped ? 0 : -1;
     };
+    auto specialRef = [](const SpecialCell& s) {
+        return ProcNb{s.cell, s.value, s.wall, s.x, s.y, s.z, (uint16_t)(s.info | kNbSpecial)};
+    };
     std::string err;
     // what a processor reads of a neighbour: its velocity, or its density and velocity
     enum { READ_U = 1, READ_RHO = 2 };
     // a neighbour of object `owner` in phase `ph`; returns its reference, or fails
     auto neighbour = [&](int owner, int ph, int x, int y, int z, int dx, int dy, int dz, int reads,
-                         uint32_t& ref) -> bool {
+                         ProcNb& ref) -> bool {
         int v[3] = {x + dx, y + dy, z + dz};
         const int n[3] = {nx, ny, nz};
         for (int a = 0; a < 3; ++a) {
@@ -456,7 +459,7 @@ int buildProcessors(Lattice& L, const std::vector<int>& planeOf, const std::vect
                 err = "a boundary processor reads a solid cell";
                 return false;
             }
-            ref = (uint32_t)c;
+            ref = ProcNb{(uint32_t)c, 0u, walls.empty() ? 0u : walls[c], (uint16_t)v[0], (uint16_t)v[1], (uint16_t)v[2], 0};
             return true;
         }
         const uint32_t kind = special[it->second].info & 3u;
@@ -484,7 +487,7 @@ int buildProcessors(Lattice& L, const std::vector<int>& planeOf, const std::vect
                 return false;
             }
         }
-        ref = it->second | kNbSpecial;
+        ref = specialRef(special[it->second]);
         return true;
     };
     for (int p = 0; p < (int)L.planes.size(); ++p) {
@@ -500,7 +503,7 @@ int buildProcessors(Lattice& L, const std::vector<int>& planeOf, const std::vect
                     const uint64_t c = at(x, y, z);
                     if (planeOf[c] != p) continue;
                     ProcCell r{};
-                    r.special = specialAt.at(c);
+                    r.self = specialRef(special[specialAt.at(c)]);
                     for (int a = 0; a < 3; ++a) r.n[a] = (int8_t)n[a];
                     if (op) {
                         const int ph = P.shape == SHAPE_CORNER ? 2 : 0;
@@ -665,7 +668,7 @@ int rebuild(Lattice& L) {
                 }
     }
     std::vector<ProcCell> procs;
-    PLBAMD_TRY(buildProcessors(L, planeOf, boxIndex, special, procs));
+    PLBAMD_TRY(buildProcessors(L, planeOf, boxIndex, special, walls, procs));
     hipFree(L.dProc); L.dProc = nullptr;
     if (!procs.empty()) {
         PLBAMD_HIP(deviceAlloc((void**)&L.dProc, procs.size() * sizeof(ProcCell)));
@@ -689,7 +692,7 @@ int rebuild(Lattice& L) {
     if (!special.empty()) {
         PLBAMD_HIP(deviceAlloc((void**)&L.dSpecial, special.size() * sizeof(SpecialCell)));
         PLBAMD_HIP(hipMemcpy(L.dSpecial, special.data(), special.size() * sizeof(SpecialCell), hipMemcpyHostToDevice));
-        L.nSpecialPartials = (special.size() + 255) / 256;
+        L.nSpecialPartials = (special.size() + kSpecialThreads - 1) / kSpecialThreads;
         PLBAMD_HIP(deviceAlloc((void**)&L.dSpecialPartials, L.nSpecialPartials * 16 * sizeof(double)));
     }
     if (!values.empty()) {

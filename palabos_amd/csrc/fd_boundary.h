@@ -22,9 +22,8 @@
 // writes it and that the phases keep the order of the objects that touch
 // (engine.hip, rebuild), so the results are those of the sequential order.
 //
-// Every neighbour is resolved on the host into a reference: a special record
-// (plane, edge or corner cell) or a plain cell of the block; the neighbour's
-// density and velocity are what its dynamics reports (Cell::computeDensity /
+// Every neighbour is resolved on the host (ProcNb: a plane, edge or corner cell
+// with its stored value, or a plain cell of the block); the neighbour's density and velocity are what its dynamics reports (Cell::computeDensity /
 // computeVelocity), from its populations at the current layout parity. A
 // plane cell of a wrapped factory is read completed, as its own processor
 // leaves it (wrappedLocalBoundaryProcessor3D.hh:41-62).
@@ -43,118 +42,77 @@ enum ProcOp : uint8_t {
     PROC_CORNER = 6,           // OuterVelocityCornerFunctional3D
 };
 
-// Neighbour reference: a special record (flag set) or a block-local cell index.
-constexpr uint32_t kNbSpecial = 0x80000000u;
+// A neighbour as the host resolved it: its position, and of a special cell
+// (plane, edge, corner) its info and stored value.
+struct ProcNb {
+    uint32_t cell;      // block-local
+    uint32_t value;     // special: index of its stored value
+    uint32_t wall;      // link-wall mask
+    uint16_t x, y, z;
+    uint16_t info;      // special: SpecialCell::info with kNbSpecial; 0: a plain cell
+};
+constexpr uint16_t kNbSpecial = 0x8000u;
 
 struct ProcCell {
-    uint32_t special;   // special record of the processed cell (position, block, stored value)
-    uint8_t op;         // ProcOp
-    int8_t n[3];        // outward normal of the boundary (zero along an edge's axis)
-    uint32_t nb[4];     // copies: nb[0] = cell - n
+    ProcNb self;        // the processed cell
+    ProcNb nb[4];       // copies: nb[0] = cell - n
                         // edges: nb[0] = cell - n1 e1, nb[1] = cell - n2 e2 (e1, e2 the axes after the
                         //        edge's axis), nb[2] / nb[3] = cell +- e along the edge
                         // corners: nb[0..2] = cell - n_x e_x, - n_y e_y, - n_z e_z
+    uint8_t op;         // ProcOp
+    int8_t n[3];        // outward normal of the boundary (zero along an edge's axis)
 };
-static_assert(sizeof(ProcCell) == 24, "processor record is 24 bytes");
 
 struct ProcArgs {
     void* arena;
     const BlockGeom* blocks;
-    const SpecialCell* special;
     double* values;          // stored boundary values (velocity: 3, density: 1), rewritten by the copies
-    const uint8_t* tags;     // bulk tags or null
-    const uint32_t* walls;   // link-wall masks or null
     const ProcCell* cells;
     uint32_t begin, end;     // the records of this phase
     int parity;              // layout parity of the state the processors act on
     double omega;
 };
 
-struct NbCell {
-    bool special;
-    SpecialCell sc;          // valid when special
-    int x, y, z;
-    uint64_t cell;
-    uint32_t wall;
-};
-
-__device__ __forceinline__ NbCell resolve_nb(const ProcArgs& a, const BlockGeom& g, uint32_t ref) {
-    NbCell c{};
-    if (ref & kNbSpecial) {
-        c.special = true;
-        c.sc = a.special[ref & ~kNbSpecial];
-        c.x = c.sc.x; c.y = c.sc.y; c.z = c.sc.z;
-        c.cell = c.sc.cell;
-        c.wall = c.sc.wall;
-    } else {
-        c.special = false;
-        c.cell = ref;
-        c.z = (int)(ref % (uint32_t)g.nz);
-        c.y = (int)((ref / (uint32_t)g.nz) % (uint32_t)g.ny);
-        c.x = (int)(ref / ((uint32_t)g.ny * (uint32_t)g.nz));
-        const uint8_t tag = a.tags ? a.tags[g.cellOffset + ref] : (uint8_t)BT_BULK;
-        c.wall = (tag == BT_WALL_NEAR && a.walls) ? a.walls[g.cellOffset + ref] : 0u;
-    }
-    return c;
-}
-
+// What a processor reads of a neighbour, from one load of its populations:
+//   rho  Cell::computeDensity: fullRho of the Dirichlet rhoBar for a plane cell
+//        (boundaryDynamics.hh:640-679, StoreDensityDynamics :229-233),
+//        fullRho(get_rhoBar) otherwise (core/dynamics.hh:278-281, boundaryDynamics.hh:82-87);
+//   u    Cell::computeVelocity: the stored velocity of edge, corner and
+//        velocity-plane cells (boundaryDynamics.hh:324-330), j / rho of a pressure
+//        plane's closure (:776-835), j / rho of the populations otherwise
+//        (compute_uLb, momentTemplates3D.h:138-144, with the sequentially summed rhoBar).
 template<typename S>
-__device__ __forceinline__ void load_nb(const ProcArgs& a, const BlockGeom& g, const NbCell& c,
-                                        typename Store<S>::T f[19]) {
+__device__ __forceinline__ void read_nb(const ProcArgs& a, const BlockGeom& g, const ProcNb& c, bool wantRho, bool wantU,
+                                        typename Store<S>::T& rho, typename Store<S>::T u[3]) {
+    using T = typename Store<S>::T;
+    const bool special = (c.info & kNbSpecial) != 0;
+    const uint32_t kind = c.info & 3u;
+    const bool plane = special && kind == SK_PLANE;
+    const bool stored = special && (kind == SK_STORE_VELOCITY || (plane && ((c.info >> 3) & 1u) == PLBAMD_VELOCITY));
+    const double* v = a.values + c.value;
+    if (wantU && stored) { u[0] = (T)v[0]; u[1] = (T)v[1]; u[2] = (T)v[2]; }
+    if (!wantRho && (!wantU || stored)) return;
+    T f[19];
     const S* base = reinterpret_cast<const S*>(a.arena) + g.offset;
 #pragma unroll
     for (int i = 0; i < 19; ++i)
         f[i] = Store<S>::load(base + pop_index(g, a.parity, c.x, c.y, c.z, i, a.parity ? c.wall : 0u, c.cell));
-}
-
-// Cell::computeDensity of a neighbour: fullRho of the Dirichlet rhoBar for a
-// plane cell (boundaryDynamics.hh:640-679, StoreDensityDynamics :229-233),
-// fullRho(get_rhoBar) otherwise (core/dynamics.hh:278-281, boundaryDynamics.hh:82-87).
-template<typename S>
-__device__ typename Store<S>::T nb_density(const ProcArgs& a, const BlockGeom& g, uint32_t ref) {
-    using T = typename Store<S>::T;
-    const NbCell c = resolve_nb(a, g, ref);
-    T f[19];
-    load_nb<S>(a, g, c, f);
-    if (c.special && (c.sc.info & 3u) == SK_PLANE) {
-        const double* v = a.values + c.sc.value;
-        if ((c.sc.info >> 7) & 1u) complete_plane(f, c.sc.info, v);
-        T rhoBar, u[3];
-        plane_macroscopic_any(f, c.sc.info, v, rhoBar, u);
-        return rhoBar + (T)1;
-    }
-    return rhobar_sum(f) + (T)1;
-}
-
-// Cell::computeVelocity of a neighbour: the stored velocity of edge, corner and
-// velocity-plane cells (boundaryDynamics.hh:324-330), j / rho of a pressure
-// plane's closure (:776-835), j / rho of the populations otherwise (compute_uLb,
-// momentTemplates3D.h:138-144, with the sequentially summed rhoBar).
-template<typename S>
-__device__ void nb_velocity(const ProcArgs& a, const BlockGeom& g, uint32_t ref, typename Store<S>::T u[3]) {
-    using T = typename Store<S>::T;
-    const NbCell c = resolve_nb(a, g, ref);
-    if (c.special) {
-        const uint32_t kind = c.sc.info & 3u;
-        if (kind == SK_STORE_VELOCITY || (kind == SK_PLANE && ((c.sc.info >> 3) & 1u) == PLBAMD_VELOCITY)) {
-            const double* v = a.values + c.sc.value;
-            u[0] = (T)v[0]; u[1] = (T)v[1]; u[2] = (T)v[2];
-            return;
-        }
-    }
-    T f[19];
-    load_nb<S>(a, g, c, f);
-    if (c.special) {
-        const double* v = a.values + c.sc.value;
-        if ((c.sc.info >> 7) & 1u) complete_plane(f, c.sc.info, v);
-        T rhoBar;
-        plane_macroscopic_any(f, c.sc.info, v, rhoBar, u);
+    if (plane) {
+        if ((c.info >> 7) & 1u) complete_plane(f, c.info, v);
+        T rhoBar, w[3];
+        plane_macroscopic_any(f, c.info, v, rhoBar, w);
+        rho = rhoBar + (T)1;
+        if (!stored) { u[0] = w[0]; u[1] = w[1]; u[2] = w[2]; }
         return;
     }
-    T rb, j[3];
-    rhobar_j(f, rb, j);
-    const T ir = inv_rho(rhobar_sum(f));
-    u[0] = j[0] * ir; u[1] = j[1] * ir; u[2] = j[2] * ir;
+    const T rhoBar = rhobar_sum(f);
+    rho = rhoBar + (T)1;
+    if (!stored) {
+        T rb, j[3];
+        rhobar_j(f, rb, j);
+        const T ir = inv_rho(rhoBar);
+        u[0] = j[0] * ir; u[1] = j[1] * ir; u[2] = j[2] * ir;
+    }
 }
 
 // pi from the velocity gradient g[a][b] = d_a u_b and the density
@@ -173,7 +131,7 @@ __device__ __forceinline__ void strain_to_pi(const T g[3][3], T rho, T omega, T 
 // IsoThermalBulkDynamics::regularize (isoThermalDynamics.hh:55-69) with
 // j = rho u and rhoBar = rho - 1, written to the cell's own populations.
 template<typename S>
-__device__ void regularize_store(const ProcArgs& a, const BlockGeom& g, const SpecialCell& sc,
+__device__ __forceinline__ void regularize_store(const ProcArgs& a, const BlockGeom& g, const ProcNb& sc,
                                  typename Store<S>::T rho, const typename Store<S>::T u[3],
                                  const typename Store<S>::T pi[6]) {
     using T = typename Store<S>::T;
@@ -198,73 +156,81 @@ __device__ void regularize_store(const ProcArgs& a, const BlockGeom& g, const Sp
         Store<S>::store(base + pop_index(g, a.parity, sc.x, sc.y, sc.z, i, a.parity ? sc.wall : 0u, sc.cell), f[i]);
 }
 
+// A wavefront per neighbour: what a record reads (up to four neighbours, each a
+// chain of record and population loads and a plane's completion) is under way at
+// once, and the lanes of a wavefront complete planes of one orientation. The
+// first wavefront then combines and writes. kProcRecords: few lanes per
+// wavefront, so that a few hundred records spread over the compute units. (One
+// thread per record went through the neighbours one after the other, seven
+// chains for an edge cell: 30 us a launch whatever the number of records.)
+constexpr int kProcRecords = 16;
 template<typename S>
 __global__ void __launch_bounds__(256) boundary_processors(ProcArgs a) {
     using T = typename Store<S>::T;
-    const uint32_t k = a.begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= a.end) return;
-    const ProcCell p = a.cells[k];
-    const SpecialCell sc = a.special[p.special];
-    const BlockGeom g = a.blocks[sc.block];
+    __shared__ T got[4][4][kProcRecords];
+    const int lane = (int)(threadIdx.x & 63u), q = (int)(threadIdx.x >> 6);
+    const uint32_t k = a.begin + blockIdx.x * kProcRecords + (uint32_t)lane;
+    const bool live = lane < kProcRecords && k < a.end;
+    const BlockGeom g = a.blocks[0];     // single-block lattices only (buildProcessors)
+    const ProcCell& p = a.cells[live ? k : a.begin];
+    const uint8_t op = p.op;
+    if (live && q < (op == PROC_EDGE ? 4 : (op == PROC_CORNER ? 3 : 1))) {
+        const bool wantRho = op == PROC_COPY_DENSITY || (op == PROC_EDGE && q < 2) || op == PROC_CORNER;
+        T r = T(), w[3] = {T(), T(), T()};
+        read_nb<S>(a, g, p.nb[q], wantRho, op != PROC_COPY_DENSITY, r, w);
+        got[q][0][lane] = r;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) got[q][1 + c][lane] = w[c];
+    }
+    __syncthreads();
+    if (!live || q != 0) return;
+    const ProcNb sc = p.self;
     double* v = a.values + sc.value;
     const T omega = (T)a.omega;
-    if (p.op == PROC_COPY_DENSITY) {
-        v[0] = (double)nb_density<S>(a, g, p.nb[0]);
-    } else if (p.op <= PROC_COPY_NORMAL) {
-        T u[3];
-        nb_velocity<S>(a, g, p.nb[0], u);
+    T rho[4], u[4][3];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        rho[n] = got[n][0][lane];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) u[n][c] = got[n][1 + c][lane];
+    }
+    if (op == PROC_COPY_DENSITY) {
+        v[0] = (double)rho[0];
+    } else if (op <= PROC_COPY_NORMAL) {
+        T w[3] = {u[0][0], u[0][1], u[0][2]};
+#pragma unroll
         for (int c = 0; c < 3; ++c) {
-            if (p.op == PROC_COPY_TANGENTIAL && p.n[c] != 0) u[c] = T();
-            if (p.op == PROC_COPY_NORMAL && p.n[c] == 0) u[c] = T();
+            if (op == PROC_COPY_TANGENTIAL && p.n[c] != 0) w[c] = T();
+            if (op == PROC_COPY_NORMAL && p.n[c] == 0) w[c] = T();
         }
-        v[0] = (double)u[0]; v[1] = (double)u[1]; v[2] = (double)u[2];
-    } else if (p.op == PROC_EDGE) {
-        const int plane = p.n[0] == 0 ? 0 : (p.n[1] == 0 ? 1 : 2);
-        const int d1 = (plane + 1) % 3, d2 = (plane + 2) % 3;
-        const T n1 = (T)(-p.n[d1]), n2 = (T)(-p.n[d2]);   // -orientation of the one-sided differences
-        const T rho10 = nb_density<S>(a, g, p.nb[0]);
-        const T rho01 = nb_density<S>(a, g, p.nb[1]);
-        const T rho = (T)0.5 * (rho01 + rho10);
-        const T u0[3] = {(T)v[0], (T)v[1], (T)v[2]};
-        T u10[3], u01[3], up[3], um[3];
-        nb_velocity<S>(a, g, p.nb[0], u10);
-        nb_velocity<S>(a, g, p.nb[1], u01);
-        nb_velocity<S>(a, g, p.nb[2], up);
-        nb_velocity<S>(a, g, p.nb[3], um);
-        T gr[3][3];
+        v[0] = (double)w[0]; v[1] = (double)w[1]; v[2] = (double)w[2];
+    } else {
+        const T self[3] = {(T)v[0], (T)v[1], (T)v[2]};
+        T gr[3][3], r;
+        if (op == PROC_EDGE) {
+            const int plane = p.n[0] == 0 ? 0 : (p.n[1] == 0 ? 1 : 2);
+            const int d1 = (plane + 1) % 3, d2 = (plane + 2) % 3;
+            const T n1 = (T)(-(d1 == 0 ? p.n[0] : d1 == 1 ? p.n[1] : p.n[2]));   // -orientation of the
+            const T n2 = (T)(-(d2 == 0 ? p.n[0] : d2 == 1 ? p.n[1] : p.n[2]));   // one-sided differences
+            r = (T)0.5 * (rho[1] + rho[0]);
 #pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            const T along = (up[b] - um[b]) / (T)2;       // fd::ctl_diff
-            const T g1 = n1 * (-u0[b] + u10[b]);          // -orientation * fd::o1_fwd_diff
-            const T g2 = n2 * (-u0[b] + u01[b]);
+            for (int b = 0; b < 3; ++b) {
+                const T along = (u[2][b] - u[3][b]) / (T)2;      // fd::ctl_diff
+                const T g1 = n1 * (-self[b] + u[0][b]);          // -orientation * fd::o1_fwd_diff
+                const T g2 = n2 * (-self[b] + u[1][b]);
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                if (r == plane) gr[r][b] = along;
-                else if (r == d1) gr[r][b] = g1;
-                else gr[r][b] = g2;
+                for (int c = 0; c < 3; ++c) gr[c][b] = c == plane ? along : (c == d1 ? g1 : g2);
             }
+        } else {   // PROC_CORNER
+            r = (T)1 / (T)3 * (rho[2] + rho[1] + rho[0]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int b = 0; b < 3; ++b) gr[c][b] = (T)(-p.n[c]) * (-self[b] + u[c][b]);
         }
         T pi[6];
-        strain_to_pi(gr, rho, omega, pi);
-        regularize_store<S>(a, g, sc, rho, u0, pi);
-    } else {   // PROC_CORNER
-        const T rho100 = nb_density<S>(a, g, p.nb[0]);
-        const T rho010 = nb_density<S>(a, g, p.nb[1]);
-        const T rho001 = nb_density<S>(a, g, p.nb[2]);
-        const T rho = (T)1 / (T)3 * (rho001 + rho010 + rho100);
-        const T u0[3] = {(T)v[0], (T)v[1], (T)v[2]};
-        T un[3][3];
-        nb_velocity<S>(a, g, p.nb[0], un[0]);
-        nb_velocity<S>(a, g, p.nb[1], un[1]);
-        nb_velocity<S>(a, g, p.nb[2], un[2]);
-        T gr[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int b = 0; b < 3; ++b) gr[r][b] = (T)(-p.n[r]) * (-u0[b] + un[r][b]);
-        T pi[6];
-        strain_to_pi(gr, rho, omega, pi);
-        regularize_store<S>(a, g, sc, rho, u0, pi);
+        strain_to_pi(gr, r, omega, pi);
+        regularize_store<S>(a, g, sc, r, self, pi);
     }
 }
 

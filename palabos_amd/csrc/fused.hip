@@ -47,14 +47,14 @@ int launchFused(Lattice& L, FusedOp op) {
     }
     SpecialArgs s{};
     if (L.nSpecial) {
-        s.arena = L.arena; s.blocks = L.dGeom; s.omega = L.desc.omega;
+        s.arena = L.arena; s.blocks = L.dGeom; s.nBlocks = (int)L.geom.size(); s.omega = L.desc.omega;
         for (int c = 0; c < 3; ++c) s.force[c] = L.desc.force[c];
         s.alpha = L.dAlpha;
         s.cells = L.dSpecial; s.count = L.nSpecial; s.values = L.dValues;
         s.pre = L.dPre;
-        const dim3 sg((L.nSpecial + 255) / 256);
-        if (forced) hipLaunchKernelGGL((special_step<S, DYN, true, false, true>), sg, dim3(256), 0, L.stream, s);
-        else hipLaunchKernelGGL((special_step<S, DYN, true, false, false>), sg, dim3(256), 0, L.stream, s);
+        const dim3 sg((L.nSpecial + kSpecialThreads - 1) / kSpecialThreads);
+        if (forced) hipLaunchKernelGGL((special_step<S, DYN, true, false, true>), sg, dim3(kSpecialThreads), 0, L.stream, s);
+        else hipLaunchKernelGGL((special_step<S, DYN, true, false, false>), sg, dim3(kSpecialThreads), 0, L.stream, s);
     }
     FusedArgs a{};
     a.src = L.arena;
@@ -83,9 +83,9 @@ int launchFused(Lattice& L, FusedOp op) {
     if (L.nSpecial) {
         s.arena = L.spare;
         s.pre = nullptr;
-        const dim3 sg((L.nSpecial + 255) / 256);
-        if (forced) hipLaunchKernelGGL((special_step<S, DYN, false, false, true>), sg, dim3(256), 0, L.stream, s);
-        else hipLaunchKernelGGL((special_step<S, DYN, false, false, false>), sg, dim3(256), 0, L.stream, s);
+        const dim3 sg((L.nSpecial + kSpecialThreads - 1) / kSpecialThreads);
+        if (forced) hipLaunchKernelGGL((special_step<S, DYN, false, false, true>), sg, dim3(kSpecialThreads), 0, L.stream, s);
+        else hipLaunchKernelGGL((special_step<S, DYN, false, false, false>), sg, dim3(kSpecialThreads), 0, L.stream, s);
     }
     PLBAMD_HIP(hipGetLastError());
     std::swap(L.arena, L.spare);

@@ -1310,6 +1310,7 @@ static_assert(sizeof(SpecialCell) == 32, "special record is 32 bytes");
 struct SpecialArgs {
     void* arena;
     const BlockGeom* blocks;
+    int nBlocks;
     double omega;
     double force[3];
     const void* alpha;    // Brinkman porosity per cell (all blocks), in the arithmetic type, or null
@@ -1325,8 +1326,9 @@ struct SpecialArgs {
                           // streaming (the first of two fused steps, fused.h)
 };
 
+constexpr int kSpecialThreads = 64;
 template<typename S, int DYN, bool ODD, bool STATS, bool FORCED>
-__global__ void __launch_bounds__(256) special_step(SpecialArgs a) {
+__global__ void __launch_bounds__(kSpecialThreads) special_step(SpecialArgs a) {
     using T = typename Store<S>::T;
     const T omega = (T)a.omega;
     const T F[3] = {(T)a.force[0], (T)a.force[1], (T)a.force[2]};
@@ -1335,7 +1337,8 @@ __global__ void __launch_bounds__(256) special_step(SpecialArgs a) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < a.count) {
         const SpecialCell sc = a.cells[k];
-        const BlockGeom g = a.blocks[sc.block];
+        // one block: its geometry without waiting for the record
+        const BlockGeom g = a.blocks[a.nBlocks == 1 ? 0 : sc.block];
         S* __restrict__ f = reinterpret_cast<S*>(a.arena) + g.offset;
         const int x = sc.x, y = sc.y, z = sc.z;
         const uint64_t cell = sc.cell;

@@ -155,7 +155,7 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
     PLBAMD_HIP(hipGetLastError());
     if (L.nSpecial) {
         SpecialArgs s{};
-        s.arena = L.arena; s.blocks = L.dGeom; s.omega = L.desc.omega;
+        s.arena = L.arena; s.blocks = L.dGeom; s.nBlocks = (int)L.geom.size(); s.omega = L.desc.omega;
         for (int c = 0; c < 3; ++c) s.force[c] = L.desc.force[c];
         s.alpha = L.dAlpha;
         s.cells = L.dSpecial; s.count = L.nSpecial; s.values = L.dValues;
@@ -165,7 +165,7 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
             s.momStride = record->momStride;
             s.dumpF = record->specialF;
         }
-        dim3 sg((L.nSpecial + 255) / 256), sb(256);
+        const dim3 sg((L.nSpecial + kSpecialThreads - 1) / kSpecialThreads), sb(kSpecialThreads);
 #define PLBAMD_SPECIAL(O, ST, FO) hipLaunchKernelGGL((special_step<S, DYN, O, ST, FO>), sg, sb, 0, L.stream, s)
 #define PLBAMD_SPECIAL_F(O, ST) if (forced) PLBAMD_SPECIAL(O, ST, true); else PLBAMD_SPECIAL(O, ST, false)
         if (odd) {

@@ -306,10 +306,7 @@ int launchProcessors(Lattice& L, int parity) {
     ProcArgs a{};
     a.arena = L.arena;
     a.blocks = L.dGeom;
-    a.special = L.dSpecial;
     a.values = L.dValues;
-    a.tags = L.dTags;
-    a.walls = L.dWalls;
     a.cells = L.dProc;
     a.parity = parity;
     a.omega = L.desc.omega;
@@ -317,7 +314,8 @@ int launchProcessors(Lattice& L, int parity) {
         a.begin = L.procPhase[ph];
         a.end = L.procPhase[ph + 1];
         if (a.end == a.begin) continue;
-        hipLaunchKernelGGL((boundary_processors<S>), dim3((a.end - a.begin + 255) / 256), dim3(256), 0, L.stream, a);
+        hipLaunchKernelGGL((boundary_processors<S>), dim3((a.end - a.begin + kProcRecords - 1) / kProcRecords),
+                           dim3(256), 0, L.stream, a);
         PLBAMD_HIP(hipGetLastError());
     }
     return PLBAMD_OK;
