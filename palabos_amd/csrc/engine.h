@@ -66,8 +66,11 @@ struct Plane {
     int bcType = PLBAMD_BC_DIRICHLET;
 };
 
+struct HostSlots;   // hostio.h
+
 struct Lattice {
     plbamd_lattice_desc desc;
+    std::shared_ptr<HostSlots> hostSlots;   // once a transfer has used them
     int device = -1;                  // HIP device the lattice lives on
     bool multi = false;
     std::vector<plbamd_box> bulk;     // global bulk box of each block
@@ -231,7 +234,7 @@ int launchFused(Lattice& L, FusedOp op);
 template<typename S>
 int exchange(Lattice& L);
 template<typename S>
-hipError_t transferDevice(Lattice& L, const plbamd_box& b, int elem, void* staging, bool up);
+hipError_t transferDevice(Lattice& L, const plbamd_box& b, int elem, void* staging, bool up, hipStream_t stream);
 template<typename S>
 int transfer(Lattice& L, const plbamd_box& b, int elem, void* data, size_t bytes, bool up);
 template<typename S>

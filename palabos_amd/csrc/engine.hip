@@ -6,6 +6,7 @@
 #include <unordered_map>
 
 #include "fused.h"
+#include "hostio.h"
 
 namespace plbamd {
 
@@ -34,6 +35,33 @@ Lattice* find(int handle) {
     std::lock_guard<std::mutex> lock(g_mutex);
     auto it = g_lattices.find(handle);
     return it == g_lattices.end() ? nullptr : it->second.get();
+}
+
+HostSlots::~HostSlots() {
+    for (hipStream_t s : stream) if (s) (void)hipStreamDestroy(s);
+    if (pinned) (void)hipHostFree(pinned);
+}
+
+std::shared_ptr<HostSlots> hostSlots(Lattice& L) {
+    static std::mutex table;
+    static std::map<int, std::weak_ptr<HostSlots>> byDevice;
+    if (L.hostSlots) return L.hostSlots;
+    std::lock_guard<std::mutex> lock(table);
+    std::shared_ptr<HostSlots> s = byDevice[L.device].lock();
+    if (!s) {
+        s = std::make_shared<HostSlots>();
+        s->device = L.device;
+        bool ok = hipHostMalloc((void**)&s->pinned, HostSlots::kSlots * HostSlots::kBytes, hipHostMallocDefault) == hipSuccess &&
+                  !getenv("PLBAMD_NO_PINNED");   // the way without pinned memory, for its test
+        for (hipStream_t& q : s->stream) ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        byDevice[L.device] = s;
+    }
+    L.hostSlots = s;
+    return s;
 }
 
 void releaseSpares() {

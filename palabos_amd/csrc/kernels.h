@@ -1326,6 +1326,10 @@ struct SpecialArgs {
                           // streaming (the first of two fused steps, fused.h)
 };
 
+// 64 threads a workgroup: the cells of a z plane lie nz apart, so that every lane
+// moves its own cache lines and a compute unit takes long over a wavefront; a few
+// thousand cells spread over four times the units (the 3844 lid cells of a 64^3
+// FP64 cavity: even step 22.2 -> 8.9 us, odd 20.8 -> 11.8 us).
 constexpr int kSpecialThreads = 64;
 template<typename S, int DYN, bool ODD, bool STATS, bool FORCED>
 __global__ void __launch_bounds__(kSpecialThreads) special_step(SpecialArgs a) {

@@ -3,6 +3,7 @@
 // initialisation and moments.
 #include "engine.h"
 #include "external.h"
+#include "hostio.h"
 
 #if !defined(PLBAMD_S)
 #error "compile with -DPLBAMD_S=<storage type>"
@@ -23,29 +24,29 @@ int exchange(Lattice& L) {
 // Populations of box b between the lattice and a device buffer of boxCells(b)
 // * 19 elements of type elem, C order; launches only (no host copy, no wait).
 template<typename S>
-hipError_t transferDevice(Lattice& L, const plbamd_box& b, int elem, void* staging, bool up) {
+hipError_t transferDevice(Lattice& L, const plbamd_box& b, int elem, void* staging, bool up, hipStream_t stream) {
     hipError_t err = hipSuccess;
     for (size_t bi = 0; bi < L.geom.size() && err == hipSuccess; ++bi) {
         BoxArgs a;
         if (!boxArgs(L, bi, b, a)) continue;
         const dim3 grid = gridFor((uint64_t)a.ilx * a.ily * a.ilz), block(256);
         if (up) {
-            if (elem == PLBAMD_F64) hipLaunchKernelGGL((upload_box<S, double>), grid, block, 0, L.stream, L.arena, a, (const double*)staging);
-            else if (elem == PLBAMD_F32) hipLaunchKernelGGL((upload_box<S, float>), grid, block, 0, L.stream, L.arena, a, (const float*)staging);
-            else hipLaunchKernelGGL((upload_box_raw<S>), grid, block, 0, L.stream, L.arena, a, (const uint16_t*)staging);
+            if (elem == PLBAMD_F64) hipLaunchKernelGGL((upload_box<S, double>), grid, block, 0, stream, L.arena, a, (const double*)staging);
+            else if (elem == PLBAMD_F32) hipLaunchKernelGGL((upload_box<S, float>), grid, block, 0, stream, L.arena, a, (const float*)staging);
+            else hipLaunchKernelGGL((upload_box_raw<S>), grid, block, 0, stream, L.arena, a, (const uint16_t*)staging);
         } else {
-            if (elem == PLBAMD_F64) hipLaunchKernelGGL((download_box<S, double>), grid, block, 0, L.stream, L.arena, a, (double*)staging);
-            else if (elem == PLBAMD_F32) hipLaunchKernelGGL((download_box<S, float>), grid, block, 0, L.stream, L.arena, a, (float*)staging);
-            else hipLaunchKernelGGL((download_box_raw<S>), grid, block, 0, L.stream, L.arena, a, (uint16_t*)staging);
+            if (elem == PLBAMD_F64) hipLaunchKernelGGL((download_box<S, double>), grid, block, 0, stream, L.arena, a, (double*)staging);
+            else if (elem == PLBAMD_F32) hipLaunchKernelGGL((download_box<S, float>), grid, block, 0, stream, L.arena, a, (float*)staging);
+            else hipLaunchKernelGGL((download_box_raw<S>), grid, block, 0, stream, L.arena, a, (uint16_t*)staging);
             err = hipGetLastError();
             if (err == hipSuccess && L.anyWrapped && L.nSpecial) {
                 const dim3 g2 = gridFor(L.nSpecial);
                 if (elem == PLBAMD_F64)
-                    hipLaunchKernelGGL((complete_download<S, double>), g2, block, 0, L.stream, L.arena, a, L.dValues, (double*)staging, 0);
+                    hipLaunchKernelGGL((complete_download<S, double>), g2, block, 0, stream, L.arena, a, L.dValues, (double*)staging, 0);
                 else if (elem == PLBAMD_F32)
-                    hipLaunchKernelGGL((complete_download<S, float>), g2, block, 0, L.stream, L.arena, a, L.dValues, (float*)staging, 0);
+                    hipLaunchKernelGGL((complete_download<S, float>), g2, block, 0, stream, L.arena, a, L.dValues, (float*)staging, 0);
                 else
-                    hipLaunchKernelGGL((complete_download<S, float>), g2, block, 0, L.stream, L.arena, a, L.dValues, (float*)staging, 1);
+                    hipLaunchKernelGGL((complete_download<S, float>), g2, block, 0, stream, L.arena, a, L.dValues, (float*)staging, 1);
             }
         }
         if (err == hipSuccess) err = hipGetLastError();
@@ -63,16 +64,15 @@ int transfer(Lattice& L, const plbamd_box& b, int elem, void* data, size_t bytes
     if (up && L.multi && (L.time & 1))
         return fail(PLBAMD_ESTATE, "upload: a multi-block lattice accepts populations after an even number of steps");
     PLBAMD_TRY(rebuild(L));
-    void* staging = nullptr;
-    PLBAMD_HIP(deviceAlloc(&staging, bytes));
-    hipError_t err = hipSuccess;
-    if (up) err = hipMemcpyAsync(staging, data, bytes, hipMemcpyHostToDevice, L.stream);
-    if (err == hipSuccess) err = transferDevice<S>(L, b, elem, staging, up);
-    if (err == hipSuccess && up && exchange<S>(L) != PLBAMD_OK) err = hipErrorUnknown;
-    if (err == hipSuccess && !up) err = hipMemcpyAsync(data, staging, bytes, hipMemcpyDeviceToHost, L.stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(L.stream);
-    hipFree(staging);
-    if (err != hipSuccess) return fail(PLBAMD_EHIP, std::string("transfer: ") + hipGetErrorString(err));
+    PLBAMD_HIP(hipStreamSynchronize(L.stream));
+    const HostPart part{static_cast<char*>(data), 19 * hostElem};
+    PLBAMD_TRY(hostTransfer(L, b, &part, 1, up, [&](const plbamd_box& k, void* const* staged, hipStream_t stream) {
+        return transferDevice<S>(L, k, elem, staged[0], up, stream);
+    }));
+    if (up && L.multi) {
+        PLBAMD_TRY(exchange<S>(L));
+        PLBAMD_HIP(hipStreamSynchronize(L.stream));
+    }
     return PLBAMD_OK;
 }
 
@@ -103,7 +103,7 @@ int checkpointTyped(Lattice& L, const char* path, int elem, bool force, bool enf
     if (save) {
         // cells in no block are zeros, as the reference's forward ordering writes them
         PLBAMD_HIP(hipMemsetAsync(pops, 0, cells * 19 * sizeof(T), L.stream));
-        PLBAMD_HIP(transferDevice<S>(L, whole, elem, pops, false));
+        PLBAMD_HIP(transferDevice<S>(L, whole, elem, pops, false, L.stream));
         if (force) hipLaunchKernelGGL((append_force<T>), itemsGrid(cells), dim3(256), 0, L.stream, pops, rec, cells, fx, fy, fz);
         hipLaunchKernelGGL(base64_encode, itemsGrid(dataBytes / kB64Bytes + 1), dim3(256), 0, L.stream,
                            reinterpret_cast<const uint8_t*>(rec), dataBytes, text);
@@ -165,7 +165,7 @@ int checkpointTyped(Lattice& L, const char* path, int elem, bool force, bool enf
     PLBAMD_HIP(hipStreamSynchronize(L.stream));
     if (flags[0]) return fail(PLBAMD_EINVAL, "load_binary_block: the cell data is not base64");
     if (flags[1]) return fail(PLBAMD_EINVAL, "load_binary_block: the force externals differ from the lattice's force");
-    PLBAMD_HIP(transferDevice<S>(L, whole, elem, pops, true));
+    PLBAMD_HIP(transferDevice<S>(L, whole, elem, pops, true, L.stream));
     PLBAMD_TRY(exchange<S>(L));
     PLBAMD_HIP(hipStreamSynchronize(L.stream));
     return PLBAMD_OK;
@@ -179,32 +179,31 @@ int checkpoint(Lattice& L, const char* path, int elem, bool force, bool enforceU
 
 template<typename S>
 int equilibrium(Lattice& L, const plbamd_box& b, const double* rho, const double* u) {
-    const uint64_t n = boxCells(b);
     if (L.multi && (L.time & 1))
         return fail(PLBAMD_ESTATE, "initialize_at_equilibrium: a multi-block lattice accepts populations after an even number of steps");
     PLBAMD_TRY(rebuild(L));
-    double* d = nullptr;
-    PLBAMD_HIP(deviceAlloc((void**)&d, n * 4 * sizeof(double)));
-    hipError_t err = hipMemcpyAsync(d, rho, n * sizeof(double), hipMemcpyHostToDevice, L.stream);
-    if (err == hipSuccess) err = hipMemcpyAsync(d + n, u, 3 * n * sizeof(double), hipMemcpyHostToDevice, L.stream);
-    for (size_t bi = 0; bi < L.geom.size() && err == hipSuccess; ++bi) {
-        BoxArgs a;
-        if (!boxArgs(L, bi, b, a)) continue;
-        hipLaunchKernelGGL((equilibrium_box<S>), gridFor((uint64_t)a.ilx * a.ily * a.ilz), dim3(256), 0, L.stream,
-                           L.arena, a, d, d + n);
-        err = hipGetLastError();
+    PLBAMD_HIP(hipStreamSynchronize(L.stream));
+    const HostPart parts[2] = {{reinterpret_cast<char*>(const_cast<double*>(rho)), 8},
+                               {reinterpret_cast<char*>(const_cast<double*>(u)), 24}};
+    PLBAMD_TRY(hostTransfer(L, b, parts, 2, true, [&](const plbamd_box& k, void* const* staged, hipStream_t stream) {
+        for (size_t bi = 0; bi < L.geom.size(); ++bi) {
+            BoxArgs a;
+            if (!boxArgs(L, bi, k, a)) continue;
+            hipLaunchKernelGGL((equilibrium_box<S>), gridFor((uint64_t)a.ilx * a.ily * a.ilz), dim3(256), 0, stream,
+                               L.arena, a, (const double*)staged[0], (const double*)staged[1]);
+        }
+        return hipGetLastError();
+    }));
+    if (L.multi) {
+        PLBAMD_TRY(exchange<S>(L));
+        PLBAMD_HIP(hipStreamSynchronize(L.stream));
     }
-    if (err == hipSuccess && exchange<S>(L) != PLBAMD_OK) err = hipErrorUnknown;
-    if (err == hipSuccess) err = hipStreamSynchronize(L.stream);
-    hipFree(d);
-    if (err != hipSuccess) return fail(PLBAMD_EHIP, std::string("equilibrium: ") + hipGetErrorString(err));
     return PLBAMD_OK;
 }
 
 template<typename S>
 int moments(Lattice& L, const plbamd_box& b, double* rho, double* u, double* sums, double* fields,
             const MomentsScratch* scratch) {
-    const uint64_t n = boxCells(b);
     if (scratch) {
         if (rho || u || fields) return fail(PLBAMD_EINVAL, "moments: a fixed scratch takes the sums only");
         if (L.dirty)
@@ -213,16 +212,45 @@ int moments(Lattice& L, const plbamd_box& b, double* rho, double* u, double* sum
     } else {
         PLBAMD_TRY(rebuild(L));
     }
-    uint64_t nRecords = 0;
     const bool planes = L.nSpecial > 0 && L.dValues != nullptr;
+    MomentsArgs m{};
+    m.tags = L.dTags;
+    m.values = L.dValues;
+    for (int c = 0; c < 3; ++c) m.force[c] = L.desc.force[c];
+    m.forced = L.desc.force[0] != 0 || L.desc.force[1] != 0 || L.desc.force[2] != 0;
+    for (int k = 0; k < 3; ++k) m.solidRho[k] = L.solidRho[k];
+    if (!sums) {
+        // per-cell values only, straight into the host's chunks
+        PLBAMD_HIP(hipStreamSynchronize(L.stream));
+        const HostPart parts[3] = {{reinterpret_cast<char*>(rho), 8}, {reinterpret_cast<char*>(u), 24},
+                                   {reinterpret_cast<char*>(fields), 56}};
+        return hostTransfer(L, b, parts, 3, false, [&](const plbamd_box& k, void* const* staged, hipStream_t stream) {
+            MomentsArgs mk = m;
+            mk.fields = (double*)staged[2];
+            for (size_t bi = 0; bi < L.geom.size(); ++bi) {
+                BoxArgs a;
+                if (!boxArgs(L, bi, k, a)) continue;
+                const dim3 grid = gridFor((uint64_t)a.ilx * a.ily * a.ilz);
+                if (a.parity)
+                    hipLaunchKernelGGL((moments_box<S, 1>), grid, dim3(256), 0, stream, L.arena, a, mk, (double*)staged[0],
+                                       (double*)staged[1], (double*)nullptr);
+                else
+                    hipLaunchKernelGGL((moments_box<S, 0>), grid, dim3(256), 0, stream, L.arena, a, mk, (double*)staged[0],
+                                       (double*)staged[1], (double*)nullptr);
+                if (planes)
+                    hipLaunchKernelGGL((moments_planes<S>), gridFor(L.nSpecial), dim3(256), 0, stream, L.arena, a, mk,
+                                       (double*)staged[0], (double*)staged[1], (double*)nullptr);
+            }
+            return hipGetLastError();
+        });
+    }
+    uint64_t nRecords = 0;
     for (size_t bi = 0; bi < L.geom.size(); ++bi) {
         BoxArgs a;
         if (!boxArgs(L, bi, b, a)) continue;
         nRecords += gridFor((uint64_t)a.ilx * a.ily * a.ilz).x;
         if (planes) nRecords += gridFor(L.nSpecial).x;
     }
-    const size_t fieldDoubles = (rho || u) ? n * 4 : 0;
-    const size_t analysisDoubles = fields ? n * 7 : 0;
     // records reduced in two levels when there are many: kMomentsLevel1 workgroups, then one
     const uint32_t level1 = nRecords > 4096 ? kMomentsLevel1 : 0u;
     double* d = nullptr;
@@ -235,21 +263,12 @@ int moments(Lattice& L, const plbamd_box& b, double* rho, double* u, double* sum
         dPart = scratch->base;
         dLevel1 = dPart + 8 * scratch->maxRecords;
     } else {
-        PLBAMD_HIP(deviceAlloc((void**)&d, (fieldDoubles + analysisDoubles + nRecords * 8 + 8 * level1 + 8) * sizeof(double)));
-        dPart = d + fieldDoubles + analysisDoubles;
+        PLBAMD_HIP(deviceAlloc((void**)&d, (nRecords * 8 + 8 * level1 + 8) * sizeof(double)));
+        dPart = d;
         dLevel1 = dPart + nRecords * 8;
     }
-    double* dRho = rho ? d : nullptr;
-    double* dU = u ? d + n : nullptr;
-    double* dFields = fields ? d + fieldDoubles : nullptr;
+    double* const none = nullptr;
     double* dSum = dLevel1 + 8 * (scratch ? kMomentsLevel1 : level1);
-    MomentsArgs m{};
-    m.tags = L.dTags;
-    m.values = L.dValues;
-    for (int c = 0; c < 3; ++c) m.force[c] = L.desc.force[c];
-    m.forced = L.desc.force[0] != 0 || L.desc.force[1] != 0 || L.desc.force[2] != 0;
-    m.fields = dFields;
-    for (int k = 0; k < 3; ++k) m.solidRho[k] = L.solidRho[k];
     hipError_t err = hipSuccess;
     uint64_t rec = 0;
     for (size_t bi = 0; bi < L.geom.size(); ++bi) {
@@ -257,15 +276,15 @@ int moments(Lattice& L, const plbamd_box& b, double* rho, double* u, double* sum
         if (!boxArgs(L, bi, b, a)) continue;
         const dim3 grid = gridFor((uint64_t)a.ilx * a.ily * a.ilz);
         if (a.parity)
-            hipLaunchKernelGGL((moments_box<S, 1>), grid, dim3(256), 0, L.stream, L.arena, a, m, dRho, dU, dPart + rec * 8);
+            hipLaunchKernelGGL((moments_box<S, 1>), grid, dim3(256), 0, L.stream, L.arena, a, m, none, none, dPart + rec * 8);
         else
-            hipLaunchKernelGGL((moments_box<S, 0>), grid, dim3(256), 0, L.stream, L.arena, a, m, dRho, dU, dPart + rec * 8);
+            hipLaunchKernelGGL((moments_box<S, 0>), grid, dim3(256), 0, L.stream, L.arena, a, m, none, none, dPart + rec * 8);
         rec += grid.x;
         err = hipGetLastError();
         if (err != hipSuccess) break;
         if (planes) {
             const dim3 pg = gridFor(L.nSpecial);
-            hipLaunchKernelGGL((moments_planes<S>), pg, dim3(256), 0, L.stream, L.arena, a, m, dRho, dU, dPart + rec * 8);
+            hipLaunchKernelGGL((moments_planes<S>), pg, dim3(256), 0, L.stream, L.arena, a, m, none, none, dPart + rec * 8);
             rec += pg.x;
             err = hipGetLastError();
             if (err != hipSuccess) break;
@@ -281,21 +300,15 @@ int moments(Lattice& L, const plbamd_box& b, double* rho, double* u, double* sum
         err = hipGetLastError();
     }
     double host[8];
-    if (err == hipSuccess && rho) err = hipMemcpyAsync(rho, dRho, n * sizeof(double), hipMemcpyDeviceToHost, L.stream);
-    if (err == hipSuccess && u) err = hipMemcpyAsync(u, dU, 3 * n * sizeof(double), hipMemcpyDeviceToHost, L.stream);
-    if (err == hipSuccess && fields)
-        err = hipMemcpyAsync(fields, dFields, 7 * n * sizeof(double), hipMemcpyDeviceToHost, L.stream);
     if (err == hipSuccess) err = hipMemcpyAsync(host, dSum, sizeof(host), hipMemcpyDeviceToHost, L.stream);
     if (err == hipSuccess) err = hipStreamSynchronize(L.stream);
     if (d) hipFree(d);
     if (err != hipSuccess) return fail(PLBAMD_EHIP, std::string("moments: ") + hipGetErrorString(err));
-    if (sums) {
-        sums[0] = host[0];  // sum of rhoBar
-        sums[1] = host[1];  // sum of |u|^2
-        sums[2] = host[3];  // sum of u
-        sums[3] = host[4];
-        sums[4] = host[5];
-    }
+    sums[0] = host[0];  // sum of rhoBar
+    sums[1] = host[1];  // sum of |u|^2
+    sums[2] = host[3];  // sum of u
+    sums[3] = host[4];
+    sums[4] = host[5];
     return PLBAMD_OK;
 }
 
@@ -335,7 +348,6 @@ int externalField(Lattice& L, const plbamd_box& b, double* rhoBar, double* j, in
     T* field = static_cast<T*>(L.dExtField);
     BoxArgs a;
     if (!boxArgs(L, 0, b, a)) return fail(PLBAMD_EINVAL, "rhobar_j: box outside the lattice");
-    const uint64_t n = boxCells(b);
     const dim3 grid = gridFor((uint64_t)a.ilx * a.ily * a.ilz);
     if (op == 0) {
         if (a.parity)
@@ -348,23 +360,20 @@ int externalField(Lattice& L, const plbamd_box& b, double* rhoBar, double* j, in
         PLBAMD_HIP(hipStreamSynchronize(L.stream));
         return PLBAMD_OK;
     }
-    DeviceBuffers buf;
-    double* d = static_cast<double*>(buf.get(4 * n * sizeof(double)));
-    if (!d) return fail(PLBAMD_ENOMEM, "rhobar_j: staging allocation");
-    if (op == 1) {
-        hipLaunchKernelGGL((field_get<T>), grid, dim3(256), 0, L.stream, a, (const T*)field, L.allocCells, d, d + n);
-        PLBAMD_HIP(hipGetLastError());
-        PLBAMD_HIP(hipMemcpyAsync(rhoBar, d, n * sizeof(double), hipMemcpyDeviceToHost, L.stream));
-        PLBAMD_HIP(hipMemcpyAsync(j, d + n, 3 * n * sizeof(double), hipMemcpyDeviceToHost, L.stream));
-    } else {
-        PLBAMD_HIP(hipMemcpyAsync(d, rhoBar, n * sizeof(double), hipMemcpyHostToDevice, L.stream));
-        PLBAMD_HIP(hipMemcpyAsync(d + n, j, 3 * n * sizeof(double), hipMemcpyHostToDevice, L.stream));
-        hipLaunchKernelGGL((field_set<T>), grid, dim3(256), 0, L.stream, a, field, L.allocCells,
-                           (const double*)d, (const double*)(d + n));
-        PLBAMD_HIP(hipGetLastError());
-    }
     PLBAMD_HIP(hipStreamSynchronize(L.stream));
-    return PLBAMD_OK;
+    const HostPart parts[2] = {{reinterpret_cast<char*>(rhoBar), 8}, {reinterpret_cast<char*>(j), 24}};
+    return hostTransfer(L, b, parts, 2, op == 2, [&](const plbamd_box& k, void* const* staged, hipStream_t stream) {
+        BoxArgs c;
+        (void)boxArgs(L, 0, k, c);
+        const dim3 g = gridFor((uint64_t)c.ilx * c.ily * c.ilz);
+        if (op == 1)
+            hipLaunchKernelGGL((field_get<T>), g, dim3(256), 0, stream, c, (const T*)field, L.allocCells,
+                               (double*)staged[0], (double*)staged[1]);
+        else
+            hipLaunchKernelGGL((field_set<T>), g, dim3(256), 0, stream, c, field, L.allocCells,
+                               (const double*)staged[0], (const double*)staged[1]);
+        return hipGetLastError();
+    });
 }
 
 // nsteps ExternalRhoJcollideAndStream3D steps with the field as it is.
@@ -398,7 +407,7 @@ template int externalField<PLBAMD_S>(Lattice&, const plbamd_box&, double*, doubl
 template int externalSteps<PLBAMD_S>(Lattice&, int);
 template int launchProcessors<PLBAMD_S>(Lattice&, int);
 template int exchange<PLBAMD_S>(Lattice&);
-template hipError_t transferDevice<PLBAMD_S>(Lattice&, const plbamd_box&, int, void*, bool);
+template hipError_t transferDevice<PLBAMD_S>(Lattice&, const plbamd_box&, int, void*, bool, hipStream_t);
 template int transfer<PLBAMD_S>(Lattice&, const plbamd_box&, int, void*, size_t, bool);
 template int checkpoint<PLBAMD_S>(Lattice&, const char*, int, bool, bool, bool);
 template int equilibrium<PLBAMD_S>(Lattice&, const plbamd_box&, const double*, const double*);
