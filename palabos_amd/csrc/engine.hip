@@ -11,7 +11,7 @@
 namespace plbamd {
 
 // Cells up to which the odd steps write their z-moving outputs with ordinary
-// stores (bulk_odd_staged and bulk_pairs CACHEDZ). Measured on periodic n^3
+// stores (cache policy 1 of the step kernels). Measured on periodic n^3
 // lattices (step time, nontemporal -> ordinary): FP64 128^3 -9 %, 224^3 -6 %,
 // 384^3 -1.4 %, 512^3 +1.5 %; FP32 192^3 -11 %, 384^3 -0.6 %, 512^3 +2 %;
 // FP16 192^3 -7 %, 256^3 -7 %, 384^3 -1.4 %, 512^3 +1.8 %: the turn lies
@@ -19,6 +19,8 @@ namespace plbamd {
 // 256x128x128 -10 % (FP32) and -11 % (FP64); the 384x256x256 porous medium
 // (FP16) -3 %.
 constexpr uint64_t kCachedZCells = uint64_t(1) << 26;
+// Populations up to which the loads are ordinary too (policy 2; figures in kernels.h).
+constexpr uint64_t kCachedBytes = 256000000;
 
 thread_local std::string g_lastError;
 
@@ -301,9 +303,10 @@ int setup(Lattice& L) {
     L.elemSize = storageSize(d.storage);
     const size_t bytes = offset * L.elemSize;
     // ordinary stores for the odd steps' z-moving outputs on lattices of at most
-    // kCachedZCells cells (PLBAMD_CACHED_Z=0/1 overrides)
-    L.cachedZ = cellOffset <= kCachedZCells;
-    if (const char* e = getenv("PLBAMD_CACHED_Z")) L.cachedZ = atoi(e) != 0;
+    // kCachedZCells cells, ordinary loads up to kCachedBytes of populations
+    // (PLBAMD_CACHED_Z=0/1/2 overrides)
+    L.policy = bytes <= kCachedBytes ? 2 : (cellOffset <= kCachedZCells ? 1 : 0);
+    if (const char* e = getenv("PLBAMD_CACHED_Z")) L.policy = std::max(0, std::min(2, atoi(e)));
     if (deviceAlloc(&L.arena, bytes) != hipSuccess) {
         (void)hipGetLastError();
         return fail(PLBAMD_ENOMEM, "lattice_create: cannot allocate " + std::to_string(bytes) + " bytes");
@@ -799,36 +802,44 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size) {
 // Whether the next steps may be taken two at a time (fused.h), with the second
 // array allocated: one block, no boundary processors, no link walls together
 // with nodes, a second array of at most an eighth of the free device memory, and
-// a lattice on which it is the faster way (us a step on periodic n^3 lattices,
-// single -> fused):
-//   FP64 from 64^3 on     64^3 14.4 -> 12.7, 96^3 48.9 -> 31.1, 128^3 97.8 -> 82.6,
-//                         256^3 903 -> 642, 512^3 7357 -> 5325 (48^3 and below: equal)
-//   FP32 from 64^3 on     64^3 9.1 -> 8.0, 128^3 52.4 -> 50.8, 200^3 277 -> 185,
-//                         256^3 445 -> 352, 512^3 3737 -> 2831; not with link walls (their
-//                         reflections cost a tile's workgroup more than the second pass
-//                         over memory: 256x160x128 171 -> 193; FP64 323 -> 270)
-//   16 bits               bound by the arithmetic of two collisions where the pair kernel
-//                         is not (256^3 206 -> 239): below 96^3, in the last-level cache
-//                         (64^3 9.5 -> 7.4, 96^3 16.0 -> 14.4, 112^3 22.2 -> 24.4), and for odd
-//                         nz, which has no pair kernel (191x203x197 225 -> 136); bulk
-//                         cells only
-// Planes and momentum-exchange nodes bring two more small launches: from a
-// million cells on (FP64 channel 192x96x96 108 -> 101, 128x64x64 equal).
+// a lattice on which it is the faster way. us a step on n^3 lattices, single ->
+// fused, with each side's cache policy:
+//   FP64   periodic 64^3 12.9 -> 12.6, 72^3 19.1 -> 16.4, 96^3 40.6 -> 30.7, 112^3 64.3 -> 62.5,
+//          128^3 96.7 -> 82.7, 256^3 903 -> 642, 512^3 7357 -> 5325; with edges 64^3 13.5 ->
+//          15.0, 72^3 19.7 -> 18.7, 160^3 218 -> 148; link walls 256x160x128 323 -> 270
+//   FP32   periodic 64^3 7.7 -> 7.9, 72^3 12.9 -> 9.7, 112^3 29.8 -> 25.8, 128^3 40.3 -> 50.7 and
+//          144^3 63.9 -> 65.7 (one array fits the last-level cache, two do not), 160^3 102 ->
+//          88, 256^3 445 -> 352, 512^3 3737 -> 2831; with edges 96^3 22.4 -> 22.4, 144^3 71.7
+//          -> 75.0, 160^3 103.5 -> 98.2, 192^3 183 -> 164; not with link walls, whose
+//          reflections cost a tile more than the second pass over memory (256x160x128
+//          171 -> 193)
+//   16 bit bound by the arithmetic of two collisions where the pair kernel is not
+//          (256^3 206 -> 239): periodic lattices in the last-level cache (64^3 10.1 -> 7.3,
+//          80^3 13.7 -> 11.0, 96^3 14.4 -> 14.4), and odd nz, which has no pair kernel
+//          (191x203x197 225 -> 136)
+// Planes and momentum-exchange nodes bring two more small launches, which single
+// steps of small lattices do without (bulk_and_special): FP64 channel 128x64x64
+// 31.1 -> 40.2, cavity 96^3 64.4 -> 56.6, channel 192x96x96 107 -> 100.
 // PLBAMD_FUSED=0/1 overrides the choice.
 static bool fusedReady(Lattice& L) {
     if (L.multi || L.dProc || L.nodeBesideWall) return false;
     const BlockGeom& g = L.geom[0];
-    bool wanted = L.cells >= 200000;
-    if (L.nSpecial) wanted = L.cells >= 1000000;
-    if (L.elemSize == 4) wanted = wanted && !L.anySolid;
-    if (L.elemSize == 2) wanted = !L.nSpecial && !L.anySolid && (!L.pairs || L.cells <= 1000000);
-    if (const char* e = getenv("PLBAMD_FUSED")) wanted = atoi(e) != 0;
     const bool needInfo = L.dTags || !(g.px && g.py && g.pz);
+    const uint64_t bytes = 19 * g.slot * L.elemSize;
+    bool wanted;
+    if (L.elemSize == 8) {
+        wanted = L.cells >= (L.nSpecial ? 700000u : needInfo ? 370000u : 250000u);
+    } else if (L.elemSize == 4) {
+        wanted = !L.anySolid && (needInfo ? bytes >= 260000000u
+                                          : L.cells >= 300000 && !(bytes > 128000000u && bytes < 230000000u));
+    } else {
+        wanted = !L.anySolid && (!L.pairs || (!needInfo && L.cells <= 600000));
+    }
+    if (const char* e = getenv("PLBAMD_FUSED")) wanted = atoi(e) != 0;
     // 32-bit lane offsets: within a plane, or (reflections) over ten slots
     const uint64_t span = (needInfo ? 10 * g.slot : (uint64_t)g.ny * g.nz) * L.elemSize;
     if (!wanted || span > 0xffffffffull) return false;
     if (!L.spare) {
-        const uint64_t bytes = 19 * g.slot * L.elemSize;
         size_t freeB = 0, totalB = 0;
         if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || bytes > freeB / 8 || hipMalloc(&L.spare, bytes) != hipSuccess) {
             (void)hipGetLastError();

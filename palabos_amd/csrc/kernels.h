@@ -158,6 +158,30 @@ __device__ __forceinline__ S* at(S* base, uint32_t byteOffset) {
     return reinterpret_cast<S*>(reinterpret_cast<char*>(base) + byteOffset);
 }
 
+// Cache policy of a step kernel (chosen per lattice in setup):
+//   0  nontemporal loads and stores
+//   1  ordinary stores for the odd steps' z-moving outputs
+//   2  and ordinary loads: the lattice stays in the last-level cache between steps
+// With 2, us a step on periodic n^3 lattices (nontemporal loads -> ordinary): FP64
+// 64^3 14.3 -> 12.9, 96^3 49.1 -> 40.5, 128^3 98.5 -> 95.6, 160^3 216 -> 248; FP32 96^3
+// 26.2 -> 21.7, 128^3 52.1 -> 40.3, 160^3 105 -> 102, 256^3 442 -> 493; FP16 112^3 22.1 -> 18.3,
+// 200^3 109 -> 98, 256^3 207 -> 229: from about 320 MB of populations on, the lines
+// that ordinary loads leave push out others to no use.
+template<typename S, bool PLAIN>
+__device__ __forceinline__ typename Store<S>::R ld_raw(const S* p) {
+    if constexpr (PLAIN) return *reinterpret_cast<const typename Store<S>::R*>(p);
+    else return Store<S>::load_raw(p);
+}
+template<bool PLAIN>
+__device__ __forceinline__ uint32_t ld_pair(const void* p) {
+    if constexpr (PLAIN) return *reinterpret_cast<const uint32_t*>(p);
+    else return __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
+}
+template<typename S, bool PLAIN>
+__device__ __forceinline__ typename Store<S>::T ld(const S* p) {
+    return Store<S>::from_raw(ld_raw<S, PLAIN>(p));
+}
+
 // ---------------------------------------------------------------------------
 // Bulk kernel. One launch covers every block: a workgroup takes one segment
 // of zChunk cells of a row (x, y) of one block (TY rows when the row is
@@ -325,10 +349,9 @@ __device__ __forceinline__ void store_bulk_stats(double st[8], const double wf[3
     }
 }
 
-template<typename S, int DYN, bool ODD, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false>
-__global__ void __launch_bounds__(512) bulk_step(StepArgs a) {
+template<typename S, int DYN, bool ODD, bool TAGS, bool STATS, bool FORCED, bool MOMENTS, bool PLAIN>
+__device__ __forceinline__ void bulk_step_body(const StepArgs& a, uint32_t wg) {
     using T = typename Store<S>::T;
-    const uint32_t wg = a.xcdRemap ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x;
     const int b = block_of(a, wg);
     const BlockGeom g = a.blocks[b];
     S* __restrict__ f = reinterpret_cast<S*>(a.arena) + g.offset;
@@ -387,18 +410,18 @@ __global__ void __launch_bounds__(512) bulk_step(StepArgs a) {
             T fc[19];
             if constexpr (!ODD) {
 #pragma unroll
-                for (int i = 0; i < 19; ++i) fc[i] = Store<S>::load(at(rows[1][1] + (uint64_t)i * g.slot, zb[1]));
+                for (int i = 0; i < 19; ++i) fc[i] = ld<S, PLAIN>(at(rows[1][1] + (uint64_t)i * g.slot, zb[1]));
                 if constexpr (TAGS) {
                     if (tag == BT_SKIP) continue;
                 }
             } else if (fast) {
 #pragma unroll
                 for (int i = 0; i < 19; ++i)
-                    fc[i] = Store<S>::load(at(rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot, zb[1 - cz(i)]));
+                    fc[i] = ld<S, PLAIN>(at(rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot, zb[1 - cz(i)]));
             } else {
                 const int zs[3] = {zm, z, zp};
                 const bool vz[3] = {vzm, true, vzp};
-                fc[0] = Store<S>::load(f + cell);
+                fc[0] = ld<S, PLAIN>(f + cell);
 #pragma unroll
                 for (int i = 1; i < 19; ++i) {
                     const int ax = 1 - cx(i), ay = 1 - cy(i), az = 1 - cz(i);
@@ -406,7 +429,7 @@ __global__ void __launch_bounds__(512) bulk_step(StepArgs a) {
                     const uint64_t src = ok ? (uint64_t)opp(i) * g.slot +
                                                   (((uint64_t)xs[ax] * g.ny + ys[ay]) * g.nz + zs[az])
                                             : (uint64_t)i * g.slot + cell;
-                    fc[i] = Store<S>::load(f + src);
+                    fc[i] = ld<S, PLAIN>(f + src);
                 }
             }
 
@@ -439,6 +462,11 @@ __global__ void __launch_bounds__(512) bulk_step(StepArgs a) {
     store_bulk_stats<STATS, FORCED>(st, wf, a.partials, wg, a.walls);
 }
 
+template<typename S, int DYN, bool ODD, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false, bool PLAIN = false>
+__global__ void __launch_bounds__(512) bulk_step(StepArgs a) {
+    bulk_step_body<S, DYN, ODD, TAGS, STATS, FORCED, MOMENTS, PLAIN>(a, a.xcdRemap ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // Even step over a block's cells in memory order. The even step is local (each
 // cell reads and writes only its own slots), so a workgroup takes a run of
@@ -446,7 +474,7 @@ __global__ void __launch_bounds__(512) bulk_step(StepArgs a) {
 // block's rows are short. 16-bit storage moves two cells per thread with
 // 32-bit pair accesses (every block's cell count is even then).
 
-template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false>
+template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false, bool PLAIN = false>
 __global__ void __launch_bounds__(512) bulk_even_linear(StepArgs a) {
     using T = typename Store<S>::T;
     constexpr int CPT = sizeof(typename Store<S>::R) == 2 ? 2 : 1;
@@ -463,13 +491,13 @@ __global__ void __launch_bounds__(512) bulk_even_linear(StepArgs a) {
         if constexpr (CPT == 2) {
 #pragma unroll
             for (int i = 0; i < 19; ++i) {
-                const uint32_t v = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(f + (uint64_t)i * g.slot + c0));
+                const uint32_t v = ld_pair<PLAIN>(f + (uint64_t)i * g.slot + c0);
                 fc[0][i] = Store<S>::from_raw((uint16_t)(v & 0xffffu));
                 fc[1][i] = Store<S>::from_raw((uint16_t)(v >> 16));
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 19; ++i) fc[0][i] = Store<S>::load(f + (uint64_t)i * g.slot + c0);
+            for (int i = 0; i < 19; ++i) fc[0][i] = ld<S, PLAIN>(f + (uint64_t)i * g.slot + c0);
         }
         bool comp[CPT];
 #pragma unroll
@@ -532,7 +560,7 @@ __global__ void __launch_bounds__(512) bulk_even_linear(StepArgs a) {
 // Rows at a non-periodic x/y edge of the block take the per-lane general path.
 
 // One cell of an odd step by per-lane neighbour tests (rows at block edges).
-template<typename S, int DYN, bool STATS, bool FORCED, bool MOMENTS>
+template<typename S, int DYN, bool STATS, bool FORCED, bool MOMENTS, bool PLAIN>
 __device__ __forceinline__ void odd_cell_general(const StepArgs& a, const BlockGeom& g, S* f, int z, uint64_t cell,
                                                  uint8_t tag, bool inBulk, const int xs[3], const int ys[3],
                                                  const bool vx[3], const bool vy[3], double st[8], uint32_t wall,
@@ -543,14 +571,14 @@ __device__ __forceinline__ void odd_cell_general(const StepArgs& a, const BlockG
     const int zs[3] = {zm, z, zp};
     const bool vz[3] = {vzm, true, vzp};
     T fc[19];
-    fc[0] = Store<S>::load(f + cell);
+    fc[0] = ld<S, PLAIN>(f + cell);
 #pragma unroll
     for (int i = 1; i < 19; ++i) {
         const int ax = 1 - cx(i), ay = 1 - cy(i), az = 1 - cz(i);
         const bool ok = vx[ax] && vy[ay] && vz[az] && !((wall >> opp(i)) & 1u);
         const uint64_t src = ok ? (uint64_t)opp(i) * g.slot + (((uint64_t)xs[ax] * g.ny + ys[ay]) * g.nz + zs[az])
                                 : (uint64_t)i * g.slot + cell;
-        fc[i] = Store<S>::load(f + src);
+        fc[i] = ld<S, PLAIN>(f + src);
     }
     collide_cell<S, DYN, STATS, FORCED, MOMENTS>(a, g, cell, tag, inBulk, fc, st, wall, wf);
     Store<S>::store(f + cell, fc[0]);
@@ -588,23 +616,16 @@ __device__ __forceinline__ void zdir(int m, int& dir, int& k) {
     }
 }
 
-// FP32 statistics variants without forcing: asking for 7 waves per SIMD keeps
-// them at 72 VGPRs (2-6 spilled; 99 unconstrained, 4 waves), which the
-// short-row lattices need (one 128-lane workgroup per row): the sphere
-// channel's FP32 odd step with statistics took 131 us at 6 waves (79 VGPRs, no
-// spills) and takes 126 us at 7. Every other instantiation is unconstrained
-// (1 = the default).
-//
-// CACHEDZ: the z-moving outputs (staged rows, halo elements, row-end
+// POLICY 1, 2: the z-moving outputs (staged rows, halo elements, row-end
 // reflections) are written with ordinary stores instead of nontemporal ones.
 // Chosen for lattices small enough that those lines can stay in the device's
 // last-level cache until the next step reads them (the lines that two
 // workgroups write in parts also merge there).
-template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false, bool CACHEDZ = false>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
-    (sizeof(S) == 4 && STATS && !FORCED) ? 7 : 1))) bulk_odd_staged(StepArgs a) {
+template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, bool MOMENTS, int POLICY>
+__device__ __forceinline__ void bulk_odd_staged_body(const StepArgs& a, uint32_t wg) {
     using T = typename Store<S>::T;
     using R = typename Store<S>::R;
+    constexpr bool PLAIN = POLICY == 2;
     // LDS words of at least 32 bits: 16-bit values would put two lanes on one bank word
     using L = typename std::conditional<(sizeof(R) < 4), uint32_t, R>::type;
     extern __shared__ __align__(16) unsigned char ldsRaw[];
@@ -615,7 +636,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     // send along c_i (its link-wall mask; all bits when it is not collided here)
     uint32_t* blocked = reinterpret_cast<uint32_t*>(ldsRaw + (size_t)kZMoving * P * sizeof(L));
 
-    const uint32_t wg = a.xcdRemap ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x;
     const int b = block_of(a, wg);
     const BlockGeom g = a.blocks[b];
     S* __restrict__ f = reinterpret_cast<S*>(a.arena) + g.offset;
@@ -660,7 +680,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         // outermost envelope layer of a block are skipped: nothing they would write
         // reaches the bulk, and the envelope exchange after this step replaces them.
         if (compute && !outer_envelope_row(g, x, y))
-            odd_cell_general<S, DYN, STATS, FORCED, MOMENTS>(a, g, f, z, cell, tag, inBulk, xs, ys, vx, vy, st, wall, wf);
+            odd_cell_general<S, DYN, STATS, FORCED, MOMENTS, PLAIN>(a, g, f, z, cell, tag, inBulk, xs, ys, vx, vy, st, wall, wf);
     } else {
         S* rows[3][3];
 #pragma unroll
@@ -686,8 +706,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int i = 0; i < 19; ++i) {
             const S* src = rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot;
-            if (cz(i) == 0) fc[i] = Store<S>::load(src + zc);
-            else raw[zmove_index(i)] = Store<S>::load_raw(src + zc);
+            if (cz(i) == 0) fc[i] = ld<S, PLAIN>(src + zc);
+            else raw[zmove_index(i)] = ld_raw<S, PLAIN>(src + zc);
         }
         if constexpr (TAGS) {
             // a link wall at x - c_i: f_i comes back from the cell's own slot i
@@ -695,7 +715,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
             if (wall) {
 #pragma unroll
                 for (int i = 0; i < 19; ++i)
-                    if (cz(i) == 0 && ((wall >> opp(i)) & 1u)) fc[i] = Store<S>::load(f + (uint64_t)i * g.slot + cell);
+                    if (cz(i) == 0 && ((wall >> opp(i)) & 1u)) fc[i] = ld<S, PLAIN>(f + (uint64_t)i * g.slot + cell);
             }
         }
         if constexpr (TAGS) {
@@ -704,7 +724,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
             if (compute && wall) {
 #pragma unroll
                 for (int i = 0; i < 19; ++i)
-                    if (cz(i) != 0 && ((wall >> opp(i)) & 1u)) fc[i] = Store<S>::load(f + (uint64_t)i * g.slot + cell);
+                    if (cz(i) != 0 && ((wall >> opp(i)) & 1u)) fc[i] = ld<S, PLAIN>(f + (uint64_t)i * g.slot + cell);
             }
         }
         // Non-periodic row ends: the edge cell's five inputs from beyond the end
@@ -721,7 +741,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
             zdir<1>(t, eDir, eK);
             zdir<-1>(t - 5, dHi, kHi);
             if (hiEdge) { eDir = dHi; eK = kHi; }
-            eVal = Store<S>::load_raw(f + (uint64_t)eDir * g.slot + rowBase + (loEdge ? z0 : z0 + len - 1));
+            eVal = ld_raw<S, PLAIN>(f + (uint64_t)eDir * g.slot + rowBase + (loEdge ? z0 : z0 + len - 1));
         }
         // Halo elements inside a periodic or segmented row: the source elements
         // beyond the segment ends.
@@ -732,7 +752,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int i = 0; i < 19; ++i)
                 if (cz(i) != 0)
-                    halo[zmove_index(i)] = Store<S>::load_raw(rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot + zh);
+                    halo[zmove_index(i)] = ld_raw<S, PLAIN>(rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot + zh);
         }
         if (active) {
 #pragma unroll
@@ -784,7 +804,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         // 3. aligned stores of the z-moving destination rows; position q takes the
         // output of cell q - c_z when that cell is in this segment and was computed
         auto storeZ = [](S* p, R v) {
-            if constexpr (CACHEDZ) Store<S>::store_raw_cached(p, v);
+            if constexpr (POLICY >= 1) Store<S>::store_raw_cached(p, v);
             else Store<S>::store_raw(p, v);
         };
 #pragma unroll
@@ -829,6 +849,19 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     store_bulk_stats<STATS, FORCED>(st, wf, a.partials, wg, a.walls);
 }
 
+// FP32 statistics variants without forcing: asking for 7 waves per SIMD keeps
+// them at 72 VGPRs (2-6 spilled; 99 unconstrained, 4 waves), which the
+// short-row lattices need (one 128-lane workgroup per row): the sphere
+// channel's FP32 odd step with statistics took 131 us at 6 waves (79 VGPRs, no
+// spills) and takes 126 us at 7. Every other instantiation is unconstrained
+// (1 = the default).
+template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false, int POLICY = 0>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
+    (sizeof(S) == 4 && STATS && !FORCED) ? 7 : 1))) bulk_odd_staged(StepArgs a) {
+    bulk_odd_staged_body<S, DYN, TAGS, STATS, FORCED, MOMENTS, POLICY>(
+        a, a.xcdRemap ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // 16-bit storage, two cells per thread. A thread owns the cell pair (z, z+1),
 // z even, and moves both 16-bit values of a slot with one aligned 32-bit
@@ -840,9 +873,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 // kernel. Requires nz even for every block. Rows at a non-periodic x/y edge
 // take the per-cell general path.
 
-__device__ __forceinline__ uint32_t ld_pair(const void* p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
-}
 __device__ __forceinline__ void st_pair(void* p, uint32_t v) {
     __builtin_nontemporal_store(v, reinterpret_cast<uint32_t*>(p));
 }
@@ -857,13 +887,14 @@ __device__ __forceinline__ uint32_t pack16(uint16_t lo, uint16_t hi) { return (u
 // 2W cells of one row and the row is wavefront-uniform. ZWRAP: every block is
 // periodic along z (no z edge: the edge handling is compiled out, which keeps
 // the kernel within 80 registers).
-// CACHEDZ (odd steps): ordinary stores for the z-moving rows, the single halves
-// and the reflections, as bulk_odd_staged's CACHEDZ.
+// POLICY (odd steps 1, 2): ordinary stores for the z-moving rows, the single
+// halves and the reflections, as in bulk_odd_staged.
 template<typename S, int DYN, bool ODD, bool TAGS, bool STATS, bool FORCED, bool MOMENTS = false, bool PACKED = false,
-         bool ZWRAP = false, bool CACHEDZ = false>
+         bool ZWRAP = false, int POLICY = 0>
 __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
     static_assert(sizeof(typename Store<S>::R) == 2, "pairs of 16-bit values");
     using T = typename Store<S>::T;
+    constexpr bool PLAIN = POLICY == 2;
     extern __shared__ __align__(16) unsigned char ldsRaw[];
     const int W = (int)blockDim.x;            // threads per workgroup
     // pitch in pair words per staged direction: per segment a low halo word, the
@@ -946,7 +977,7 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
         if (active) {
 #pragma unroll
             for (int i = 0; i < 19; ++i) {
-                const uint32_t v = ld_pair(own + (uint64_t)i * g.slot);
+                const uint32_t v = ld_pair<PLAIN>(own + (uint64_t)i * g.slot);
                 fa[i] = Store<S>::from_raw(lo16(v));
                 fb[i] = Store<S>::from_raw(hi16(v));
             }
@@ -986,10 +1017,10 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
         // envelope layer is not collided: see bulk_odd_staged)
         if (rowOk && !allValid && !outer_envelope_row(g, x, y)) {
                 if (compA)
-                odd_cell_general<S, DYN, STATS, FORCED, MOMENTS>(a, g, f, zA, cellA, tagA, inBulkA, xs, ys, vx, vy, st,
+                odd_cell_general<S, DYN, STATS, FORCED, MOMENTS, PLAIN>(a, g, f, zA, cellA, tagA, inBulkA, xs, ys, vx, vy, st,
                                                                  wallA, wf);
             if (compB)
-                odd_cell_general<S, DYN, STATS, FORCED, MOMENTS>(a, g, f, zB, cellB, tagB, inBulkB, xs, ys, vx, vy, st,
+                odd_cell_general<S, DYN, STATS, FORCED, MOMENTS, PLAIN>(a, g, f, zB, cellB, tagB, inBulkB, xs, ys, vx, vy, st,
                                                                  wallB, wf);
         }
         // staged rows. Unpacked, the row is workgroup-uniform; packed, every thread
@@ -1021,11 +1052,11 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
                 for (int i = 0; i < 19; ++i) {
                     const S* src = rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot;
                     if (cz(i) == 0) {
-                        const uint32_t v = ld_pair(src + zc);
+                        const uint32_t v = ld_pair<PLAIN>(src + zc);
                         fa[i] = Store<S>::from_raw(lo16(v));
                         fb[i] = Store<S>::from_raw(hi16(v));
                     } else {
-                        raw[zmove_index(i)] = ld_pair(src + zc);
+                        raw[zmove_index(i)] = ld_pair<PLAIN>(src + zc);
                     }
                 }
             }
@@ -1041,7 +1072,7 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
                     for (int i = 0; i < 19; ++i) {
                         if (cz(i) != 0) continue;
                         if (((wallA | wallB) >> opp(i)) & 1u) {
-                            const uint32_t v = ld_pair(f + (uint64_t)i * g.slot + cellA);
+                            const uint32_t v = ld_pair<PLAIN>(f + (uint64_t)i * g.slot + cellA);
                             if ((wallA >> opp(i)) & 1u) fa[i] = Store<S>::from_raw(lo16(v));
                             if ((wallB >> opp(i)) & 1u) fb[i] = Store<S>::from_raw(hi16(v));
                         }
@@ -1058,7 +1089,7 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
                 for (int i = 0; i < 19; ++i) {
                     if (cz(i) == 0) continue;
                     if (sAct && (((wallA | wallB) >> opp(i)) & 1u))
-                        wref[zmove_index(i)] = ld_pair(f + (uint64_t)i * g.slot + cellA);
+                        wref[zmove_index(i)] = ld_pair<PLAIN>(f + (uint64_t)i * g.slot + cellA);
                 }
             }
             // Halo words. Inside a periodic or segmented row: the source pairs beyond
@@ -1080,7 +1111,7 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
                     if (cz(i) != 0) {
                         const S* src = edge ? f + rowBase + (uint64_t)i * g.slot
                                             : rows[1 - cx(i)][1 - cy(i)] + (uint64_t)opp(i) * g.slot;
-                        const uint32_t v = ld_pair(src + zh);
+                        const uint32_t v = ld_pair<PLAIN>(src + zh);
                         halo[zmove_index(i)] = !edge ? v : (loEdge ? (v << 16) : (v >> 16));
                     }
             }
@@ -1158,17 +1189,17 @@ __global__ void __launch_bounds__(512) bulk_pairs(StepArgs a) {
                                    g.cellOffset + cellA);
             // outputs: aligned directions to HBM, z-moving ones to LDS. PL: a plain
             // wavefront (or no tags): every active cell collided here, no walls.
-            // reflections and z-moving rows: nontemporal, or ordinary (CACHEDZ)
+            // reflections and z-moving rows: nontemporal, or ordinary (POLICY)
             auto storeZ = [](S* p, T v) {
-                if constexpr (CACHEDZ) Store<S>::store_raw_cached(p, Store<S>::to_raw(v));
+                if constexpr (POLICY >= 1) Store<S>::store_raw_cached(p, Store<S>::to_raw(v));
                 else Store<S>::store(p, v);
             };
             auto storeRawZ = [](S* p, uint16_t v) {
-                if constexpr (CACHEDZ) Store<S>::store_raw_cached(p, v);
+                if constexpr (POLICY >= 1) Store<S>::store_raw_cached(p, v);
                 else Store<S>::store_raw(p, v);
             };
             auto storePairZ = [](S* p, uint32_t v) {
-                if constexpr (CACHEDZ) *reinterpret_cast<uint32_t*>(p) = v;
+                if constexpr (POLICY >= 1) *reinterpret_cast<uint32_t*>(p) = v;
                 else st_pair(p, v);
             };
             auto emitOutputs = [&](auto plainTag) {
@@ -1332,14 +1363,14 @@ struct SpecialArgs {
 // FP64 cavity: even step 22.2 -> 8.9 us, odd 20.8 -> 11.8 us).
 constexpr int kSpecialThreads = 64;
 template<typename S, int DYN, bool ODD, bool STATS, bool FORCED>
-__global__ void __launch_bounds__(kSpecialThreads) special_step(SpecialArgs a) {
+__device__ __forceinline__ void special_body(const SpecialArgs& a, uint32_t wg) {
     using T = typename Store<S>::T;
     const T omega = (T)a.omega;
     const T F[3] = {(T)a.force[0], (T)a.force[1], (T)a.force[2]};
     double st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     double sp[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < a.count) {
+    const uint32_t k = wg * kSpecialThreads + threadIdx.x;
+    if (threadIdx.x < kSpecialThreads && k < a.count) {
         const SpecialCell sc = a.cells[k];
         // one block: its geometry without waiting for the record
         const BlockGeom g = a.blocks[a.nBlocks == 1 ? 0 : sc.block];
@@ -1426,9 +1457,31 @@ __global__ void __launch_bounds__(kSpecialThreads) special_step(SpecialArgs a) {
         }
     }
     if constexpr (STATS) {
-        block_reduce_store(st, a.partials + 16 * (uint64_t)blockIdx.x);
-        block_reduce_store(sp, a.partials + 16 * (uint64_t)blockIdx.x + 8);
+        block_reduce_store(st, a.partials + 16 * (uint64_t)wg);
+        block_reduce_store(sp, a.partials + 16 * (uint64_t)wg + 8);
     }
+}
+
+template<typename S, int DYN, bool ODD, bool STATS, bool FORCED>
+__global__ void __launch_bounds__(kSpecialThreads) special_step(SpecialArgs a) {
+    special_body<S, DYN, ODD, STATS, FORCED>(a, blockIdx.x);
+}
+
+// Bulk and special cells of a tagged lattice in one launch (they touch disjoint
+// slots): the first nSpecial workgroups take the special cells, the others the
+// bulk rows as bulk_step (even) or bulk_odd_staged. The kernel has the special
+// cells' registers, two wavefronts per SIMD in FP64, so it is for lattices of so
+// few wavefronts that the second launch costs more than the occupancy.
+template<typename S, int DYN, bool ODD, bool STATS, bool FORCED, bool MOMENTS>
+__global__ void __launch_bounds__(512) bulk_and_special(StepArgs a, SpecialArgs s, uint32_t nSpecial) {
+    if (blockIdx.x < nSpecial) {
+        if (blockIdx.x * kSpecialThreads < s.count) special_body<S, DYN, ODD, STATS, FORCED>(s, blockIdx.x);
+        return;
+    }
+    const uint32_t n = gridDim.x - nSpecial, b = blockIdx.x - nSpecial;
+    const uint32_t wg = a.xcdRemap ? xcd_item(b, n) : b;
+    if constexpr (ODD) bulk_odd_staged_body<S, DYN, true, STATS, FORCED, MOMENTS, 2>(a, wg);
+    else bulk_step_body<S, DYN, false, true, STATS, FORCED, MOMENTS, true>(a, wg);
 }
 
 // Final statistics reduction: one workgroup, fixed order. out[0..7]:

@@ -9,6 +9,12 @@
 
 namespace plbamd {
 
+// Rows up to which the special cells go into the bulk launch (us a step, two
+// launches -> one): FP64 cavity 32^3 16.4 -> 10.3, 64^3 (4096 rows) 27.3 -> 21.9, 96^3
+// (9216) 70.7 -> 67.4, 128^3 (16384) 131.2 -> 131.0; FP32 64^3 21.2 -> 15.4, 96^3 47.2 -> 44.5,
+// 128^3 83.4 -> 85.5.
+constexpr uint64_t kTogetherRows = 12288;
+
 template<typename S, int DYN>
 int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
     StepArgs a{};
@@ -29,7 +35,46 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
     const bool tags = L.dTags != nullptr;
     const dim3 grid((unsigned)L.nBulkPartials);
     if (record && stats) return fail(PLBAMD_EINVAL, "recording step: statistics must be off");
-    if (!odd && L.linearEven) {
+    // the special cells in the bulk launch (bulk_and_special)
+    SpecialArgs s{};
+    s.arena = L.arena; s.blocks = L.dGeom; s.nBlocks = (int)L.geom.size(); s.omega = L.desc.omega;
+    for (int c = 0; c < 3; ++c) s.force[c] = L.desc.force[c];
+    s.alpha = L.dAlpha;
+    s.cells = L.dSpecial; s.count = L.nSpecial; s.values = L.dValues;
+    s.partials = L.dSpecialPartials;
+    if (record) {
+        s.moments = record->moments;
+        s.momStride = record->momStride;
+        s.dumpF = record->specialF;
+    }
+    const bool together = sizeof(typename Store<S>::R) >= 4 && L.nSpecial && L.staged && L.policy == 2 && !L.linearEven &&
+                          L.nBulkPartials <= kTogetherRows;
+    if (together) {
+        if constexpr (sizeof(typename Store<S>::R) >= 4) {
+            if (record) {
+                a.moments = record->moments;
+                a.momStride = record->momStride;
+            }
+            const uint32_t ns = ((L.nSpecial + kSpecialThreads - 1) / kSpecialThreads + 7) / 8 * 8;   // keeps the XCD order
+            const dim3 tg(ns + (unsigned)L.nBulkPartials);
+#define PLBAMD_TOG(O, ST, FO, MO)                                                                                   \
+    hipLaunchKernelGGL((bulk_and_special<S, DYN, O, ST, FO, MO>), tg, L.bulkBlock, O ? L.stagedLds : 0, L.stream, a, s, ns)
+#define PLBAMD_TOG_F(O, ST, MO) do { if (forced) PLBAMD_TOG(O, ST, true, MO); else PLBAMD_TOG(O, ST, false, MO); } while (0)
+            if (record) {
+                if constexpr (std::is_same<S, double>::value) {
+                    if (odd) PLBAMD_TOG_F(true, false, true); else PLBAMD_TOG_F(false, false, true);
+                } else {
+                    return fail(PLBAMD_EINVAL, "recording step: FP64 or 16-bit storage");
+                }
+            } else if (stats) {
+                if (odd) PLBAMD_TOG_F(true, true, false); else PLBAMD_TOG_F(false, true, false);
+            } else {
+                if (odd) PLBAMD_TOG_F(true, false, false); else PLBAMD_TOG_F(false, false, false);
+            }
+#undef PLBAMD_TOG_F
+#undef PLBAMD_TOG
+        }
+    } else if (!odd && L.linearEven) {
         // even steps in memory order (bulk_even_linear)
         a.evenBlock = L.dEvenBlock;
         const dim3 eg((unsigned)L.nEven), eb(kEvenThreads);
@@ -37,7 +82,11 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
             a.moments = record->moments;
             a.momStride = record->momStride;
             if constexpr (std::is_same<S, double>::value || sizeof(typename Store<S>::R) == 2) {
-#define PLBAMD_EVR(TG, FO) hipLaunchKernelGGL((bulk_even_linear<S, DYN, TG, false, FO, true>), eg, eb, 0, L.stream, a)
+#define PLBAMD_EVR(TG, FO)                                                                                          \
+    do {                                                                                                            \
+        if (L.policy == 2) hipLaunchKernelGGL((bulk_even_linear<S, DYN, TG, false, FO, true, true>), eg, eb, 0, L.stream, a); \
+        else hipLaunchKernelGGL((bulk_even_linear<S, DYN, TG, false, FO, true>), eg, eb, 0, L.stream, a);           \
+    } while (0)
                 if (tags) { if (forced) PLBAMD_EVR(true, true); else PLBAMD_EVR(true, false); }
                 else { if (forced) PLBAMD_EVR(false, true); else PLBAMD_EVR(false, false); }
 #undef PLBAMD_EVR
@@ -45,7 +94,11 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
                 return fail(PLBAMD_EINVAL, "recording step: FP64 or 16-bit storage");
             }
         } else {
-#define PLBAMD_EV(TG, ST, FO) hipLaunchKernelGGL((bulk_even_linear<S, DYN, TG, ST, FO>), eg, eb, 0, L.stream, a)
+#define PLBAMD_EV(TG, ST, FO)                                                                                       \
+    do {                                                                                                            \
+        if (L.policy == 2) hipLaunchKernelGGL((bulk_even_linear<S, DYN, TG, ST, FO, false, true>), eg, eb, 0, L.stream, a); \
+        else hipLaunchKernelGGL((bulk_even_linear<S, DYN, TG, ST, FO>), eg, eb, 0, L.stream, a);                    \
+    } while (0)
 #define PLBAMD_EV_F(TG, ST) if (forced) PLBAMD_EV(TG, ST, true); else PLBAMD_EV(TG, ST, false)
 #define PLBAMD_EV_S(TG) if (stats) { PLBAMD_EV_F(TG, true); } else { PLBAMD_EV_F(TG, false); }
             if (tags) { PLBAMD_EV_S(true) } else { PLBAMD_EV_S(false) }
@@ -59,12 +112,17 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
         if constexpr (std::is_same<S, double>::value) {
 #define PLBAMD_REC(O, TG, FO)                                                                                   \
     do {                                                                                                        \
-        if (O && L.staged && L.cachedZ)                                                                         \
-            hipLaunchKernelGGL((bulk_odd_staged<double, DYN, TG, false, FO, true, true>), grid, L.bulkBlock,     \
+        if (O && L.staged && L.policy == 2)                                                                     \
+            hipLaunchKernelGGL((bulk_odd_staged<double, DYN, TG, false, FO, true, 2>), grid, L.bulkBlock,        \
+                               L.stagedLds, L.stream, a);                                                       \
+        else if (O && L.staged && L.policy == 1)                                                                \
+            hipLaunchKernelGGL((bulk_odd_staged<double, DYN, TG, false, FO, true, 1>), grid, L.bulkBlock,        \
                                L.stagedLds, L.stream, a);                                                       \
         else if (O && L.staged)                                                                                 \
             hipLaunchKernelGGL((bulk_odd_staged<double, DYN, TG, false, FO, true>), grid, L.bulkBlock,           \
                                L.stagedLds, L.stream, a);                                                       \
+        else if (!O && L.policy == 2)                                                                           \
+            hipLaunchKernelGGL((bulk_step<double, DYN, O, TG, false, FO, true, !O>), grid, L.bulkBlock, 0, L.stream, a); \
         else                                                                                                    \
             hipLaunchKernelGGL((bulk_step<double, DYN, O, TG, false, FO, true>), grid, L.bulkBlock, 0, L.stream, a); \
     } while (0)
@@ -81,7 +139,10 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
         if (L.packed)                                                                                           \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, false, FO, true, true>), grid, L.bulkBlock,           \
                                O ? L.pairsLds : 0, L.stream, a);                                                \
-        else if (O && L.cachedZ)                                                                                \
+        else if (O && L.policy == 2)                                                                            \
+            hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, false, FO, true, false, false, O ? 2 : 0>), grid,   \
+                               L.bulkBlock, L.pairsLds, L.stream, a);                                           \
+        else if (O && L.policy == 1)                                                                            \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, false, FO, true, false, false, O>), grid,           \
                                L.bulkBlock, L.pairsLds, L.stream, a);                                           \
         else                                                                                                    \
@@ -101,19 +162,28 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
         if constexpr (sizeof(typename Store<S>::R) == 2) {
 #define PLBAMD_PAIRS(O, TG, ST, FO)                                                                             \
     do {                                                                                                        \
-        if (L.packed && O && L.cachedZ)                                                                         \
+        if (L.packed && O && L.policy == 2)                                                                     \
+            hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, true, false, O ? 2 : 0>), grid,      \
+                               L.bulkBlock, L.pairsLds, L.stream, a);                                           \
+        else if (L.packed && O && L.policy == 1)                                                                \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, true, false, O>), grid, L.bulkBlock, \
                                L.pairsLds, L.stream, a);                                                        \
         else if (L.packed)                                                                                      \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, true>), grid, L.bulkBlock,             \
                                O ? L.pairsLds : 0, L.stream, a);                                                \
-        else if (O && L.zWrap && L.cachedZ)                                                                     \
+        else if (O && L.zWrap && L.policy == 2)                                                                 \
+            hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, false, O, O ? 2 : 0>), grid,         \
+                               L.bulkBlock, L.pairsLds, L.stream, a);                                           \
+        else if (O && L.zWrap && L.policy == 1)                                                                 \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, false, O, O>), grid, L.bulkBlock, \
                                L.pairsLds, L.stream, a);                                                        \
         else if (O && L.zWrap)                                                                                  \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, false, true>), grid, L.bulkBlock,      \
                                L.pairsLds, L.stream, a);                                                        \
-        else if (O && L.cachedZ)                                                                                \
+        else if (O && L.policy == 2)                                                                            \
+            hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, false, false, O ? 2 : 0>), grid,     \
+                               L.bulkBlock, L.pairsLds, L.stream, a);                                           \
+        else if (O && L.policy == 1)                                                                            \
             hipLaunchKernelGGL((bulk_pairs<S, DYN, O, TG, ST, FO, false, false, false, O>), grid,             \
                                L.bulkBlock, L.pairsLds, L.stream, a);                                           \
         else                                                                                                    \
@@ -134,12 +204,17 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
     } else {
 #define PLBAMD_BULK(O, TG, ST, FO)                                                                              \
     do {                                                                                                        \
-        if (O && L.staged && L.cachedZ)                                                                         \
-            hipLaunchKernelGGL((bulk_odd_staged<S, DYN, TG, ST, FO, false, true>), grid, L.bulkBlock,            \
+        if (O && L.staged && L.policy == 2)                                                                     \
+            hipLaunchKernelGGL((bulk_odd_staged<S, DYN, TG, ST, FO, false, 2>), grid, L.bulkBlock,               \
+                               L.stagedLds, L.stream, a);                                                       \
+        else if (O && L.staged && L.policy == 1)                                                                \
+            hipLaunchKernelGGL((bulk_odd_staged<S, DYN, TG, ST, FO, false, 1>), grid, L.bulkBlock,               \
                                L.stagedLds, L.stream, a);                                                       \
         else if (O && L.staged)                                                                                 \
             hipLaunchKernelGGL((bulk_odd_staged<S, DYN, TG, ST, FO>), grid, L.bulkBlock, L.stagedLds, L.stream,  \
                                a);                                                                              \
+        else if (!O && L.policy == 2)                                                                           \
+            hipLaunchKernelGGL((bulk_step<S, DYN, O, TG, ST, FO, false, !O>), grid, L.bulkBlock, 0, L.stream, a); \
         else                                                                                                    \
             hipLaunchKernelGGL((bulk_step<S, DYN, O, TG, ST, FO>), grid, L.bulkBlock, 0, L.stream, a);         \
     } while (0)
@@ -153,18 +228,7 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
 #undef PLBAMD_BULK
     }
     PLBAMD_HIP(hipGetLastError());
-    if (L.nSpecial) {
-        SpecialArgs s{};
-        s.arena = L.arena; s.blocks = L.dGeom; s.nBlocks = (int)L.geom.size(); s.omega = L.desc.omega;
-        for (int c = 0; c < 3; ++c) s.force[c] = L.desc.force[c];
-        s.alpha = L.dAlpha;
-        s.cells = L.dSpecial; s.count = L.nSpecial; s.values = L.dValues;
-        s.partials = L.dSpecialPartials;
-        if (record) {
-            s.moments = record->moments;
-            s.momStride = record->momStride;
-            s.dumpF = record->specialF;
-        }
+    if (L.nSpecial && !together) {
         const dim3 sg((L.nSpecial + kSpecialThreads - 1) / kSpecialThreads), sb(kSpecialThreads);
 #define PLBAMD_SPECIAL(O, ST, FO) hipLaunchKernelGGL((special_step<S, DYN, O, ST, FO>), sg, sb, 0, L.stream, s)
 #define PLBAMD_SPECIAL_F(O, ST) if (forced) PLBAMD_SPECIAL(O, ST, true); else PLBAMD_SPECIAL(O, ST, false)
