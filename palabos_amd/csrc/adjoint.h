@@ -93,6 +93,7 @@ struct AdjointArgs {
     // every block in one launch: block b takes workgroups [wgBegin[b], wgBegin[b+1])
     // of 64 (z) x 4 (y) threads over its (ceil(nz/64), ceil(ny/4), nx) tiles
     const BlockGeom* blocks;
+    int nBlocks;
     const uint16_t* wgBlock;  // block of every workgroup
     const uint32_t* wgBegin;  // first workgroup of every block
     double* acc;              // per workgroup: J accumulated over the reverse sweep
@@ -104,21 +105,21 @@ struct AdjointCell {
     BlockGeom g;
     int x, y, z;
 };
-__device__ __forceinline__ AdjointCell adjoint_cell_of(const AdjointArgs& a) {
+__device__ __forceinline__ AdjointCell adjoint_cell_of(const AdjointArgs& a, uint32_t wg) {
     AdjointCell c;
-    const uint32_t wg = blockIdx.x;
-    const int b = (int)a.wgBlock[wg];
+    const int b = a.nBlocks == 1 ? 0 : (int)a.wgBlock[wg];
     c.g = a.blocks[b];
     const uint32_t local = wg - a.wgBegin[b];
     const uint32_t gz = (uint32_t)(c.g.nz + 63) / 64, gy = (uint32_t)(c.g.ny + 3) / 4;
     c.z = (int)(local % gz) * 64 + (int)threadIdx.x;
     const uint32_t rest = local / gz;
-    c.y = (int)(rest % gy) * 4 + (int)threadIdx.y;
+    // a wavefront is one row of 64 cells: its y as a scalar
+    c.y = (int)(rest % gy) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     c.x = (int)(rest / gy);
     return c;
 }
 // The shuffle tree and wavefront order of block_reduce_store, for the one value.
-__device__ __forceinline__ void accumulate_J(double J, double* acc) {
+__device__ __forceinline__ void accumulate_J(double J, double* acc, uint32_t wg) {
     __shared__ double red[16];
     const int t = threadIdx.x + threadIdx.y * blockDim.x;
     const int n = blockDim.x * blockDim.y;
@@ -133,7 +134,7 @@ __device__ __forceinline__ void accumulate_J(double J, double* acc) {
     if (t == 0) {
         double r = red[0];
         for (int w = 1; w < nWaves; ++w) r += red[w];
-        acc[blockIdx.x] += r;
+        acc[wg] += r;
     }
 }
 
@@ -143,50 +144,59 @@ __device__ __forceinline__ void objective_gradient(const AdjointArgs& a, int gx,
     for (int k = 0; k < 19; ++k) djdf[k] = a.wdp * p + (a.wdrag * a.omega * alphaY + a.wflux) * (double)cx(k);
 }
 
+// Value read or written once per step: nontemporal (NT) where the adjoint states
+// are too large for the last-level cache, ordinary below.
+template<bool NT, typename LT>
+__device__ __forceinline__ LT ld_lam(const LT* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template<bool NT, typename LT>
+__device__ __forceinline__ void st_lam(LT* p, LT v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 // mu(y) gathered from lambda^{t+1} (transpose of streaming with edge
 // reflection: mu_i(y) = lambda_i(y + c_i), or lambda_opp(i)(y) where y + c_i
-// leaves the block), by the lanes of a wavefront that hold consecutive cells
-// z0 .. z0 + 63 of one row (lane = z - z0; the row, and so every x/y edge test,
-// is the wavefront's). Every direction is loaded at the lane's own z in its
-// source row, aligned; the z-moving ones are then passed one lane along by a
-// cross-lane read (ds_bpermute) instead of a load straddling one more cache line
-// per wavefront. A lane whose source lies beyond the wavefront's cells, wraps
-// around a periodic row or leaves the block loads its own value. Every lane of
-// the row with z < nz takes part (their loads are what the others read).
+// leaves the block), by the lanes of a wavefront that hold consecutive cells of
+// one row. Inside, a direction is one load from a scalar address (one of nine row
+// offsets, the slot pointer stepped along) at one of three lane offsets (z - 1, z,
+// z + 1, wrapped), all 19 in flight at once. Only wavefronts at a non-periodic
+// edge or beside a link wall choose the address lane by lane.
+// (Aligned loads with the z-moving values passed on by cross-lane reads left each
+// wavefront ten conditional loads, one after the other, for its end lanes.)
 // WALLS, wall: the cell's link-wall mask (bit i: wall at x + c_i): those
-// directions take lambda_opp(i) of the cell itself, loaded beside the row loads.
-// A lattice without link walls takes the kernel without them: no conditional
-// load between the row loads, which then go out back to back.
-template<typename LT, typename C, bool WALLS>
-__device__ __forceinline__ void gather_mu_wave(const BlockGeom& g, const LT* lamNext, int x, int y, int z, int z0,
-                                               uint64_t cell, C mu[19], uint32_t wall) {
-    const int lane = z - z0;
-    mu[0] = (C)lamNext[cell];
+// directions take lambda_opp(i) of the cell itself.
+template<typename LT, bool WALLS, bool NT>
+__device__ __forceinline__ void gather_mu_row(const BlockGeom& g, const LT* lamNext, int x, int y, int z, uint64_t row0,
+                                              LT mu[19], uint32_t wall) {
+    int zo[3] = {z, z, z}, xs[3] = {x, x, x}, ys[3] = {y, y, y};
+    const bool zin[3] = {shift(z, -1, g.nz, g.pz, zo[0]), true, shift(z, 1, g.nz, g.pz, zo[2])};
+    const bool xin[3] = {shift(x, -1, g.nx, g.px, xs[0]), true, shift(x, 1, g.nx, g.px, xs[2])};
+    const bool yin[3] = {shift(y, -1, g.ny, g.py, ys[0]), true, shift(y, 1, g.ny, g.py, ys[2])};
+    mu[0] = ld_lam<NT>(lamNext + row0 + (uint32_t)z);
+    if (xin[0] && xin[2] && yin[0] && yin[2] && __ballot(!zin[0] || !zin[2] || (WALLS && wall)) == 0) {
+        const uint32_t zb[3] = {(uint32_t)(zo[0] * (int)sizeof(LT)), (uint32_t)(z * (int)sizeof(LT)),
+                                (uint32_t)(zo[2] * (int)sizeof(LT))};
+        int64_t off[3][3];
 #pragma unroll
-    for (int i = 1; i < 19; ++i) {
-        int dx, dy;
-        const LT* refl = lamNext + (uint64_t)opp(i) * g.slot + cell;
-        if (!(shift(x, cx(i), g.nx, g.px, dx) && shift(y, cy(i), g.ny, g.py, dy))) {
-            mu[i] = (C)*refl;
-            continue;
+        for (int ax = 0; ax < 3; ++ax)
+#pragma unroll
+            for (int ay = 0; ay < 3; ++ay) off[ax][ay] = ((int64_t)xs[ax] * g.ny + ys[ay]) * g.nz;
+        const LT* slot = lamNext;
+#pragma unroll
+        for (int i = 1; i < 19; ++i) {
+            slot += g.slot;
+            mu[i] = ld_lam<NT>(at(const_cast<LT*>(slot + off[1 + cx(i)][1 + cy(i)]), zb[1 + cz(i)]));
         }
-        const bool wr = WALLS && ((wall >> i) & 1u);
-        const LT* row = lamNext + (uint64_t)i * g.slot + ((uint64_t)dx * g.ny + dy) * g.nz;
-        const LT v = row[z];
-        const LT w = wr ? *refl : LT(0);
-        if (cz(i) == 0) {
-            mu[i] = wr ? (C)w : (C)v;
-            continue;
-        }
-        const LT nb = __shfl(v, lane + cz(i), 64);
-        const int zs = z + cz(i);
-        if (wr) {
-            mu[i] = (C)w;
-        } else if (zs >= z0 && zs < z0 + 64 && zs < g.nz) {
-            mu[i] = (C)nb;
-        } else {
-            int dz;
-            mu[i] = shift(z, cz(i), g.nz, g.pz, dz) ? (C)row[dz] : (C)*refl;
+    } else {
+#pragma unroll
+        for (int i = 1; i < 19; ++i) {
+            const bool ok = xin[1 + cx(i)] && yin[1 + cy(i)] && zin[1 + cz(i)] && !(WALLS && ((wall >> i) & 1u));
+            const uint64_t from = (uint64_t)i * g.slot + ((uint64_t)xs[1 + cx(i)] * g.ny + ys[1 + cy(i)]) * g.nz + zo[1 + cz(i)];
+            const uint64_t own = (uint64_t)opp(i) * g.slot + row0 + z;
+            mu[i] = ld_lam<NT>(lamNext + (ok ? from : own));
         }
     }
 }
@@ -205,29 +215,31 @@ __device__ __forceinline__ int cx_of(uint32_t i) {
 // of the porosity and of the porosity-gradient accumulator (one segment's sum
 // for a 16-bit forward, added into an FP64 total); the objective accumulates
 // in FP64.
-template<typename LT, int DYN, bool FORCED, bool WALLS>
-__device__ __forceinline__ void adjoint_cell(const AdjointArgs& a, const BlockGeom& g, int x, int y, int z, int z0,
-                                             double& J) {
+template<typename LT, int DYN, bool FORCED, bool WALLS, bool NT>
+__device__ __forceinline__ void adjoint_cell(const AdjointArgs& a, const BlockGeom& g, int x, int y, int z, double& J) {
     using C = LT;
-    const uint64_t cell = ((uint64_t)x * g.ny + y) * g.nz + z;
-    const uint64_t idx = g.cellOffset + cell;
+    const uint64_t row0 = ((uint64_t)x * g.ny + y) * g.nz;
+    const uint64_t idx0 = g.cellOffset + row0;     // per-cell arrays: a scalar row address and the lane's z
     const LT* lamNext = reinterpret_cast<const LT*>(a.lamNext) + g.offset;
-    LT* lam = reinterpret_cast<LT*>(a.lam) + g.offset;
-    // the gather first, by every cell of the row (plane cells included: their
-    // loads feed their neighbours' lanes), then the skip test
     // a link wall at x + c_i sends f_i back into the cell's own slot opp(i) (the
     // forward's reflection): mu_i = lambda_opp(i) of the cell itself. The mask
     // is loaded first, so that those loads go out with the gather's.
-    const uint32_t wall = WALLS ? a.walls[idx] : 0u;
+    const uint32_t wall = WALLS ? (a.walls + idx0)[(uint32_t)z] : 0u;
     C mu[19];
-    gather_mu_wave<LT, C, WALLS>(g, lamNext, x, y, z, z0, cell, mu, wall);
-    if (!(a.tags && a.tags[idx] == BT_SKIP)) {
-        const C al = a.alpha ? reinterpret_cast<const LT*>(a.alpha)[idx] : C(0);
+    gather_mu_row<LT, WALLS, NT>(g, lamNext, x, y, z, row0, mu, wall);
+    if (!(a.tags && (a.tags + idx0)[(uint32_t)z] == BT_SKIP)) {
+        const C al = a.alpha ? (reinterpret_cast<const LT*>(a.alpha) + idx0)[(uint32_t)z] : C(0);
         const double al64 = (double)al;
         const C dm = C(1) - al;
         const LT* mom = reinterpret_cast<const LT*>(a.mom);
-        const C rhoBar = (C)mom[idx];
-        const C j[3] = {(C)mom[a.momStride + idx], (C)mom[2 * a.momStride + idx], (C)mom[3 * a.momStride + idx]};
+        const LT* momRow = mom + idx0;
+        const C rhoBar = ld_lam<true>(momRow + (uint32_t)z);
+        C j[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            momRow += a.momStride;
+            j[c] = ld_lam<true>(momRow + (uint32_t)z);
+        }
         const C rho = C(1) + rhoBar;
         const C F[3] = {FORCED ? (C)a.force[0] : C(0), FORCED ? (C)a.force[1] : C(0), FORCED ? (C)a.force[2] : C(0)};
         const C Jv[3] = {dm * (j[0] + rho * F[0] * C(0.5)), dm * (j[1] + rho * F[1] * C(0.5)),
@@ -301,6 +313,8 @@ __device__ __forceinline__ void adjoint_cell(const AdjointArgs& a, const BlockGe
         const C p = (C)((gx == a.xin ? a.inW : 0.0) - (gx == a.xout ? a.outW : 0.0));
         const C djBase = (C)a.wdp * p, djX = (C)(a.wdrag * a.omega * al64 + a.wflux);
         const C invT = (C)a.invT;
+        LT* out = reinterpret_cast<LT*>(a.lam) + (g.offset + row0);
+        const uint32_t zb = (uint32_t)z * (uint32_t)sizeof(LT);
 #pragma unroll
         for (int k = 0; k < 19; ++k) {
             C val = s;
@@ -320,7 +334,8 @@ __device__ __forceinline__ void adjoint_cell(const AdjointArgs& a, const BlockGe
                 val += (C(1) - w) * cMc;
             }
             if (a.explicitTerm) val += invT * (cx(k) == 0 ? djBase : (cx(k) > 0 ? djBase + djX : djBase - djX));
-            lam[(uint64_t)k * g.slot + cell] = (LT)val;
+            st_lam<NT>(at(out, zb), (LT)val);
+            out += g.slot;
         }
         if (in_bulk(g, x, y, z)) {
             const C wB = DYN == 0 ? w : C(1);
@@ -335,20 +350,29 @@ __device__ __forceinline__ void adjoint_cell(const AdjointArgs& a, const BlockGe
                 J += a.invT * (a.wdp * p64 * (double)rho + a.wdrag * a.omega * al64 * (double)j[0] +
                                a.wflux * (double)j[0]);
             }
-            if (a.gAlpha) reinterpret_cast<LT*>(a.gAlpha)[idx] += (LT)ga64;
+            if (a.gAlpha) (reinterpret_cast<LT*>(a.gAlpha) + idx0)[(uint32_t)z] += (LT)ga64;
         }
     }
 }
 
 // Reverse step of every bulk cell of every block (64 x 4 cells per workgroup).
 // WALLS: the lattice has link-wall masks (a.walls not null).
-template<typename LT, int DYN, bool FORCED, bool WALLS>
-__global__ void __launch_bounds__(256) adjoint_bulk(AdjointArgs a) {
-    const AdjointCell c = adjoint_cell_of(a);
+// FP64 is bound by memory (256x192x192: 556 us, 361 bytes a cell at 6.1 TB/s), FP32 by
+// memory and by instructions alike. Scalar row addresses instead of ones
+// recomputed per direction, and back-to-back loads: FP32
+// 192x128x128 with force and porosity 138 -> 116 us (180 bytes a cell at 4.9 TB/s), 64^3
+// 13.8 -> 10.7; FP64 channel 128x64x64 with its planes 79 -> 49.
+template<typename LT, int DYN, bool FORCED, bool WALLS, bool NT>
+__device__ __forceinline__ void adjoint_bulk_body(const AdjointArgs& a, uint32_t wg) {
+    const AdjointCell c = adjoint_cell_of(a, wg);
     double J = 0.0;
-    if (c.z < c.g.nz && c.y < c.g.ny)
-        adjoint_cell<LT, DYN, FORCED, WALLS>(a, c.g, c.x, c.y, c.z, c.z - (int)threadIdx.x, J);
-    if (a.explicitTerm) accumulate_J(J, a.acc);   // J is zero before the objective's window
+    if (c.z < c.g.nz && c.y < c.g.ny) adjoint_cell<LT, DYN, FORCED, WALLS, NT>(a, c.g, c.x, c.y, c.z, J);
+    if (a.explicitTerm) accumulate_J(J, a.acc, wg);   // J is zero before the objective's window
+}
+template<typename LT, int DYN, bool FORCED, bool WALLS, bool NT>
+__global__ void __launch_bounds__(256) adjoint_bulk(AdjointArgs a) {
+    // the tiles of a row in one XCD's L2: their z-moving loads share lines
+    adjoint_bulk_body<LT, DYN, FORCED, WALLS, NT>(a, xcd_item(blockIdx.x, gridDim.x));
 }
 
 struct AdjointSpecialArgs {
@@ -364,11 +388,11 @@ struct AdjointSpecialArgs {
 // thread per (record, direction): direction k < 19 seeds df_k and yields
 // lambda_k = mu . dC/df_k; direction 19 seeds the plane's velocity scale.
 template<typename LT>
-__global__ void __launch_bounds__(256) adjoint_planes(AdjointSpecialArgs s) {
+__device__ __forceinline__ void adjoint_planes_body(const AdjointSpecialArgs& s, uint32_t wg) {
     const AdjointArgs& a = s.base;
     const BlockGeom g = a.g;
     double J = 0.0;
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = wg * 256 + threadIdx.y * blockDim.x + threadIdx.x;
     const uint32_t k = t % s.count, dirn = t / s.count;
     if (t < 20 * s.count) {
         const SpecialCell sc = s.cells[k];
@@ -421,14 +445,31 @@ __global__ void __launch_bounds__(256) adjoint_planes(AdjointSpecialArgs s) {
             }
         }
     }
-    accumulate_J(J, s.partials);
+    accumulate_J(J, s.partials, wg);
+}
+template<typename LT>
+__global__ void __launch_bounds__(256) adjoint_planes(AdjointSpecialArgs s) {
+    adjoint_planes_body<LT>(s, blockIdx.x);
+}
+
+// Plane and bulk cells in one launch (they write disjoint cells): the first
+// planeWGs workgroups take the planes. The kernel has the dual numbers'
+// registers (two wavefronts per SIMD), so it is for lattices on which the planes'
+// own launch costs more than the occupancy.
+template<typename LT>
+__global__ void __launch_bounds__(256) adjoint_bulk_and_planes(AdjointSpecialArgs s, uint32_t planeWGs, uint32_t usedWGs) {
+    if (blockIdx.x < planeWGs) {
+        if (blockIdx.x < usedWGs) adjoint_planes_body<LT>(s, blockIdx.x);
+    } else {
+        adjoint_bulk_body<LT, 0, false, false, false>(s.base, xcd_item(blockIdx.x - planeWGs, gridDim.x - planeWGs));
+    }
 }
 
 // lambda^T = dj/df(f^T) / (T - t0); J += j(f^T) / (T - t0);
 // g_alpha += w_drag omega j_x(f^T) / (T - t0).
 template<typename LT>
 __global__ void __launch_bounds__(256) adjoint_final(AdjointArgs a) {
-    const AdjointCell c = adjoint_cell_of(a);
+    const AdjointCell c = adjoint_cell_of(a, blockIdx.x);
     const BlockGeom& g = c.g;
     const int x = c.x, y = c.y, z = c.z;
     double J = 0.0;
@@ -452,7 +493,7 @@ __global__ void __launch_bounds__(256) adjoint_final(AdjointArgs a) {
             J += a.invT * (a.wdp * p * (1.0 + rhoBar) + a.wdrag * a.omega * al * jx + a.wflux * jx);
         }
     }
-    accumulate_J(J, a.acc);
+    accumulate_J(J, a.acc, blockIdx.x);
 }
 
 // The FP32 gradient accumulator of a 16-bit adjoint (one segment's sum) added

@@ -9,6 +9,16 @@
 
 namespace plbamd {
 
+// Bytes of both adjoint states up to which they are read and written with
+// ordinary accesses and stay in the last-level cache (us a reverse step, ordinary /
+// nontemporal): FP64 128x64x64 (160 MB) 54.4 / 57.3, 96^3 (269 MB) 68.9 / 67.7, 128^3 143.6
+// / 134.3, 256x192x192 579 / 556; FP32 192x128x128 119.6 / 116.4.
+constexpr uint64_t kCachedAdjointBytes = 200000000;
+// Workgroups of the bulk reverse step up to which the planes go along with it
+// (us a step, two launches / one): FP64 channel 32^3 16.9 / 12.3, 64^3 (1024) 37.2 /
+// 32.2, 128x64x64 (2048) 54.4 / 49.2, 131x65x67 (4454) 71.8 / 72.1, 128x96x96 (6144) 126 / 134.
+constexpr uint32_t kAdjointTogetherWGs = 4096;
+
 int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, double* Jout, double* gradAlpha,
                     double* gradScale, double* timing) {
     const int st = L.desc.storage;
@@ -220,30 +230,33 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     a.xin = obj.inlet_x;
     a.xout = obj.outlet_x;
     a.blocks = L.dGeom;
+    a.nBlocks = (int)L.geom.size();
     a.wgBlock = dAdjBlock;
     a.wgBegin = dAdjBegin;
     a.acc = acc;
     const bool rbgk = L.desc.dynamics == PLBAMD_RBGK;
     const bool walls = a.walls != nullptr;
-#define PLBAMD_ADJ(LT, W) \
+    const bool nt = 2 * arenaElems * lamSize > kCachedAdjointBytes;
+#define PLBAMD_ADJ(LT, D, FO, W) \
     do { \
-        if (rbgk) { \
-            if (forced) hipLaunchKernelGGL((adjoint_bulk<LT, 1, true, W>), gr, ablock, 0, L.stream, args); \
-            else hipLaunchKernelGGL((adjoint_bulk<LT, 1, false, W>), gr, ablock, 0, L.stream, args); \
-        } else { \
-            if (forced) hipLaunchKernelGGL((adjoint_bulk<LT, 0, true, W>), gr, ablock, 0, L.stream, args); \
-            else hipLaunchKernelGGL((adjoint_bulk<LT, 0, false, W>), gr, ablock, 0, L.stream, args); \
-        } \
+        if (nt) hipLaunchKernelGGL((adjoint_bulk<LT, D, FO, W, true>), gr, ablock, 0, L.stream, args); \
+        else hipLaunchKernelGGL((adjoint_bulk<LT, D, FO, W, false>), gr, ablock, 0, L.stream, args); \
+    } while (0)
+#define PLBAMD_ADJ_W(LT, W) \
+    do { \
+        if (rbgk) { if (forced) PLBAMD_ADJ(LT, 1, true, W); else PLBAMD_ADJ(LT, 1, false, W); } \
+        else { if (forced) PLBAMD_ADJ(LT, 0, true, W); else PLBAMD_ADJ(LT, 0, false, W); } \
     } while (0)
     auto reverseKernel = [&](const AdjointArgs& args, const dim3& gr) {
         if (lam64) {
-            if (walls) PLBAMD_ADJ(double, true);
-            else PLBAMD_ADJ(double, false);
+            if (walls) PLBAMD_ADJ_W(double, true);
+            else PLBAMD_ADJ_W(double, false);
         } else {
-            if (walls) PLBAMD_ADJ(float, true);
-            else PLBAMD_ADJ(float, false);
+            if (walls) PLBAMD_ADJ_W(float, true);
+            else PLBAMD_ADJ_W(float, false);
         }
     };
+#undef PLBAMD_ADJ_W
 #undef PLBAMD_ADJ
     auto exchangeLam = [&](char* lam) {
         if (!L.multi || !L.nSegs) return;
@@ -258,14 +271,9 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
             hipLaunchKernelGGL((exchange_envelopes<float>), dim3(L.nTasks1), dim3(256), 0, L.stream, (void*)lam,
                                L.dGeom, L.dSegs1, L.dTasks1);
     };
-    // the plane cells' reverse step runs on a second stream next to the bulk one
-    hipStream_t side = nullptr;
-    hipEvent_t evIn = nullptr, evOut = nullptr;
-    if (err == hipSuccess && L.nSpecial) {
-        err = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
-        if (err == hipSuccess) err = hipEventCreateWithFlags(&evIn, hipEventDisableTiming);
-        if (err == hipSuccess) err = hipEventCreateWithFlags(&evOut, hipEventDisableTiming);
-    }
+    // the plane cells' reverse step (single block, BGK, no force, no walls) in the
+    // bulk launch on small lattices
+    const bool together = L.nSpecial && adjWGs <= kAdjointTogetherWGs;
     char* lamNext = lamA;
     char* lamCur = lamB;
     void* const arena = L.arena;
@@ -308,31 +316,28 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
             a.explicitTerm = t > obj.first_step ? 1 : 0;
             a.lamNext = lamNext;
             a.lam = lamCur;
-            if (err == hipSuccess && L.nSpecial) {
-                // plane cells (single block) on the side stream, after the previous step
+            if (L.nSpecial) {
                 AdjointSpecialArgs sa{};
-                AdjointArgs pa = a;
-                pa.g = L.geom[0];
-                sa.base = pa;
+                sa.base = a;
+                sa.base.g = L.geom[0];
                 sa.cells = L.dSpecial;
                 sa.count = L.nSpecial;
                 sa.values = L.dValues;
                 sa.partials = acc + adjWGs;
                 sa.gScale = gS;
-                err = hipEventRecord(evIn, L.stream);
-                if (err == hipSuccess) err = hipStreamWaitEvent(side, evIn, 0);
-                if (err == hipSuccess) {
-                    if (lam64) hipLaunchKernelGGL(adjoint_planes<double>, dim3(planeWGs), dim3(256), 0, side, sa);
-                    else hipLaunchKernelGGL(adjoint_planes<float>, dim3(planeWGs), dim3(256), 0, side, sa);
+                if (together) {
+                    const uint32_t pw = (planeWGs + 7) / 8 * 8;   // keeps the XCD order
+                    const dim3 tg(pw + adjWGs);
+                    if (lam64) hipLaunchKernelGGL(adjoint_bulk_and_planes<double>, tg, ablock, 0, L.stream, sa, pw, planeWGs);
+                    else hipLaunchKernelGGL(adjoint_bulk_and_planes<float>, tg, ablock, 0, L.stream, sa, pw, planeWGs);
+                } else {
+                    if (lam64) hipLaunchKernelGGL(adjoint_planes<double>, dim3(planeWGs), dim3(256), 0, L.stream, sa);
+                    else hipLaunchKernelGGL(adjoint_planes<float>, dim3(planeWGs), dim3(256), 0, L.stream, sa);
                     err = hipGetLastError();
                 }
-                if (err == hipSuccess) err = hipEventRecord(evOut, side);
             }
-            if (err == hipSuccess) {
-                reverseKernel(a, agrid);
-                err = hipGetLastError();
-            }
-            if (err == hipSuccess && L.nSpecial) err = hipStreamWaitEvent(L.stream, evOut, 0);
+            if (err == hipSuccess && !together) reverseKernel(a, agrid);
+            if (err == hipSuccess) err = hipGetLastError();
             exchangeLam(lamCur);
             std::swap(lamNext, lamCur);
         }
@@ -345,12 +350,6 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     L.arena = arena;
     L.time = time0;
     if (err == hipSuccess) err = hipEventRecord(L.ev1, L.stream);
-    if (side) {
-        (void)hipStreamSynchronize(side);
-        (void)hipStreamDestroy(side);
-    }
-    if (evIn) (void)hipEventDestroy(evIn);
-    if (evOut) (void)hipEventDestroy(evOut);
     if (err == hipSuccess) err = hipEventSynchronize(L.ev1);
     if (err == hipSuccess) err = hipEventElapsedTime(&msB, L.ev0, L.ev1);
     L.statsOn = saveStats;
