@@ -94,8 +94,8 @@ struct AdjointArgs {
     // of 64 (z) x 4 (y) threads over its (ceil(nz/64), ceil(ny/4), nx) tiles
     const BlockGeom* blocks;
     int nBlocks;
-    const uint16_t* wgBlock;  // block of every workgroup
-    const uint32_t* wgBegin;  // first workgroup of every block
+    const uint16_t* wgBlock;  // block of every workgroup, and
+    const uint32_t* wgBegin;  // first workgroup of every block (nBlocks > 1)
     double* acc;              // per workgroup: J accumulated over the reverse sweep
 };
 
@@ -109,7 +109,7 @@ __device__ __forceinline__ AdjointCell adjoint_cell_of(const AdjointArgs& a, uin
     AdjointCell c;
     const int b = a.nBlocks == 1 ? 0 : (int)a.wgBlock[wg];
     c.g = a.blocks[b];
-    const uint32_t local = wg - a.wgBegin[b];
+    const uint32_t local = a.nBlocks == 1 ? wg : wg - a.wgBegin[b];
     const uint32_t gz = (uint32_t)(c.g.nz + 63) / 64, gy = (uint32_t)(c.g.ny + 3) / 4;
     c.z = (int)(local % gz) * 64 + (int)threadIdx.x;
     const uint32_t rest = local / gz;
@@ -504,6 +504,15 @@ static __global__ void __launch_bounds__(256) flush_gradient(float* seg, double*
         total[i] += (double)seg[i];
         seg[i] = 0.0f;
     }
+}
+
+// The porosity gradient of a box to its C-order array.
+static __global__ void __launch_bounds__(256) gradient_box(const double* gAlpha, BoxArgs a, double* out) {
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (uint64_t)a.ilx * a.ily * a.ilz) return;
+    const int iz = (int)(t % a.ilz), iy = (int)(t / a.ilz % a.ily), ix = (int)(t / a.ilz / a.ily);
+    out[((uint64_t)(a.ox + ix) * a.sly + (a.oy + iy)) * a.slz + (a.oz + iz)] =
+        gAlpha[a.g.cellOffset + lin(a.g, a.ix0 + ix, a.iy0 + iy, a.iz0 + iz)];
 }
 
 // Sum of the per-workgroup accumulators of the bulk and plane kernels (one

@@ -5,7 +5,8 @@
 // K reverse steps. The last segments, as many as the recording budget holds,
 // are recorded during the forward sweep instead and need no recompute (the
 // same kernels on the same states: the same records).
-#include "engine.h"
+#include "adjoint.h"
+#include "hostio.h"
 
 namespace plbamd {
 
@@ -72,9 +73,10 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
         adjBegin[b + 1] = adjBegin[b] + (uint32_t)(((g.nz + 63) / 64) * ((g.ny + 3) / 4) * g.nx);
     }
     const uint32_t adjWGs = adjBegin.back();
-    std::vector<uint16_t> adjBlock(adjWGs);
-    for (size_t b = 0; b < L.geom.size(); ++b)
-        std::fill(adjBlock.begin() + adjBegin[b], adjBlock.begin() + adjBegin[b + 1], (uint16_t)b);
+    std::vector<uint16_t> adjBlock(L.multi ? adjWGs : 0);    // read by the kernels of several blocks only
+    if (L.multi)
+        for (size_t b = 0; b < L.geom.size(); ++b)
+            std::fill(adjBlock.begin() + adjBegin[b], adjBlock.begin() + adjBegin[b + 1], (uint16_t)b);
     const dim3 agrid(adjWGs);
     const uint32_t planeWGs = (uint32_t)((20 * (uint64_t)L.nSpecial + 255) / 256);
     // device memory: checkpoints, a working state, the recorded moments and plane
@@ -85,77 +87,129 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     // the recorded moments have the adjoint state's type (MomentType of the storage)
     // The porosity gradient: FP64 total; a 16-bit adjoint accumulates each segment
     // in FP32 (gA32, 8 bytes per cell and step less) and adds it to the total.
-    char *ck = nullptr, *work = nullptr, *lamA = nullptr, *lamB = nullptr, *mom = nullptr;
-    double *pf = nullptr, *gA = nullptr, *gS = nullptr, *acc = nullptr, *sum = nullptr;
-    float* gA32 = nullptr;
-    char* keepMom = nullptr;    // records of the segments recorded in the forward sweep
-    double* keepPf = nullptr;
-    uint16_t* dAdjBlock = nullptr;
-    uint32_t* dAdjBegin = nullptr;
-    auto release = [&]() {
-        hipFree(ck); hipFree(work); hipFree(mom); hipFree(pf); hipFree(lamA); hipFree(lamB); hipFree(gA); hipFree(gA32);
-        hipFree(keepMom); hipFree(keepPf);
-        hipFree(gS); hipFree(acc); hipFree(sum); hipFree(dAdjBlock); hipFree(dAdjBegin);
-    };
     const uint64_t nAcc = (uint64_t)adjWGs + planeWGs;   // J accumulators: bulk workgroups, then plane ones
-    hipError_t err = deviceAlloc((void**)&ck, stateBytes * nCk);
-    if (err == hipSuccess) err = deviceAlloc((void**)&work, stateBytes);
-    if (err == hipSuccess) err = deviceAlloc((void**)&mom, momElems * (K + 1) * lamSize);
-    if (err == hipSuccess) err = deviceAlloc((void**)&pf, pfElems * (K + 1) * sizeof(double));
-    if (err == hipSuccess) err = deviceAlloc((void**)&lamA, arenaElems * lamSize);
-    if (err == hipSuccess) err = deviceAlloc((void**)&lamB, arenaElems * lamSize);
-    if (err == hipSuccess) err = deviceAlloc((void**)&gA, cells * sizeof(double));
-    if (err == hipSuccess && !lam64) err = deviceAlloc((void**)&gA32, cells * sizeof(float));
-    if (err == hipSuccess) err = deviceAlloc((void**)&gS, std::max<uint32_t>(1, L.nSpecial) * sizeof(double));
-    if (err == hipSuccess) err = deviceAlloc((void**)&acc, nAcc * sizeof(double));
-    if (err == hipSuccess) err = deviceAlloc((void**)&sum, 8 * sizeof(double));
-    if (err == hipSuccess) err = deviceAlloc((void**)&dAdjBlock, adjBlock.size() * sizeof(uint16_t));
-    if (err == hipSuccess) err = deviceAlloc((void**)&dAdjBegin, adjBegin.size() * sizeof(uint32_t));
-    if (err == hipSuccess)
-        err = hipMemcpy(dAdjBlock, adjBlock.data(), adjBlock.size() * sizeof(uint16_t), hipMemcpyHostToDevice);
-    if (err == hipSuccess)
-        err = hipMemcpy(dAdjBegin, adjBegin.data(), adjBegin.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
-    if (err != hipSuccess) {
-        (void)hipGetLastError();
-        release();
-        return fail(PLBAMD_ENOMEM, "adjoint: cannot allocate the checkpoint and adjoint buffers");
+    const uint64_t nScale = std::max<uint32_t>(1, L.nSpecial);
+    // One buffer holds everything; the lattice keeps it for the next call when it is
+    // at most a sixteenth of the card's memory (thirteen allocations a call came to
+    // cost 113 ms a call once some fifty calls had been made).
+    //   fixed:      working state, adjoint states, gradients, accumulators
+    //   recompute:  checkpoints and one segment's records (not when every segment is kept)
+    //   keep:       records of the segments recorded in the forward sweep
+    auto aligned = [](uint64_t n) { return (n + 255) / 256 * 256; };
+    const uint64_t recBytes = momElems * lamSize + pfElems * sizeof(double);
+    const uint64_t fixedBytes = aligned(stateBytes) + 2 * aligned(arenaElems * lamSize) + aligned(cells * sizeof(double)) +
+                                (lam64 ? 0 : aligned(cells * sizeof(float))) + aligned(nScale * sizeof(double)) +
+                                aligned(nAcc * sizeof(double)) + aligned(8 * sizeof(double)) +
+                                aligned(adjBlock.size() * sizeof(uint16_t)) + aligned(adjBegin.size() * sizeof(uint32_t));
+    const uint64_t againBytes = aligned(stateBytes * nCk) + aligned(momElems * (K + 1) * lamSize) +
+                                aligned(pfElems * (K + 1) * sizeof(double));
+    struct Buffer {
+        Lattice& L;
+        char* p = nullptr;
+        uint64_t bytes = 0;
+        bool ensure(uint64_t n) {
+            if (bytes >= n) return true;
+            hipFree(p);
+            p = nullptr;
+            bytes = 0;
+            if (deviceAlloc((void**)&p, n) != hipSuccess) {
+                (void)hipGetLastError();
+                p = nullptr;
+                return false;
+            }
+            bytes = n;
+            return true;
+        }
+        // given back to the lattice, or freed
+        ~Buffer() {
+            size_t freeB = 0, totalB = 0;
+            if (p && hipMemGetInfo(&freeB, &totalB) == hipSuccess && bytes <= totalB / 16) {
+                std::lock_guard<std::mutex> use(L.spareMutex);
+                if (!L.adjointBuf) {
+                    L.adjointBuf = p;
+                    L.adjointBufBytes = bytes;
+                    return;
+                }
+            }
+            hipFree(p);
+        }
+    } buffer{L};
+    {
+        std::lock_guard<std::mutex> use(L.spareMutex);
+        std::swap(buffer.p, L.adjointBuf);
+        std::swap(buffer.bytes, L.adjointBufBytes);
     }
     // Segments recorded in the forward sweep: the last nKeep, whose records
-    // (len per segment, one more for f^T) fit the budget. Record r of kept
-    // segment c is keep[keepFirst[c] + r].
-    const uint64_t recBytes = momElems * lamSize + pfElems * sizeof(double);
-    uint64_t budget = 0;
-    if (L.adjointRecordBytes >= 0) {
-        budget = (uint64_t)L.adjointRecordBytes;
-    } else {
+    // (len per segment, one more for f^T) fit the budget: what the caller allows, or
+    // the free memory beyond a reserve. Record r of kept segment c is
+    // keep[keepFirst * K + r].
+    uint64_t available = 0;
+    if (L.adjointRecordBytes < 0) {
         size_t freeB = 0, totalB = 0;
         if (hipMemGetInfo(&freeB, &totalB) == hipSuccess) {
-            const uint64_t reserve = std::max<uint64_t>(4ull << 30, totalB / 32);
-            budget = freeB > reserve ? freeB - reserve : 0;
+            const uint64_t taken = std::max<uint64_t>(4ull << 30, totalB / 32) + fixedBytes;
+            available = freeB + buffer.bytes > taken ? freeB + buffer.bytes - taken : 0;
         } else {
             (void)hipGetLastError();
         }
     }
     int nKeep = 0;
     uint64_t keepRecs = 1;
-    while (nKeep < nCk) {
-        const int c = nCk - 1 - nKeep;
-        const uint64_t more = keepRecs + (uint64_t)std::min(K, T - c * K);
-        if (more * recBytes > budget) break;
-        keepRecs = more;
-        ++nKeep;
+    auto fit = [&](uint64_t budget) {
+        nKeep = 0;
+        keepRecs = 1;
+        while (nKeep < nCk) {
+            const int c = nCk - 1 - nKeep;
+            const uint64_t more = keepRecs + (uint64_t)std::min(K, T - c * K);
+            if (more * recBytes > budget) break;
+            keepRecs = more;
+            ++nKeep;
+        }
+    };
+    auto keepBytes = [&]() {
+        return nKeep ? aligned(keepRecs * momElems * lamSize) + aligned(keepRecs * pfElems * sizeof(double)) : 0;
+    };
+    auto total = [&]() { return fixedBytes + (nKeep == nCk ? 0 : againBytes) + keepBytes(); };
+    fit(L.adjointRecordBytes >= 0 ? (uint64_t)L.adjointRecordBytes : available);
+    if (nKeep < nCk && L.adjointRecordBytes < 0) fit(available > againBytes ? available - againBytes : 0);
+    bool have = buffer.ensure(total());
+    if (!have && nKeep > 0) {
+        nKeep = 0;   // the budget was not there after all: recompute everything
+        have = buffer.ensure(total());
+    }
+    if (!have) return fail(PLBAMD_ENOMEM, "adjoint: cannot allocate the checkpoint and adjoint buffers");
+    char* at = buffer.p;
+    auto take = [&](uint64_t bytes) {
+        char* q = at;
+        at += aligned(bytes);
+        return q;
+    };
+    char* const work = take(stateBytes);
+    char* const lamA = take(arenaElems * lamSize);
+    char* const lamB = take(arenaElems * lamSize);
+    double* const gA = reinterpret_cast<double*>(take(cells * sizeof(double)));
+    float* const gA32 = lam64 ? nullptr : reinterpret_cast<float*>(take(cells * sizeof(float)));
+    double* const gS = reinterpret_cast<double*>(take(nScale * sizeof(double)));
+    double* const acc = reinterpret_cast<double*>(take(nAcc * sizeof(double)));
+    double* const sum = reinterpret_cast<double*>(take(8 * sizeof(double)));
+    uint16_t* const dAdjBlock = reinterpret_cast<uint16_t*>(take(adjBlock.size() * sizeof(uint16_t)));
+    uint32_t* const dAdjBegin = reinterpret_cast<uint32_t*>(take(adjBegin.size() * sizeof(uint32_t)));
+    char *ck = nullptr, *mom = nullptr, *keepMom = nullptr;
+    double *pf = nullptr, *keepPf = nullptr;
+    if (nKeep < nCk) {
+        ck = take(stateBytes * nCk);
+        mom = take(momElems * (K + 1) * lamSize);
+        pf = reinterpret_cast<double*>(take(pfElems * (K + 1) * sizeof(double)));
     }
     if (nKeep > 0) {
-        if (deviceAlloc((void**)&keepMom, keepRecs * momElems * lamSize) != hipSuccess ||
-            deviceAlloc((void**)&keepPf, keepRecs * pfElems * sizeof(double)) != hipSuccess) {
-            // the budget was not there after all: recompute everything
-            (void)hipGetLastError();
-            hipFree(keepMom);
-            hipFree(keepPf);
-            keepMom = nullptr;
-            keepPf = nullptr;
-            nKeep = 0;
-        }
+        keepMom = take(keepRecs * momElems * lamSize);
+        keepPf = reinterpret_cast<double*>(take(keepRecs * pfElems * sizeof(double)));
+    }
+    hipError_t err = hipSuccess;
+    if (L.multi) {
+        err = hipMemcpy(dAdjBlock, adjBlock.data(), adjBlock.size() * sizeof(uint16_t), hipMemcpyHostToDevice);
+        if (err == hipSuccess)
+            err = hipMemcpy(dAdjBegin, adjBegin.data(), adjBegin.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     }
     const int keepFirst = nCk - nKeep;   // first kept segment
     auto keepMomAt = [&](int c, int r) {
@@ -168,12 +222,12 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     if (err == hipSuccess && gA32) err = hipMemsetAsync(gA32, 0, cells * sizeof(float), L.stream);
     if (err == hipSuccess) err = hipMemsetAsync(gS, 0, std::max<uint32_t>(1, L.nSpecial) * sizeof(double), L.stream);
     if (err == hipSuccess) err = hipMemsetAsync(acc, 0, nAcc * sizeof(double), L.stream);
-    // cells the odd steps skip (outermost envelope rows) keep zero moments
-    if (err == hipSuccess) err = hipMemsetAsync(mom, 0, momElems * (K + 1) * lamSize, L.stream);
+    // cells the odd steps of several blocks skip (outermost envelope rows) keep zero moments
+    if (err == hipSuccess && L.multi && mom) err = hipMemsetAsync(mom, 0, momElems * (K + 1) * lamSize, L.stream);
     const bool saveStats = L.statsOn;
     L.statsOn = false;
     float msF = 0, msB = 0;
-    if (err == hipSuccess && nKeep > 0) err = hipMemsetAsync(keepMom, 0, keepRecs * momElems * lamSize, L.stream);
+    if (err == hipSuccess && L.multi && nKeep > 0) err = hipMemsetAsync(keepMom, 0, keepRecs * momElems * lamSize, L.stream);
     // forward, with checkpoints (even time: the AA array is in natural layout);
     // the kept segments record their steps instead
     if (err == hipSuccess) err = hipEventRecord(L.ev0, L.stream);
@@ -360,28 +414,29 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     }
     double hsum[8] = {0};
     if (err == hipSuccess) err = hipMemcpyAsync(hsum, sum, sizeof(hsum), hipMemcpyDeviceToHost, L.stream);
-    std::vector<double> hgA(gradAlpha ? cells : 0), hgS(std::max<uint32_t>(1, L.nSpecial));
-    if (err == hipSuccess && gradAlpha)
-        err = hipMemcpyAsync(hgA.data(), gA, cells * sizeof(double), hipMemcpyDeviceToHost, L.stream);
+    std::vector<double> hgS(nScale);
     if (err == hipSuccess) err = hipMemcpyAsync(hgS.data(), gS, hgS.size() * sizeof(double), hipMemcpyDeviceToHost, L.stream);
     std::vector<SpecialCell> hs(L.nSpecial);
     if (err == hipSuccess && L.nSpecial)
         err = hipMemcpyAsync(hs.data(), L.dSpecial, L.nSpecial * sizeof(SpecialCell), hipMemcpyDeviceToHost, L.stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(L.stream);
-    release();
+    // the stream is empty before the buffer goes back, on every path
+    const hipError_t end = hipStreamSynchronize(L.stream);
+    if (err == hipSuccess) err = end;
     if (err != hipSuccess) return fail(PLBAMD_EHIP, std::string("adjoint: ") + hipGetErrorString(err));
     if (Jout) *Jout = hsum[0];
     if (gradAlpha) {
         // bulk cells of every block to the global [nx][ny][nz] array
-        const int ny = L.desc.ny, nz = L.desc.nz;
-        for (const BlockGeom& g : L.geom)
-            for (int x = g.bx0; x <= g.bx1; ++x)
-                for (int y = g.by0; y <= g.by1; ++y)
-                    for (int z = g.bz0; z <= g.bz1; ++z) {
-                        const uint64_t local = ((uint64_t)x * g.ny + y) * g.nz + z;
-                        const uint64_t glob = ((uint64_t)(g.gx0 + x) * ny + (g.gy0 + y)) * nz + (g.gz0 + z);
-                        gradAlpha[glob] = hgA[g.cellOffset + local];
-                    }
+        const plbamd_box all{0, L.desc.nx - 1, 0, L.desc.ny - 1, 0, L.desc.nz - 1};
+        const HostPart part{reinterpret_cast<char*>(gradAlpha), sizeof(double)};
+        PLBAMD_TRY(hostTransfer(L, all, &part, 1, false, [&](const plbamd_box& k, void* const* staged, hipStream_t stream) {
+            for (size_t bi = 0; bi < L.geom.size(); ++bi) {
+                BoxArgs box;
+                if (!boxArgs(L, bi, k, box)) continue;
+                hipLaunchKernelGGL(gradient_box, gridFor((uint64_t)box.ilx * box.ily * box.ilz), dim3(256), 0, stream, gA, box,
+                                   (double*)staged[0]);
+            }
+            return hipGetLastError();
+        }));
     }
     if (gradScale) {
         // plane of each special record from its value index

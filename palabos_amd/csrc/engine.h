@@ -107,7 +107,8 @@ struct Lattice {
     std::vector<double> hostAlpha;    // per domain cell, or empty
     double solidRho[3] = {1.0, 1.0, 1.0};  // density parameter of BounceBack, NoDynamics, momentum exchange
 
-    bool dirty = true;                // device tags / specials / porosity need a rebuild
+    bool dirty = true;                // device tags / specials / porosity need a rebuild,
+    bool tagsDirty = true;            // and not of the porosity alone
     bool anyWrapped = false;
     uint8_t* dTags = nullptr;
     SpecialCell* dSpecial = nullptr;
@@ -159,11 +160,16 @@ struct Lattice {
     uint32_t* dInfo = nullptr;
     uint32_t* dIndex = nullptr;
     void* dPre = nullptr;
+    // the adjoint's buffer between its calls (under spareMutex; adjoint.hip)
+    char* adjointBuf = nullptr;
+    uint64_t adjointBufBytes = 0;
     bool anySolid = false;         // link-wall solids
     bool nodeBesideWall = false;   // and nodes or boundary objects: single steps
 
     void releaseSpare() {
-        hipFree(spare); hipFree(dInfo); hipFree(dIndex); hipFree(dPre);
+        hipFree(spare); hipFree(dInfo); hipFree(dIndex); hipFree(dPre); hipFree(adjointBuf);
+        adjointBuf = nullptr;
+        adjointBufBytes = 0;
         spare = dPre = nullptr;
         dInfo = dIndex = nullptr;
     }
@@ -188,8 +194,8 @@ struct Recording {
     double* specialF = nullptr;
 };
 
-// hipMalloc that, short of memory, takes back the second arrays of the lattices
-// that no call is using and tries again.
+// hipMalloc that, short of memory, takes back the second arrays and adjoint buffers
+// of the lattices that no call is using and tries again.
 hipError_t deviceAlloc(void** p, size_t bytes);
 void releaseSpares();
 

@@ -71,7 +71,7 @@ void releaseSpares() {
     for (auto& e : g_lattices) {
         Lattice& L = *e.second;
         std::unique_lock<std::mutex> use(L.spareMutex, std::try_to_lock);
-        if (!use.owns_lock() || !L.spare) continue;
+        if (!use.owns_lock() || !(L.spare || L.adjointBuf)) continue;
         (void)hipStreamSynchronize(L.stream);
         L.releaseSpare();
     }
@@ -576,10 +576,60 @@ int buildProcessors(Lattice& L, const std::vector<int>& planeOf, const std::vect
     return PLBAMD_OK;
 }
 
+template<typename T>
+static __global__ void __launch_bounds__(256) store_porosity(T* alpha, const double* from, uint64_t n) {
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) alpha[t] = (T)from[t];
+}
+
+// The porosity on the device in the arithmetic type of the storage (FP32 below FP64
+// storage): the kernels use it converted to that, so the values are the same. In one
+// block its order is the host's, and a kernel takes it from the transfer's chunks (an
+// optimization sets it before every run: 3.1 million cells 1 ms, where the walk over
+// all cells of the host took 30); the envelopes of several blocks are filled here.
+template<typename T>
+static int uploadPorosity(Lattice& L) {
+    if (L.hostAlpha.empty()) {
+        hipFree(L.dAlpha);
+        L.dAlpha = nullptr;
+        return PLBAMD_OK;
+    }
+    if (!L.dAlpha) PLBAMD_HIP(deviceAlloc(&L.dAlpha, L.allocCells * sizeof(T)));
+    PLBAMD_HIP(hipStreamSynchronize(L.stream));
+    const int nx = L.desc.nx, ny = L.desc.ny, nz = L.desc.nz;
+    if (!L.multi) {
+        const plbamd_box all{0, nx - 1, 0, ny - 1, 0, nz - 1};
+        const HostPart part{reinterpret_cast<char*>(L.hostAlpha.data()), sizeof(double)};
+        return hostTransfer(L, all, &part, 1, true, [&](const plbamd_box& k, void* const* staged, hipStream_t stream) {
+            const uint64_t n = boxCells(k);   // a run of cells
+            hipLaunchKernelGGL(store_porosity<T>, itemsGrid(n), dim3(256), 0, stream,
+                               (T*)L.dAlpha + ((uint64_t)k.x0 * ny + k.y0) * nz + k.z0, (const double*)staged[0], n);
+            return hipGetLastError();
+        });
+    }
+    std::vector<T> alpha(L.allocCells, T(0));
+    auto wrapped = [](int v, int n) { return ((v % n) + n) % n; };
+    for (const BlockGeom& g : L.geom)
+        for (int lx = 0; lx < g.nx; ++lx)
+            for (int ly = 0; ly < g.ny; ++ly) {
+                const double* row =
+                    &L.hostAlpha[((uint64_t)wrapped(g.gx0 + lx, nx) * ny + wrapped(g.gy0 + ly, ny)) * nz];
+                T* out = &alpha[g.cellOffset + ((uint64_t)lx * g.ny + ly) * g.nz];
+                for (int lz = 0; lz < g.nz; ++lz) out[lz] = (T)row[wrapped(g.gz0 + lz, nz)];
+            }
+    PLBAMD_HIP(hipMemcpy(L.dAlpha, alpha.data(), alpha.size() * sizeof(T), hipMemcpyHostToDevice));
+    return PLBAMD_OK;
+}
+
 // Builds the device tags, the special-cell list and the porosity array of every
 // block from the domain-wide description (tags, planes, porosity).
 int rebuild(Lattice& L) {
     if (!L.dirty) return PLBAMD_OK;
+    if (!L.tagsDirty) {
+        PLBAMD_TRY(L.desc.storage == PLBAMD_F64 ? uploadPorosity<double>(L) : uploadPorosity<float>(L));
+        L.dirty = false;
+        return PLBAMD_OK;
+    }
     if (L.anyCopy && L.dValues) {
         // the copy processors rewrote the stored values on the device: keep them
         for (size_t p = 0; p < L.planeValueBase.size() && p < L.planes.size(); ++p)
@@ -624,12 +674,10 @@ int rebuild(Lattice& L) {
     }
     std::vector<uint8_t> dev(L.allocCells, BT_BULK);
     std::vector<uint32_t> walls;   // allocated on the first cell next to a link wall
-    std::vector<double> alpha;
-    if (!L.hostAlpha.empty()) alpha.assign(L.allocCells, 0.0);
     std::vector<SpecialCell> special;
     bool anyNonBulk = anyPlane;
     L.anyWrapped = false;
-    for (size_t bi = 0; bi < L.geom.size(); ++bi) {
+    for (size_t bi = 0; bi < L.geom.size() && (haveTags || anyPlane); ++bi) {
         const BlockGeom& g = L.geom[bi];
         for (int lx = 0; lx < g.nx; ++lx)
             for (int ly = 0; ly < g.ny; ++ly)
@@ -639,7 +687,6 @@ int rebuild(Lattice& L) {
                     const uint64_t c = at(x, y, z);
                     const uint64_t local = ((uint64_t)lx * g.ny + ly) * g.nz + lz;
                     const uint64_t slot = g.cellOffset + local;
-                    if (!alpha.empty()) alpha[slot] = L.hostAlpha[c];
                     const uint8_t t = tagOf(c);
                     const int p = anyPlane ? planeOf[c] : -1;
                     if (t == PLBAMD_TAG_WALL_LINK) { dev[slot] = BT_SKIP; anyNonBulk = true; continue; }
@@ -709,7 +756,6 @@ int rebuild(Lattice& L) {
     hipFree(L.dSpecial); L.dSpecial = nullptr;
     hipFree(L.dValues); L.dValues = nullptr;
     hipFree(L.dSpecialPartials); L.dSpecialPartials = nullptr;
-    hipFree(L.dAlpha); L.dAlpha = nullptr;
     hipFree(L.dWalls); L.dWalls = nullptr;
     L.nSpecial = (uint32_t)special.size();
     if (anyNonBulk) {
@@ -730,18 +776,7 @@ int rebuild(Lattice& L) {
         PLBAMD_HIP(deviceAlloc((void**)&L.dValues, values.size() * sizeof(double)));
         PLBAMD_HIP(hipMemcpy(L.dValues, values.data(), values.size() * sizeof(double), hipMemcpyHostToDevice));
     }
-    if (!alpha.empty()) {
-        // in the arithmetic type of the storage (FP32 below FP64 storage): the
-        // kernels use the porosity converted to it, so the values are the same
-        if (L.desc.storage == PLBAMD_F64) {
-            PLBAMD_HIP(deviceAlloc((void**)&L.dAlpha, alpha.size() * sizeof(double)));
-            PLBAMD_HIP(hipMemcpy(L.dAlpha, alpha.data(), alpha.size() * sizeof(double), hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> a32(alpha.begin(), alpha.end());
-            PLBAMD_HIP(deviceAlloc((void**)&L.dAlpha, a32.size() * sizeof(float)));
-            PLBAMD_HIP(hipMemcpy(L.dAlpha, a32.data(), a32.size() * sizeof(float), hipMemcpyHostToDevice));
-        }
-    }
+    PLBAMD_TRY(L.desc.storage == PLBAMD_F64 ? uploadPorosity<double>(L) : uploadPorosity<float>(L));
     {
         // the words of the fused steps follow the tags: built anew by the next call
         std::lock_guard<std::mutex> use(L.spareMutex);
@@ -757,7 +792,7 @@ int rebuild(Lattice& L) {
         L.anySolid = solid;
         L.nodeBesideWall = solid && other;
     }
-    L.dirty = false;
+    L.dirty = L.tagsDirty = false;
     return PLBAMD_OK;
 }
 
@@ -1167,11 +1202,11 @@ int plbamd_lattice_destroy(int handle) {
 int plbamd_set_tags(int handle, const uint8_t* tags) {
     Lattice* L = find(handle);
     if (!L) return fail(PLBAMD_EINVAL, "set_tags: unknown handle");
-    if (!tags) { L->hostTags.clear(); L->dirty = true; return PLBAMD_OK; }
+    if (!tags) { L->hostTags.clear(); L->dirty = L->tagsDirty = true; return PLBAMD_OK; }
     for (uint64_t k = 0; k < L->cells; ++k)
         if (tags[k] > PLBAMD_TAG_WALL_LINK) return fail(PLBAMD_EINVAL, "set_tags: unknown tag value");
     L->hostTags.assign(tags, tags + L->cells);
-    L->dirty = true;
+    L->dirty = L->tagsDirty = true;
     return PLBAMD_OK;
 }
 
@@ -1194,7 +1229,7 @@ int plbamd_add_plane(int handle, int family, int kind, int dir, int ori, const p
     if (kind == PLBAMD_PRESSURE) std::fill(p.values.begin(), p.values.end(), 1.0);
     L->planes.push_back(p);
     if (plane) *plane = (int)L->planes.size() - 1;
-    L->dirty = true;
+    L->dirty = L->tagsDirty = true;
     return PLBAMD_OK;
 }
 
@@ -1203,7 +1238,7 @@ static int addBoundaryObject(Lattice& L, const Plane& p, int* id) {
         return fail(PLBAMD_EINVAL, "boundaries are not combined with a body force");
     L.planes.push_back(p);
     if (id) *id = (int)L.planes.size() - 1;
-    L.dirty = true;
+    L.dirty = L.tagsDirty = true;
     return PLBAMD_OK;
 }
 
@@ -1249,7 +1284,7 @@ int plbamd_set_boundary_type(int handle, int id, int bc_type) {
     if (bc_type < PLBAMD_BC_DIRICHLET || bc_type > PLBAMD_BC_NORMAL_OUTFLOW)
         return fail(PLBAMD_EINVAL, "set_boundary_type: unknown boundary type");
     L->planes[id].bcType = bc_type;
-    L->dirty = true;
+    L->dirty = L->tagsDirty = true;
     return PLBAMD_OK;
 }
 
@@ -1283,7 +1318,7 @@ int plbamd_set_plane_values(int handle, int plane, const double* values, size_t 
                              hipMemcpyHostToDevice));
         return PLBAMD_OK;
     }
-    L->dirty = true;
+    L->dirty = L->tagsDirty = true;
     return PLBAMD_OK;
 }
 
