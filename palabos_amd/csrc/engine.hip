@@ -803,18 +803,22 @@ int rebuild(Lattice& L) {
 // of it hits in L2), and those it writes; rows that do not start on 64-byte
 // boundaries write lines in parts. Against 900 timed combinations of tile and
 // chunk on eleven lattices (64^3 to 384x256x256, 191x203x197 among them) the
-// choice is 0.4 % (FP64) and 4 % (FP32) from the fastest on average, 5 % and
-// 19 % at worst; the fewest tiles alone chose 18x23 cells at 160^3 (FP64 218 us a
-// step; with 10x40 144 us).
-static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size) {
-    const int wgsPerCU = size == 8 ? 1 : 2;     // by registers
-    const double rim = size == 8 ? 0.3 : 0.5, slots = 256.0 * wgsPerCU;
+// choice is 1-5 % from the fastest; the fewest tiles alone chose 18x23 cells at
+// 160^3 (FP64 218 us a step; with 10x40 144 us). FP64 with edges or tags: at most 64
+// cells wide (72^3 with edges 19.6 -> 16.3 us), and with special cells, whose tiles take
+// longer, half a round more, which prefers shorter chunks (channel 192x96x96
+// 100 -> 90, 256x128x128 194 -> 182, 256x160x160 270 -> 280).
+static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, bool specials) {
+    const int threads = fused_threads(std::max<size_t>(4, size));
+    const double rim = size == 8 ? 0.3 : 0.5, slots = 256.0;
     const bool rowLines = g.nz * size % 128 == 0;
     Lattice::FusedPlan best;
     double least = 1e300;
-    for (int width = 8; width <= 128; width += 2) {
+    const double waves = specials && size == 8 ? 0.5 : 0.0;
+    for (int width = 8; width <= (info && size == 8 ? 64 : 128); width += 2) {
         const int w = std::min(width, g.nz), tz = (g.nz + w - 1) / w;
-        int rows = kFusedThreads / (w + 2) - 2;
+        int rows = threads / (w + 2) - 2;
+        if (rows < 1) break;
         const int ty = (g.ny + rows - 1) / rows;
         rows = (g.ny + ty - 1) / ty;
         const bool aligned = rowLines && w * size % 64 == 0, lines = rowLines && w * size % 128 == 0;
@@ -824,7 +828,7 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size) {
         for (int chunks = 1; chunks <= g.nx; ++chunks) {
             const int len = (g.nx + chunks - 1) / chunks;
             const double wgs = (double)ty * tz * ((g.nx + len - 1) / len);
-            const double cost = std::ceil(wgs / slots) * (len + 2.5) * bytes;
+            const double cost = (std::ceil(wgs / slots) + waves) * (len + 2.5) * bytes;
             if (cost >= least) continue;
             least = cost;
             best.rows = rows + 2; best.cols = w + 2; best.tilesY = ty; best.tilesZ = tz; best.len = len;
@@ -837,38 +841,40 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size) {
 // Whether the next steps may be taken two at a time (fused.h), with the second
 // array allocated: one block, no boundary processors, no link walls together
 // with nodes, a second array of at most an eighth of the free device memory, and
-// a lattice on which it is the faster way. us a step on n^3 lattices, single ->
-// fused, with each side's cache policy:
-//   FP64   periodic 64^3 12.9 -> 12.6, 72^3 19.1 -> 16.4, 96^3 40.6 -> 30.7, 112^3 64.3 -> 62.5,
-//          128^3 96.7 -> 82.7, 256^3 903 -> 642, 512^3 7357 -> 5325; with edges 64^3 13.5 ->
-//          15.0, 72^3 19.7 -> 18.7, 160^3 218 -> 148; link walls 256x160x128 323 -> 270
-//   FP32   periodic 64^3 7.7 -> 7.9, 72^3 12.9 -> 9.7, 112^3 29.8 -> 25.8, 128^3 40.3 -> 50.7 and
-//          144^3 63.9 -> 65.7 (one array fits the last-level cache, two do not), 160^3 102 ->
-//          88, 256^3 445 -> 352, 512^3 3737 -> 2831; with edges 96^3 22.4 -> 22.4, 144^3 71.7
-//          -> 75.0, 160^3 103.5 -> 98.2, 192^3 183 -> 164; not with link walls, whose
-//          reflections cost a tile more than the second pass over memory (256x160x128
-//          171 -> 193)
-//   16 bit bound by the arithmetic of two collisions where the pair kernel is not
-//          (256^3 206 -> 239): periodic lattices in the last-level cache (64^3 10.1 -> 7.3,
-//          80^3 13.7 -> 11.0, 96^3 14.4 -> 14.4), and odd nz, which has no pair kernel
-//          (191x203x197 225 -> 136)
+// a lattice on which it is the faster way. us a step, single -> fused, with each
+// side's cache policy:
+//   FP64   periodic 64^3 12.9 -> 11.7, 72^3 19.1 -> 15.5, 128^3 96.7 -> 76.6, 256^3 903 -> 612; with
+//          edges 64^3 13.5 -> 15.0, 72^3 19.7 -> 16.3, 160^3 218 -> 139; link walls 256x160x128
+//          323 -> 268
+//   FP32   periodic 56^3 7.2 -> 7.3, 64^3 7.9 -> 8.8, 72^3 12.8 -> 9.6, 112^3 29.6 -> 21.6, 128^3
+//          41.8 -> 43.9 and 144^3 62.2 -> 63.3 (one array fits the last-level cache, two do
+//          not), 160^3 105 -> 77, 256^3 447 -> 303, 320^3 970 -> 575; with edges 96^3 22.5 ->
+//          22.2, 144^3 63.1 -> 68.7, 160^3 110 -> 83, 256^3 463 -> 315; link walls 256x160x128
+//          167 -> 154. Rows that are not whole lines cost single steps more: 63x65x67
+//          11.4 -> 9.0, 129x97x75 with edges 26.2 -> 22.7, 191x203x197 298 -> 159
+//   16 bit bound by instructions where the pair kernel is not (256^3 208 -> 238, 320^3 447
+//          -> 428): periodic lattices in the last-level cache (56^3 8.0 -> 6.8, 80^3 13.8 -> 10.5,
+//          96^3 14.4 -> 14.2), and odd nz, which has no pair kernel (191x203x197 213 -> 109;
+//          with edges 234 -> 148, but 63x65x67 11.4 -> 13.1)
 // Planes and momentum-exchange nodes bring two more small launches, which single
 // steps of small lattices do without (bulk_and_special): FP64 channel 128x64x64
-// 31.1 -> 40.2, cavity 96^3 64.4 -> 56.6, channel 192x96x96 107 -> 100.
+// 31.1 -> 40.2, cavity 96^3 64.4 -> 56.6, channel 192x96x96 107 -> 90; FP32 256x128x128
+// 114.6 -> 116, 256x160x160 197 -> 149.
 // PLBAMD_FUSED=0/1 overrides the choice.
 static bool fusedReady(Lattice& L) {
     if (L.multi || L.dProc || L.nodeBesideWall) return false;
     const BlockGeom& g = L.geom[0];
     const bool needInfo = L.dTags || !(g.px && g.py && g.pz);
     const uint64_t bytes = 19 * g.slot * L.elemSize;
+    const bool lines = g.nz * L.elemSize % 128 == 0;   // rows of whole lines: the better case of single steps
     bool wanted;
     if (L.elemSize == 8) {
         wanted = L.cells >= (L.nSpecial ? 700000u : needInfo ? 370000u : 250000u);
     } else if (L.elemSize == 4) {
-        wanted = !L.anySolid && (needInfo ? bytes >= 260000000u
-                                          : L.cells >= 300000 && !(bytes > 128000000u && bytes < 230000000u));
+        wanted = needInfo ? bytes >= 300000000u || (!lines && L.cells >= 600000)
+                          : L.cells >= (lines ? 300000u : 250000u) && !(lines && bytes > 128000000u && bytes < 230000000u);
     } else {
-        wanted = !L.anySolid && (!L.pairs || (!needInfo && L.cells <= 600000));
+        wanted = L.pairs ? !needInfo && L.cells <= 600000 : !needInfo || L.cells >= 600000;
     }
     if (const char* e = getenv("PLBAMD_FUSED")) wanted = atoi(e) != 0;
     // 32-bit lane offsets: within a plane, or (reflections) over ten slots
@@ -881,7 +887,7 @@ static bool fusedReady(Lattice& L) {
             L.spare = nullptr;
             return false;
         }
-        L.fused = planFused(g, L.elemSize);
+        L.fused = planFused(g, L.elemSize, needInfo, L.nSpecial != 0);
     }
     if (needInfo && !L.dInfo) {
         bool ok = hipMalloc(&L.dInfo, L.cells * sizeof(uint32_t)) == hipSuccess;
@@ -894,6 +900,7 @@ static bool fusedReady(Lattice& L) {
             L.releaseSpare();
             return false;
         }
+        L.fused = planFused(g, L.elemSize, needInfo, L.nSpecial != 0);
     }
     return true;
 }

@@ -22,15 +22,23 @@
 // The arithmetic is the single-step kernels' (collide_bulk on the same values
 // in the same order), so the populations are bit-identical to theirs.
 //
-// Bytes per cell and two steps: 19 values read, plus the rim's share, and 19
-// written (the single steps move twice as much).
+// Bytes per cell and two steps: 19 values read, plus the rim's share (half of the
+// rim misses L2: FP64 256^3 reads 1.24 times its populations), and 19 written (the
+// single steps move twice as much). FP64 256^3 runs at 4.7 TB/s of those bytes, FP32
+// 5.0: with one workgroup per CU the loads of a plane wait for the plane before.
+// 16-bit storage is bound by instructions (57 % of the time in vector ones).
 #pragma once
 
 #include "kernels.h"
 
 namespace plbamd {
 
-constexpr int kFusedThreads = 512;
+// Threads of a workgroup: one workgroup per CU takes all its registers. `arith` is
+// the size of the arithmetic type. The larger the tile, the smaller the share of its
+// rim: two workgroups of 512 threads per CU instead of one of 1024 cost FP32 256^3
+// 348 us a step instead of 303, 200^3 185 instead of 148 (FP16 122 instead of 107);
+// FP64 has registers for 512 threads only (768 spill: 652 instead of 612).
+constexpr int fused_threads(size_t arith) { return arith == 8 ? 512 : 1024; }
 
 // Per-cell word of lattices with edges or tags: bit i (1-18) set where f_i comes
 // back from the cell's own f*_opp(i) (a non-periodic edge or a link wall at
@@ -44,7 +52,7 @@ struct FusedArgs {
     uint64_t slot;
     int nx, ny, nz;
     int px, py, pz;
-    int rows, cols;           // tile with its rim: rows * cols <= kFusedThreads
+    int rows, cols;           // tile with its rim: rows * cols <= fused_threads
     int tilesY, tilesZ;
     int len;                  // planes along x per workgroup
     double omega;
@@ -118,12 +126,13 @@ __device__ __forceinline__ void fused_collide(const FusedArgs& a, uint64_t cell,
 // plane k + 1 where they are written: moved up, they would be live through a
 // collision.
 template<typename S, int DYN, bool INFO, bool FORCED>
-__global__ void __launch_bounds__(kFusedThreads)
-    __attribute__((amdgpu_waves_per_eu(sizeof(typename Store<S>::T) == 8 ? 2 : 4))) fused_two_steps(FusedArgs a) {
+__global__ void __launch_bounds__(fused_threads(sizeof(typename Store<S>::T)))
+    __attribute__((amdgpu_waves_per_eu(fused_threads(sizeof(typename Store<S>::T)) / 256))) fused_two_steps(FusedArgs a) {
     using T = typename Store<S>::T;
+    constexpr int kThreads = fused_threads(sizeof(T));
     using R = typename Store<S>::R;
     extern __shared__ __align__(16) unsigned char ldsRaw[];
-    R* lds = reinterpret_cast<R*>(ldsRaw);     // [19][kFusedThreads]
+    R* lds = reinterpret_cast<R*>(ldsRaw);     // [19][kThreads]
     const uint32_t wg = xcd_item(blockIdx.x, gridDim.x);
     const uint32_t tiles = (uint32_t)a.tilesY * a.tilesZ;
     const uint32_t chunk = wg / tiles, tile = wg % tiles;
@@ -219,14 +228,18 @@ __global__ void __launch_bounds__(kFusedThreads)
         const bool planeOk = act && shift(k, 0, a.nx, a.px, xk);
         const uint32_t kind = word >> kFusedKind;
         T g[19];
-        if (planeOk) {
 #pragma unroll
-            for (int i = 0; i < 19; ++i) g[i] = Store<S>::from_raw(next[i]);
-            fused_collide<S, DYN, FORCED>(a, (uint64_t)xk * plane + ownCell, kind, g);
-        }
+        for (int i = 0; i < 19; ++i) g[i] = Store<S>::from_raw(next[i]);
+        // plane k + 1 goes out before plane k is collided: its loads are in flight
+        // through both collisions and the barriers (issued after the barriers: FP64
+        // 128^3 83 us a step, now 77; 256^3 632, now 612)
+        __builtin_amdgcn_sched_barrier(0);
+        if (k < xb) gather(k + 1, wordNext, recNext);
+        __builtin_amdgcn_sched_barrier(0);
+        if (planeOk) fused_collide<S, DYN, FORCED>(a, (uint64_t)xk * plane + ownCell, kind, g);
         __builtin_amdgcn_sched_barrier(0);
         // what plane k - 1 (in LDS) sends to its own cells and to plane k
-        auto arriving = [&](int i) -> R { return lds[i * kFusedThreads + (t - cy(i) * a.cols - cz(i))]; };
+        auto arriving = [&](int i) -> R { return lds[i * kThreads + (t - cy(i) * a.cols - cz(i))]; };
         R p1[19], hold[19];
         if (inner && k >= xa) {
             if (!INFO || __ballot(wordPrev & 0x7ffffu) == 0) {
@@ -246,14 +259,14 @@ __global__ void __launch_bounds__(kFusedThreads)
                 for (int i = 0; i < 19; ++i) {
                     const bool back = (wordPrev >> i) & 1u;
                     if (cx(i) > 0) {
-                        const R v = lds[opp(i) * kFusedThreads + here];
+                        const R v = lds[opp(i) * kThreads + here];
                         hold[i] = back ? v : p2[i];
-                        p1[i] = lds[i * kFusedThreads + (here - cy(i) * a.cols - cz(i))];
+                        p1[i] = lds[i * kThreads + (here - cy(i) * a.cols - cz(i))];
                     } else if (cx(i) == 0) {
-                        hold[i] = lds[here + (back ? opp(i) * kFusedThreads
-                                                   : i * kFusedThreads - cy(i) * a.cols - cz(i))];
+                        hold[i] = lds[here + (back ? opp(i) * kThreads
+                                                   : i * kThreads - cy(i) * a.cols - cz(i))];
                     } else {
-                        refl[i] = lds[opp(i) * kFusedThreads + here];
+                        refl[i] = lds[opp(i) * kThreads + here];
                     }
                 }
             }
@@ -261,13 +274,12 @@ __global__ void __launch_bounds__(kFusedThreads)
         __syncthreads();   // plane k - 1 is read
         if (planeOk) {
 #pragma unroll
-            for (int i = 0; i < 19; ++i) lds[i * kFusedThreads + t] = Store<S>::to_raw(g[i]);
+            for (int i = 0; i < 19; ++i) lds[i * kThreads + t] = Store<S>::to_raw(g[i]);
         }
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t wordAhead = (k + 2 <= xb) ? infoOf(a.info, k + 2) : 0u;
         const uint32_t recAhead = (specials && k + 2 <= xb) ? infoOf(a.index, k + 2) : 0u;
-        if (k < xb) gather(k + 1, wordNext, recNext);
         __builtin_amdgcn_sched_barrier(0);
         if (inner && k >= xa) {
             if (k > xa) {

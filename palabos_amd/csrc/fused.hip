@@ -9,7 +9,7 @@
 
 namespace plbamd {
 
-// FP64 tiles take 76 KB of LDS, above the default limit per workgroup.
+// FP64 and FP32 tiles take 76 KB of LDS, above the default limit per workgroup.
 template<typename K>
 static int allowLds(K kernel, size_t bytes) {
     if (bytes > 65536)
@@ -22,7 +22,8 @@ template<typename S, int DYN>
 int launchFused(Lattice& L, FusedOp op) {
     const BlockGeom& g = L.geom[0];
     const bool forced = L.dAlpha || L.desc.force[0] != 0 || L.desc.force[1] != 0 || L.desc.force[2] != 0;
-    const size_t lds = 19 * (size_t)kFusedThreads * sizeof(typename Store<S>::R);
+    constexpr int threads = fused_threads(sizeof(typename Store<S>::T));
+    const size_t lds = 19 * (size_t)threads * sizeof(typename Store<S>::R);
     if (op == FUSED_PREPARE) {
         PLBAMD_TRY(allowLds(fused_two_steps<S, DYN, false, false>, lds));
         PLBAMD_TRY(allowLds(fused_two_steps<S, DYN, false, true>, lds));
@@ -72,7 +73,7 @@ int launchFused(Lattice& L, FusedOp op) {
     a.index = L.dIndex;
     a.outputs = L.dPre;
     a.nSpecial = L.nSpecial;
-    const dim3 grid((unsigned)(a.tilesY * a.tilesZ * ((g.nx + a.len - 1) / a.len))), block(kFusedThreads);
+    const dim3 grid((unsigned)(a.tilesY * a.tilesZ * ((g.nx + a.len - 1) / a.len))), block(threads);
     if (L.dInfo) {
         if (forced) hipLaunchKernelGGL((fused_two_steps<S, DYN, true, true>), grid, block, lds, L.stream, a);
         else hipLaunchKernelGGL((fused_two_steps<S, DYN, true, false>), grid, block, lds, L.stream, a);

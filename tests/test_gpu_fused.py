@@ -113,3 +113,10 @@ def test_walls_beside_nodes_keep_single_steps(gpu):
     want, _ = oracle.run(case, f0, 6)
     got, _ = fused_run(case, f0, [6])
     assert np.array_equal(got[~solid], want[~solid])
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("periodic", [(True, True, True), (False, False, False)])
+@pytest.mark.parametrize("shape", [(5, 70, 150), (40, 34, 66), (3, 65, 128)])
+def test_several_tiles_of_1024_threads(gpu, storage, periodic, shape):
+    check(Case(*shape, storage=storage, omega=1.7, periodic=periodic), [6])
