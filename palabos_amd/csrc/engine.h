@@ -79,6 +79,7 @@ struct Lattice {
     uint16_t* dWgBlock = nullptr;   // block of every bulk work item (multi-block)
     uint32_t* dWalls = nullptr;     // link-wall mask per allocated cell (cells next to link walls)
     bool linearEven = false;        // even steps through bulk_even_linear
+    bool linearOdd = false;         // odd steps through bulk_odd_linear
     uint64_t nEven = 0;             // its workgroups
     uint16_t* dEvenBlock = nullptr; // its block of every workgroup (multi-block)
     CopyTask* dTasks = nullptr;     // envelope exchange: one workgroup per task

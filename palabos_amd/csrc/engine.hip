@@ -19,6 +19,12 @@ namespace plbamd {
 // 256x128x128 -10 % (FP32) and -11 % (FP64); the 384x256x256 porous medium
 // (FP16) -3 %.
 constexpr uint64_t kCachedZCells = uint64_t(1) << 26;
+// Populations of several blocks up to which their odd steps run in memory order
+// (bulk_odd_linear; us a step, rows -> memory order): FP32 64^3 in 2 / 8 blocks 14.4 -> 8.7 /
+// 21.3 -> 18.3, 129x97x75 in 12 54.7 -> 51.4, 128^3 in 8 87.6 -> 77.5; FP64 128^3 (380 MB) 171 ->
+// 162; beyond the last-level cache the shifted stores write lines in parts (FP32
+// 192x128x256 in 4 blocks, 520 MB, 233 -> 249, 256^3 in 8 702 -> 799).
+constexpr uint64_t kLinearOddBytes = 400000000;
 // Populations up to which the loads are ordinary too (policy 2; figures in kernels.h).
 constexpr uint64_t kCachedBytes = 256000000;
 
@@ -298,6 +304,8 @@ int setup(Lattice& L) {
             ew += ((uint64_t)g.nx * g.ny * g.nz + perWG - 1) / perWG;
         }
         if (ew >= (1ull << 31)) L.linearEven = false;
+        L.linearOdd = L.linearEven && storageSize(d.storage) >= 4 && offset * storageSize(d.storage) <= kLinearOddBytes;
+        if (const char* e = getenv("PLBAMD_LINEAR_ODD")) L.linearOdd = L.linearOdd && atoi(e) != 0;
         L.nEven = ew;
     }
     L.elemSize = storageSize(d.storage);

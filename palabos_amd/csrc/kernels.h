@@ -592,6 +592,85 @@ __device__ __forceinline__ void odd_cell_general(const StepArgs& a, const BlockG
     }
 }
 
+// ---------------------------------------------------------------------------
+// Odd step of several blocks over each block's cells in memory order, as
+// bulk_even_linear: the rows of a lattice cut into blocks are short, and the staged
+// kernel, one row per workgroup, leaves lanes idle (blocks of 129x97x75 FP32: 38 %) and
+// is bound by its instructions. Here a lane's populations are at a scalar slot address
+// and one 32-bit lane offset each, computed once: the cell gathers f_i where it later
+// scatters f*_opp(i) (slot opp(i) of x - c_i, or its own slot i where that is beyond an
+// edge or a link wall). Needs the populations within 4 GB (kLinearOddBytes is less).
+template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, int POLICY>
+__global__ void __launch_bounds__(512) bulk_odd_linear(StepArgs a) {
+    using T = typename Store<S>::T;
+    constexpr bool PLAIN = POLICY == 2;
+    const uint32_t wg = blockIdx.x;
+    const int b = a.evenBlock ? (int)a.evenBlock[wg] : 0;
+    const BlockGeom g = a.blocks[b];
+    S* __restrict__ f = reinterpret_cast<S*>(a.arena) + g.offset;
+    const uint32_t plane = (uint32_t)g.ny * (uint32_t)g.nz, cells = (uint32_t)g.nx * plane;
+    const uint32_t cell = (wg - g.evenBegin) * blockDim.x + threadIdx.x;
+    double st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double wf[3] = {0, 0, 0};
+    if (cell < cells) {
+        const int x = (int)(cell / plane);
+        const uint32_t rem = cell % plane;
+        const int y = (int)(rem / (uint32_t)g.nz), z = (int)(rem % (uint32_t)g.nz);
+        uint8_t tag = BT_BULK;
+        uint32_t wall = 0;
+        if constexpr (TAGS) {
+            tag = a.tags[g.cellOffset + cell];
+            if (a.walls) wall = a.walls[g.cellOffset + cell];
+        }
+        // the outermost envelope layer is not collided (see bulk_odd_staged)
+        const bool outer = outer_envelope_row(g, x, y) || (g.bz0 > 1 && z == 0) || (g.bz1 < g.nz - 2 && z == g.nz - 1);
+        if (tag != BT_SKIP && !outer) {
+            int xs[3] = {x, x, x}, ys[3] = {y, y, y}, zs[3] = {z, z, z};
+            // directions whose source x - c_i is beyond an edge or a link wall
+            uint32_t beyond = ((wall >> 9) & 0x3feu) | ((wall & 0x3feu) << 9);
+            auto edge = [&](bool in, int axis, int sign) {
+                uint32_t m = 0;
+#pragma unroll
+                for (int i = 1; i < 19; ++i)
+                    if (ci(i, axis) == -sign) m |= 1u << i;
+                if (!in) beyond |= m;
+            };
+            edge(shift(x, -1, g.nx, g.px, xs[0]), 0, -1);
+            edge(shift(x, 1, g.nx, g.px, xs[2]), 0, 1);
+            edge(shift(y, -1, g.ny, g.py, ys[0]), 1, -1);
+            edge(shift(y, 1, g.ny, g.py, ys[2]), 1, 1);
+            edge(shift(z, -1, g.nz, g.pz, zs[0]), 2, -1);
+            edge(shift(z, 1, g.nz, g.pz, zs[2]), 2, 1);
+            uint32_t ox[3], oy[3], oz[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                ox[k] = (uint32_t)xs[k] * plane * (uint32_t)sizeof(S);
+                oy[k] = (uint32_t)ys[k] * (uint32_t)g.nz * (uint32_t)sizeof(S);
+                oz[k] = (uint32_t)zs[k] * (uint32_t)sizeof(S);
+            }
+            const uint32_t slotBytes = (uint32_t)(g.slot * sizeof(S));
+            const uint32_t own = cell * (uint32_t)sizeof(S);
+            uint32_t off[19];
+            T fc[19];
+            off[0] = own;
+#pragma unroll
+            for (int i = 1; i < 19; ++i) {
+                const uint32_t there = ox[1 - cx(i)] + oy[1 - cy(i)] + oz[1 - cz(i)] + (uint32_t)opp(i) * slotBytes;
+                off[i] = ((beyond >> i) & 1u) ? own + (uint32_t)i * slotBytes : there;
+            }
+#pragma unroll
+            for (int i = 0; i < 19; ++i) fc[i] = ld<S, PLAIN>(at(f, off[i]));
+            collide_cell<S, DYN, STATS, FORCED, false>(a, g, cell, tag, in_bulk(g, x, y, z), fc, st, wall, wf);
+#pragma unroll
+            for (int i = 0; i < 19; ++i) {
+                if constexpr (POLICY >= 1) Store<S>::store_raw_cached(at(f, off[opp(i)]), Store<S>::to_raw(fc[i]));
+                else Store<S>::store(at(f, off[opp(i)]), fc[i]);
+            }
+        }
+    }
+    store_bulk_stats<STATS, FORCED>(st, wf, a.partials, wg, a.walls);
+}
+
 // Index of direction i among the z-moving directions, or -1.
 __host__ __device__ constexpr int zmove_index(int i) {
     int k = 0;

@@ -106,6 +106,22 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
 #undef PLBAMD_EV_F
 #undef PLBAMD_EV
         }
+    } else if (odd && L.linearOdd && !record) {
+        if constexpr (sizeof(typename Store<S>::R) >= 4) {
+            a.evenBlock = L.dEvenBlock;
+            const dim3 eg((unsigned)L.nEven), eb(kEvenThreads);
+#define PLBAMD_OD(TG, ST, FO)                                                                                       \
+    do {                                                                                                            \
+        if (L.policy == 2) hipLaunchKernelGGL((bulk_odd_linear<S, DYN, TG, ST, FO, 2>), eg, eb, 0, L.stream, a);    \
+        else hipLaunchKernelGGL((bulk_odd_linear<S, DYN, TG, ST, FO, 1>), eg, eb, 0, L.stream, a);                  \
+    } while (0)
+#define PLBAMD_OD_F(TG, ST) do { if (forced) PLBAMD_OD(TG, ST, true); else PLBAMD_OD(TG, ST, false); } while (0)
+#define PLBAMD_OD_S(TG) do { if (stats) PLBAMD_OD_F(TG, true); else PLBAMD_OD_F(TG, false); } while (0)
+            if (tags) PLBAMD_OD_S(true); else PLBAMD_OD_S(false);
+#undef PLBAMD_OD_S
+#undef PLBAMD_OD_F
+#undef PLBAMD_OD
+        }
     } else if (record) {
         a.moments = record->moments;
         a.momStride = record->momStride;
@@ -247,7 +263,7 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
         // two levels when there are many records (a single workgroup reading
         // 65536 records took 40 % of a 256^3 step): kStatsLevel1 workgroups in a
         // fixed order, then one
-        const uint64_t nb = (!odd && L.linearEven) ? L.nEven : L.nBulkPartials;
+        const uint64_t nb = (odd ? L.linearOdd && !record : L.linearEven) ? L.nEven : L.nBulkPartials;
         const double* bulk = L.dBulkPartials;
         uint64_t nr = nb;
         if (nb > 4 * kStatsLevel1) {
