@@ -14,11 +14,13 @@ recomputed.
 
 value        MLUPS = cells * steps / wall seconds / 1e6 over the timed steps,
              populations resident in HBM before the timed region starts.
-roofline     the collide-and-stream launches: algorithmic bytes per launch
-             (read + write 19 populations per cell) / average launch duration,
-             measured with HIP events on the stream the kernels run on; one
-             launch per step (even and odd steps alternate two kernels).
-             "traffic" is the HBM bytes per launch from rocprofv3 counters
+roofline     the collide-and-stream launches: the bytes they have to move / their
+             time, measured with HIP events on the stream the kernels run on. At
+             this size FP64 and FP32 take two steps per launch and so read and
+             write the 19 populations of a cell once per two steps; 16-bit storage
+             takes one step per launch (even and odd steps alternate two kernels).
+             "algorithmic_bytes_per_cell" is per step; "traffic" is the HBM bytes
+             per launch from rocprofv3 counters
              (profiles/bulk_step_tg512_counters.txt).
 cpu_baseline the compiled Palabos reference (oracle/_ref/ref_driver, serial) on a
              bounded sample (periodic BGK FP64 128^3): "value" is the aggregate
@@ -45,13 +47,16 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-BYTES_PER_CELL = {"f64": 19 * 2 * 8, "f32": 19 * 2 * 4, "f16": 19 * 2 * 2, "bf16": 19 * 2 * 2}
-# The launches that make one step at this workload (even / odd steps alternate;
-# the roofline figure is their average launch duration).
-KERNELS = {"f64": "plbamd::bulk_step (even) / plbamd::bulk_odd_staged (odd)",
-           "f32": "plbamd::bulk_step (even) / plbamd::bulk_odd_staged (odd)",
+# Bytes a step has to move per cell: 19 populations read and written once per step,
+# or once per two steps where one launch takes both.
+BYTES_PER_CELL = {"f64": 19 * 8, "f32": 19 * 4, "f16": 19 * 2 * 2, "bf16": 19 * 2 * 2}
+# The launches at this workload (the first and the last step of a call with an even
+# number of steps are single ones).
+KERNELS = {"f64": "plbamd::fused_two_steps (two steps)",
+           "f32": "plbamd::fused_two_steps (two steps)",
            "f16": "plbamd::bulk_even_linear (even) / plbamd::bulk_pairs (odd)",
            "bf16": "plbamd::bulk_even_linear (even) / plbamd::bulk_pairs (odd)"}
+STEPS_PER_LAUNCH = {"f64": 2, "f32": 2, "f16": 1, "bf16": 1}
 
 
 def taylor_green_init(lat, n, u0):
@@ -297,7 +302,8 @@ def main():
         "roofline": {"bound": "hbm", "achieved": main_run["achieved_gbs"], "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": main_run["frac"], "traffic": traffic,
                      "kernel": KERNELS[args.precision], "algorithmic_bytes_per_cell": BYTES_PER_CELL[args.precision],
-                     "event_ms_per_launch": main_run["event_ms_per_step"]},
+                     "steps_per_launch": STEPS_PER_LAUNCH[args.precision],
+                     "event_ms_per_launch": main_run["event_ms_per_step"] * STEPS_PER_LAUNCH[args.precision]},
         "variants": variants,
     }
     if not args.no_adjoint:

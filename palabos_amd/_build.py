@@ -101,21 +101,24 @@ def build_cpp_examples(verbose=False):
 
 
 def resource_usage(storage, dyn, match=None):
-    """The compiler's figures for the step kernels of one translation unit
+    """The compiler's figures for the step kernels of one storage and dynamics
     (gfx950 device pass with -Rpass-analysis=kernel-resource-usage): per
     kernel, VGPRs, SGPRs, spills, static LDS and the occupancy in waves per SIMD
     that the register count allows. Returns [(demangled name, {field: value})]."""
     import re
     include = ["-I", os.path.join(ROOT, "include")]
-    cmd = ([HIPCC] + FLAGS + include + [f"-DPLBAMD_S={storage}", f"-DPLBAMD_DYN={dyn}", "--cuda-device-only",
-            "-Rpass-analysis=kernel-resource-usage", "-c", os.path.join(CSRC, "step.hip"), "-o", os.devnull])
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + res.stderr)
+    report = ""
+    for src in ("step.hip", "fused.hip"):
+        cmd = ([HIPCC] + FLAGS + include + [f"-DPLBAMD_S={storage}", f"-DPLBAMD_DYN={dyn}", "--cuda-device-only",
+                "-Rpass-analysis=kernel-resource-usage", "-c", os.path.join(CSRC, src), "-o", os.devnull])
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        if res.returncode != 0:
+            raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + res.stderr)
+        report += res.stderr
     fields = {"VGPRs": "vgpr", "TotalSGPRs": "sgpr", "VGPRs Spill": "vgpr_spill",
               "LDS Size [bytes/block]": "static_lds", "Occupancy [waves/SIMD]": "waves_per_simd"}
     out = []
-    for block in res.stderr.split("remark: Function Name: ")[1:]:
+    for block in report.split("remark: Function Name: ")[1:]:
         name = block.split()[0]
         demangled = subprocess.run(["c++filt", name], capture_output=True, text=True).stdout.strip() or name
         if match and not re.search(match, demangled):
