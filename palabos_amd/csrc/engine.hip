@@ -812,8 +812,10 @@ int rebuild(Lattice& L) {
 // boundaries write lines in parts. Against 900 timed combinations of tile and
 // chunk on eleven lattices (64^3 to 384x256x256, 191x203x197 among them) the
 // choice is 1-5 % from the fastest; the fewest tiles alone chose 18x23 cells at
-// 160^3 (FP64 218 us a step; with 10x40 144 us). FP64 with edges or tags: at most 64
-// cells wide (72^3 with edges 19.6 -> 16.3 us), and with special cells, whose tiles take
+// 160^3 (FP64 218 us a step; with 10x40 144 us). With edges or tags, at most 64 cells
+// wide for FP64 (72^3 19.6 -> 16.3 us) and 126 otherwise, as every wavefront of a
+// whole-row tile holds edges (FP32 256x128x128 with edges 105 -> 89, channel 117 -> 110,
+// link walls 256x160x128 154 -> 159); FP64 with special cells, whose tiles take
 // longer, half a round more, which prefers shorter chunks (channel 192x96x96
 // 100 -> 90, 256x128x128 194 -> 182, 256x160x160 270 -> 280).
 static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, bool specials) {
@@ -823,7 +825,7 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
     Lattice::FusedPlan best;
     double least = 1e300;
     const double waves = specials && size == 8 ? 0.5 : 0.0;
-    for (int width = 8; width <= (info && size == 8 ? 64 : 128); width += 2) {
+    for (int width = 8; width <= (info ? (size == 8 ? 64 : 126) : 128); width += 2) {
         const int w = std::min(width, g.nz), tz = (g.nz + w - 1) / w;
         int rows = threads / (w + 2) - 2;
         if (rows < 1) break;
@@ -858,7 +860,7 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
 //          41.8 -> 43.9 and 144^3 62.2 -> 63.3 (one array fits the last-level cache, two do
 //          not), 160^3 105 -> 77, 256^3 447 -> 303, 320^3 970 -> 575; with edges 96^3 22.5 ->
 //          22.2, 144^3 63.1 -> 68.7, 160^3 110 -> 83, 256^3 463 -> 315; link walls 256x160x128
-//          167 -> 154. Rows that are not whole lines cost single steps more: 63x65x67
+//          167 -> 159. Rows that are not whole lines cost single steps more: 63x65x67
 //          11.4 -> 9.0, 129x97x75 with edges 26.2 -> 22.7, 191x203x197 298 -> 159
 //   16 bit bound by instructions where the pair kernel is not (256^3 208 -> 238, 320^3 447
 //          -> 428): periodic lattices in the last-level cache (56^3 8.0 -> 6.8, 80^3 13.8 -> 10.5,
@@ -867,7 +869,7 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
 // Planes and momentum-exchange nodes bring two more small launches, which single
 // steps of small lattices do without (bulk_and_special): FP64 channel 128x64x64
 // 31.1 -> 40.2, cavity 96^3 64.4 -> 56.6, channel 192x96x96 107 -> 90; FP32 256x128x128
-// 114.6 -> 116, 256x160x160 197 -> 149.
+// 114.6 -> 110, 256x160x160 197 -> 149.
 // PLBAMD_FUSED=0/1 overrides the choice.
 static bool fusedReady(Lattice& L) {
     if (L.multi || L.dProc || L.nodeBesideWall) return false;
