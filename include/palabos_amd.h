@@ -364,6 +364,19 @@ int plbamd_set_adjoint_record_bytes(int handle, int64_t bytes);
  * sweep, and the device bytes of those records. No Palabos counterpart. */
 int plbamd_get_adjoint_record_info(int handle, int* kept_segments, int64_t* bytes);
 
+/* How the lattice runs: counts since it was created and what it holds, for
+ * tests and benchmarks that say which way a call took (the results do not depend
+ * on it). out: PLBAMD_NUM_RUN_INFO values. No Palabos counterpart. */
+#define PLBAMD_RUN_TWO_STEP_LAUNCHES 0  /* launches that took two steps at once               */
+#define PLBAMD_RUN_KEPT_BYTES 1         /* device bytes kept between calls to make them faster: the
+                                           second population array and its tables, the adjoint's buffer */
+#define PLBAMD_RUN_PINNED_TRANSFERS 2   /* transfers of host arrays through pinned memory      */
+#define PLBAMD_RUN_PAGEABLE_TRANSFERS 3 /* and without it                                     */
+#define PLBAMD_RUN_SLOT_STRIDE 4        /* elements from one population's array to the next (first block) */
+#define PLBAMD_RUN_CACHE_POLICY 5       /* 0: nontemporal accesses, 1: ordinary stores along z, 2: ordinary loads too */
+#define PLBAMD_NUM_RUN_INFO 6
+int plbamd_get_run_info(int handle, int64_t* out);
+
 /* Number of completed steps. */
 int plbamd_get_time(int handle, int64_t* t);
 

@@ -165,8 +165,15 @@ struct Lattice {
     char* adjointBuf = nullptr;
     uint64_t adjointBufBytes = 0;
     bool anySolid = false;         // link-wall solids
+    // what ran, for plbamd_get_run_info
+    int64_t twoStepLaunches = 0, pinnedTransfers = 0, pageableTransfers = 0;
     bool nodeBesideWall = false;   // and nodes or boundary objects: single steps
 
+    // device bytes held by all of these (under spareMutex)
+    uint64_t keptBytes() const {
+        return (spare ? 19 * geom[0].slot * elemSize : 0) + (dInfo ? 4 * cells : 0) + (dIndex ? 4 * cells : 0) +
+               (dPre ? 19 * (uint64_t)nSpecial * elemSize : 0) + adjointBufBytes;
+    }
     void releaseSpare() {
         hipFree(spare); hipFree(dInfo); hipFree(dIndex); hipFree(dPre); hipFree(adjointBuf);
         adjointBuf = nullptr;

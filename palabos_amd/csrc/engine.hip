@@ -951,6 +951,7 @@ int step(Lattice& L, int nsteps) {
         const bool odd = (L.time & 1) != 0;
         if (fused && odd && nsteps - s - (L.statsOn ? 1 : 0) >= 2) {
             PLBAMD_TRY(fusedDispatch(L, FUSED_STEPS));
+            ++L.twoStepLaunches;
             L.time += 2;
             ++s;
             continue;
@@ -1514,6 +1515,19 @@ int plbamd_get_adjoint_record_info(int handle, int* kept_segments, int64_t* byte
     if (!L || !kept_segments || !bytes) return fail(PLBAMD_EINVAL, "get_adjoint_record_info: bad argument");
     *kept_segments = L->adjointKept;
     *bytes = L->adjointKeptBytes;
+    return PLBAMD_OK;
+}
+
+int plbamd_get_run_info(int handle, int64_t* out) {
+    Lattice* L = find(handle);
+    if (!L || !out) return fail(PLBAMD_EINVAL, "get_run_info: bad argument");
+    std::lock_guard<std::mutex> use(L->spareMutex);
+    out[PLBAMD_RUN_TWO_STEP_LAUNCHES] = L->twoStepLaunches;
+    out[PLBAMD_RUN_KEPT_BYTES] = (int64_t)L->keptBytes();
+    out[PLBAMD_RUN_PINNED_TRANSFERS] = L->pinnedTransfers;
+    out[PLBAMD_RUN_PAGEABLE_TRANSFERS] = L->pageableTransfers;
+    out[PLBAMD_RUN_SLOT_STRIDE] = (int64_t)L->geom[0].slot;
+    out[PLBAMD_RUN_CACHE_POLICY] = L->policy;
     return PLBAMD_OK;
 }
 

@@ -67,7 +67,9 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     char* onDevice = nullptr;
     if (slots) {
         lock = std::unique_lock<std::mutex>(slots->use);
+        ++L.pinnedTransfers;
     } else {
+        ++L.pageableTransfers;
         pageable.resize(chunkBytes);
         onDevice = static_cast<char*>(buf.get(chunkBytes));
         if (!onDevice) return fail(PLBAMD_ENOMEM, "transfer: cannot allocate a staging buffer");

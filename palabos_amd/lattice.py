@@ -416,6 +416,14 @@ class Block3D:
         check(lib().plbamd_get_adjoint_record_info(self.handle, ctypes.byref(n), ctypes.byref(b)))
         return n.value, b.value
 
+    def runInfo(self):
+        """Which way the lattice's calls took (the results do not depend on it): a dict
+        of two_step_launches, kept_bytes (device memory held between calls),
+        pinned_transfers, pageable_transfers, slot_stride and cache_policy."""
+        out = np.zeros(len(native.RUN_INFO), dtype=np.int64)
+        check(lib().plbamd_get_run_info(self.handle, out.ctypes.data))
+        return dict(zip(native.RUN_INFO, out.tolist()))
+
     def toggleInternalStatistics(self, on):
         check(lib().plbamd_toggle_statistics(self.handle, int(bool(on))))
 

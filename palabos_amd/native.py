@@ -22,6 +22,8 @@ KEEP_BLOCKS = 1           # plbamd_multiblock_create_ex: keep the given blocks
 BC_TYPES = {"dirichlet": 0, "neumann": 1, "freeslip": 2, "density": 3, "outflow": 4, "normalOutflow": 5}
 VELOCITY, PRESSURE = 0, 1
 NUM_STATS = 10
+RUN_INFO = ("two_step_launches", "kept_bytes", "pinned_transfers", "pageable_transfers", "slot_stride",
+            "cache_policy")
 
 STORAGE_CODES = {"f64": F64, "f32": F32, "f16": F16, "bf16": BF16}
 STORAGE_NUMPY = {"f64": np.float64, "f32": np.float32, "f16": np.uint16, "bf16": np.uint16}
@@ -37,7 +39,7 @@ EXPORTS = (
     "plbamd_adjoint_gradient", "plbamd_set_adjoint_record_bytes", "plbamd_get_adjoint_record_info", "plbamd_get_time", "plbamd_save_binary_block", "plbamd_load_binary_block",
     "plbamd_compute_fields", "plbamd_set_solid_density", "plbamd_reduce_moments_noalloc",
     "plbamd_add_velocity_edge", "plbamd_add_velocity_corner", "plbamd_set_boundary_type",
-    "plbamd_execute_processors", "plbamd_bandwidth_probe", "plbamd_multiblock_create_ex",
+    "plbamd_execute_processors", "plbamd_get_run_info", "plbamd_bandwidth_probe", "plbamd_multiblock_create_ex",
     "plbamd_get_block_count", "plbamd_compute_rhobar_j", "plbamd_get_rhobar_j", "plbamd_set_rhobar_j",
     "plbamd_external_collide_and_stream",
 )
@@ -129,6 +131,7 @@ def lib():
         "plbamd_execute_processors": [i32],
         "plbamd_compute_fields": [i32, pbox, vp],
         "plbamd_set_solid_density": [i32, i32, ctypes.c_double],
+        "plbamd_get_run_info": [i32, vp],
         "plbamd_get_time": [i32, ctypes.POINTER(ctypes.c_int64)],
         "plbamd_adjoint_gradient": [i32, i32, i32, ctypes.POINTER(Objective), vp, vp, vp, vp],
         "plbamd_set_adjoint_record_bytes": [i32, ctypes.c_int64],

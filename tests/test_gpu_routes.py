@@ -1,0 +1,72 @@
+"""Which way a call runs (plbamd_get_run_info). The ways give the same
+populations bit for bit, so the tests that compare results pass whichever was
+taken: here the counts are compared."""
+import pytest
+
+import palabos_amd as plb
+from cases import (TAG_BB, TAG_MEBB, TAG_NODYN, TAG_WALL, Case, cavity_case, channel_case, gpu_lattice,
+                   sphere_tags)
+
+pytestmark = pytest.mark.gpu
+
+
+def pairs_of(calls, stats=False):
+    """Launches of two steps in a sequence of calls: from an odd time on, as long as two steps are left that
+    need not report statistics."""
+    t = n = 0
+    for steps in calls:
+        end = t + steps
+        while t < end:
+            if t % 2 == 1 and end - t - int(stats) >= 2:
+                t, n = t + 2, n + 1
+            else:
+                t += 1
+    return n
+
+
+def two_step_launches(lat, calls, stats=False):
+    try:
+        lat.toggleInternalStatistics(stats)
+        for n in calls:
+            lat.collideAndStream(n)
+        return lat.runInfo()["two_step_launches"]
+    finally:
+        lat.close()
+
+
+def cases_with_two_steps():
+    nodes = Case(9, 17, 36, storage="f16", omega=1.8, periodic=(False, True, False))
+    nodes.tags = sphere_tags(nodes.shape, (4, 8, 30), 4.2, TAG_BB)
+    nodes.tags[2:4, 1:4, 0:3] = TAG_NODYN
+    walls = Case(10, 16, 40, storage="f32", dynamics="rbgk", omega=1.7, periodic=(True, True, True), force=(1e-4, 0.0, 0.0))
+    walls.tags = sphere_tags(walls.shape, (1, 14, 31), 4.5, TAG_WALL)
+    return [Case(1, 1, 1, omega=1.7, periodic=(True, True, True)),
+            Case(5, 14, 33, storage="bf16", omega=1.7, periodic=(True, True, True)),
+            Case(7, 16, 34, storage="f32", dynamics="rbgk", omega=1.5, periodic=(False, False, False)),
+            nodes, walls, channel_case(12, 17, 35, 1.8, 0.05, sphere=((5, 8, 31), 4.3))]
+
+
+@pytest.mark.parametrize("stats", [False, True])
+@pytest.mark.parametrize("calls", [[2], [3], [4], [5, 4], [1, 2, 3], [8]])
+@pytest.mark.parametrize("case", cases_with_two_steps(), ids=lambda c: f"{c.storage}-{c.nx}x{c.ny}x{c.nz}")
+def test_two_steps_are_launched(gpu, monkeypatch, case, calls, stats):
+    monkeypatch.setenv("PLBAMD_FUSED", "1")
+    assert two_step_launches(gpu_lattice(case), calls, stats) == pairs_of(calls, stats)
+
+
+def test_two_steps_are_left_to_single_ones(gpu, monkeypatch):
+    """Link walls beside nodes, boundary processors, several blocks, and PLBAMD_FUSED=0."""
+    monkeypatch.setenv("PLBAMD_FUSED", "1")
+    for tag in (TAG_BB, TAG_MEBB, TAG_NODYN):
+        case = Case(8, 9, 33, omega=1.7, periodic=(True, True, True))
+        case.tags = sphere_tags(case.shape, (4, 4, 10), 2.5, TAG_WALL)
+        case.tags[1, 1, 30] = tag
+        assert two_step_launches(gpu_lattice(case), [6]) == 0
+    lat = plb.Block3D(8, 9, 10, plb.D3Q19, plb.BGK(1.7), storage="f64")
+    lat.setVelocityConditionOnBlockBoundaries()
+    assert two_step_launches(lat, [6]) == 0
+    blocks = [(0, 7, 0, 8, 0, 9), (8, 15, 0, 8, 0, 9)]
+    assert two_step_launches(plb.Block3D(16, 9, 10, plb.D3Q19, plb.BGK(1.7), storage="f64", periodic=True, blocks=blocks,
+                                         keep_blocks=True), [6]) == 0
+    monkeypatch.setenv("PLBAMD_FUSED", "0")
+    assert two_step_launches(gpu_lattice(cavity_case(14, 1.4, 0.05)), [6]) == 0
