@@ -1,0 +1,30 @@
+"""Times of steps against each other, where a slip of the compiler or of the set-up
+has cost a fifth and more before. Best of several runs in one process, with room
+for the noise of small ratios."""
+import pytest
+
+import palabos_amd as plb
+
+pytestmark = pytest.mark.gpu
+
+
+def step_us(lat, steps, repeats=6):
+    lat.toggleInternalStatistics(False)
+    lat.collideAndStream(9)
+    return min(lat.collideAndStreamTimed(steps) for _ in range(repeats)) * 1e3 / steps
+
+
+def test_tagged_odd_steps_keep_their_loads_together(gpu, monkeypatch):
+    """Odd nz in 16-bit storage takes the unstaged kernel. With tags it reads one byte a
+    cell more than without (1/38 of its traffic) and tests it: 1.11 times the time, and
+    1.24 times with a wait after each of the loads."""
+    monkeypatch.setenv("PLBAMD_FUSED", "0")
+    monkeypatch.setenv("PLBAMD_CACHED_Z", "1")
+    shape, us = (191, 203, 197), []
+    for tagged in (False, True):
+        with plb.Block3D(*shape, plb.D3Q19, plb.BGK(1.8), storage="bf16", periodic=True) as lat:
+            if tagged:
+                lat.defineDynamics((0, 0, 0, shape[1] - 1, 0, shape[2] - 1), plb.BounceBack)
+            us.append(step_us(lat, 50))
+    print(f"[step time] plain {us[0]:.1f} us, tagged {us[1]:.1f} us", flush=True)
+    assert us[1] < 1.17 * us[0]
