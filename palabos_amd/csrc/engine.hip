@@ -269,12 +269,15 @@ int setup(Lattice& L) {
     for (BlockGeom& g : L.geom) {
         const uint64_t cells = (uint64_t)g.nx * g.ny * g.nz;
         if (cells >= (1ull << 32)) return fail(PLBAMD_EINVAL, "lattice_create: at most 2^32 - 1 cells per block");
-        // Slots start an odd number of 64-element runs apart, so that the 19 streams
-        // of a launch do not all start on the same memory channels where the cell
-        // count is a multiple of a large power of two (fused steps, us a step:
-        // FP64 256^3 670 -> 645, FP32 320^3 758 -> 717, FP16 320^3 493 -> 469; single
-        // steps within 1 %).
-        g.slot = (cells + 511) / 512 * 512 + 64;
+        // Where two steps are taken per launch, slots start an odd number of 64-element
+        // runs apart, so that the 19 streams of a launch do not all start on the same
+        // memory channels (us a step at n^3, unpadded -> padded: FP64 128^3 79.6 -> 76.9, 320^3
+        // 1301 -> 1180, 512^3 5209 -> 4868; FP32 256^3 319 -> 307, 512^3 2930 -> 2544). Single steps
+        // gain nothing by it, and those of 16-bit storage lose (FP16 256^3 201 -> 211, 384^3
+        // 759 -> 778, 512^3 1770 -> 1814; two steps per launch the same): 16-bit lattices and
+        // several blocks, which take single steps, are not padded.
+        g.slot = (cells + 63) / 64 * 64;
+        if (storageSize(d.storage) >= 4 && !L.multi) g.slot = (cells + 511) / 512 * 512 + 64;
         g.offset = offset;
         g.cellOffset = cellOffset;
         g.nzChunks = (g.nz + L.zChunk - 1) / L.zChunk;

@@ -70,3 +70,15 @@ def test_two_steps_are_left_to_single_ones(gpu, monkeypatch):
                                          keep_blocks=True), [6]) == 0
     monkeypatch.setenv("PLBAMD_FUSED", "0")
     assert two_step_launches(gpu_lattice(cavity_case(14, 1.4, 0.05)), [6]) == 0
+
+
+def test_slots_are_padded_where_two_steps_are_taken(gpu):
+    """16-bit lattices and several blocks, whose single steps the padding slows down, have none."""
+    def stride(storage, **kw):
+        with plb.Block3D(32, 24, 40, plb.D3Q19, plb.BGK(1.7), storage=storage, periodic=True, **kw) as lat:
+            return lat.runInfo()["slot_stride"]
+    cells = 32 * 24 * 40
+    assert stride("f64") % 128 == stride("f32") % 128 == 64
+    assert stride("f16") == stride("bf16") == cells
+    blocks = [(0, 31, 0, 11, 0, 39), (0, 31, 12, 23, 0, 39)]
+    assert stride("f32", blocks=blocks, keep_blocks=True) == 36 * 16 * 44   # two envelope layers a side
