@@ -317,6 +317,11 @@ int setup(Lattice& L) {
     // kCachedZCells cells, ordinary loads up to kCachedBytes of populations
     // (PLBAMD_CACHED_Z=0/1/2 overrides)
     L.policy = bytes <= kCachedBytes ? 2 : (cellOffset <= kCachedZCells ? 1 : 0);
+    // 16-bit storage between 6 and 19 MB of populations: ordinary loads cost up to 13 %
+    // there (us a step of n^3, policy 1 -> 2: FP16 RBGK 48^3 7.21 -> 7.01, 56^3 8.71 -> 8.91, 68^3
+    // 10.92 -> 11.93, 76^3 14.2 -> 15.8, 80^3 15.1 -> 15.3, 84^3 16.0 -> 15.3; BF16 BGK 48^3 7.49 ->
+    // 7.35, 64^3 9.73 -> 10.21, 76^3 13.5 -> 15.3, 84^3 15.2 -> 14.3)
+    if (storageSize(d.storage) == 2 && cellOffset >= 150000 && cellOffset < 500000) L.policy = 1;
     if (const char* e = getenv("PLBAMD_CACHED_Z")) L.policy = std::max(0, std::min(2, atoi(e)));
     if (deviceAlloc(&L.arena, bytes) != hipSuccess) {
         (void)hipGetLastError();

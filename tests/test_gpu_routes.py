@@ -82,3 +82,12 @@ def test_slots_are_padded_where_two_steps_are_taken(gpu):
     assert stride("f16") == stride("bf16") == cells
     blocks = [(0, 31, 0, 11, 0, 39), (0, 31, 12, 23, 0, 39)]
     assert stride("f32", blocks=blocks, keep_blocks=True) == 36 * 16 * 44   # two envelope layers a side
+
+
+@pytest.mark.parametrize("storage, n, policy", [
+    ("f64", 64, 2), ("f32", 64, 2), ("f16", 48, 2), ("f16", 56, 1), ("f16", 76, 1), ("f16", 84, 2), ("bf16", 48, 2),
+    ("bf16", 56, 1), ("bf16", 76, 1), ("bf16", 84, 2), ("bf16", 65, 1)])
+def test_cache_policy_of_small_lattices(gpu, storage, n, policy):
+    """Ordinary loads (2) in the last-level cache, except 16-bit lattices of 6 to 19 MB, where they cost time."""
+    with plb.Block3D(n, n, n, plb.D3Q19, plb.BGK(1.7), storage=storage, periodic=True) as lat:
+        assert lat.runInfo()["cache_policy"] == policy
