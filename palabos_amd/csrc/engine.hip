@@ -870,10 +870,20 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
 //          22.2, 144^3 63.1 -> 68.7, 160^3 110 -> 83, 256^3 463 -> 315; link walls 256x160x128
 //          167 -> 159. Rows that are not whole lines cost single steps more: 63x65x67
 //          11.4 -> 9.0, 129x97x75 with edges 26.2 -> 22.7, 191x203x197 298 -> 159
-//   16 bit bound by instructions where the pair kernel is not (256^3 208 -> 238, 320^3 447
-//          -> 428): periodic lattices in the last-level cache (56^3 8.0 -> 6.8, 80^3 13.8 -> 10.5,
-//          96^3 14.4 -> 14.2), and odd nz, which has no pair kernel (191x203x197 213 -> 109;
-//          with edges 234 -> 148, but 63x65x67 11.4 -> 13.1)
+//          Regularized BGK or a force: periodic 68x75x62 11.0 -> 11.7, 60x88x64 with force 11.5 ->
+//          13.2, 68x66x90 16.6 -> 17.6, 72^3 14.5 -> 11.8, 80^3 16.8 -> 14.1; edges 146x51x84 25.9 -> 27.5
+//   16 bit bound by instructions, the more so with a force, regularized BGK, edges or tags.
+//          Even nz (pair kernel): FP16 BGK alone, periodic 56^3 7.8 -> 6.7, 64^3 9.4 -> 8.5,
+//          72^3 11.7 -> 8.7, 83x66x66 12.1 -> 8.5, 84^3 13.9 -> 12.3, but 44x93x128 10.9 -> 11.9 (long
+//          rows, few in a tile), 32^3 4.9 -> 5.7, 96^3 14.3 -> 14.2, 256^3 201 -> 238; RBGK 64^3 10.2 ->
+//          11.3; BF16 64^3 9.6 -> 10.9, RBGK 32^3 6.4 -> 8.4. Odd nz (one cell per thread), 150 random
+//          shapes a kind, single/fused: FP16 periodic 0.8-1.4 below 10^6 cells and 1.07-2.1 from
+//          there on, with edges or tags 0.8-1.7 below 3 10^6 and 1.0-1.6 beyond; BF16 periodic
+//          0.6-1.4 below 1.25 10^6 and 1.06-1.7 beyond, with edges or tags 0.5-1.4 in the last-level
+//          cache (6.7 10^6 cells) and 1.0-1.5 beyond (191x203x197 with nodes 218 -> 159)
+//   A force on FP64 with edges or tags (two collisions with it and the cell's word in
+//   178 registers): link walls 80^3 31.3 -> 25.9, 96^3 47.6 -> 47.2, 112^3 69.9 -> 83.7, 128^3 105.9 ->
+//   115.3, 160^3 229 -> 199; 97^3 55.1 -> 56.3, 129^3 159 -> 124
 // Planes and momentum-exchange nodes bring two more small launches, which single
 // steps of small lattices do without (bulk_and_special): FP64 channel 128x64x64
 // 31.1 -> 40.2, cavity 96^3 64.4 -> 56.6, channel 192x96x96 107 -> 90; FP32 256x128x128
@@ -886,13 +896,21 @@ static bool fusedReady(Lattice& L) {
     const uint64_t bytes = 19 * g.slot * L.elemSize;
     const bool lines = g.nz * L.elemSize % 128 == 0;   // rows of whole lines: the better case of single steps
     bool wanted;
+    const bool forced = L.dAlpha || L.desc.force[0] != 0 || L.desc.force[1] != 0 || L.desc.force[2] != 0;
+    const bool heavy = forced || L.desc.dynamics != PLBAMD_BGK;   // more instructions a cell
     if (L.elemSize == 8) {
-        wanted = L.cells >= (L.nSpecial ? 700000u : needInfo ? 370000u : 250000u);
+        wanted = L.cells >= (L.nSpecial ? 700000u : needInfo ? 370000u : 250000u) &&
+                 !(needInfo && forced && L.cells >= 800000 && (lines ? L.cells < 3000000 : bytes <= kCachedBytes));
     } else if (L.elemSize == 4) {
-        wanted = needInfo ? bytes >= 300000000u || (!lines && L.cells >= 600000)
-                          : L.cells >= (lines ? 300000u : 250000u) && !(lines && bytes > 128000000u && bytes < 230000000u);
+        wanted = needInfo ? bytes >= 300000000u || (!lines && L.cells >= (heavy ? 900000u : 600000u))
+                          : L.cells >= (heavy ? 430000u : lines ? 300000u : 250000u) &&
+                                !(lines && bytes > 128000000u && bytes < 230000000u);
     } else {
-        wanted = L.pairs ? !needInfo && L.cells <= 600000 : !needInfo || L.cells >= 600000;
+        const bool f16 = L.desc.storage == PLBAMD_F16;
+        if (L.pairs)
+            wanted = f16 && !heavy && !needInfo && L.cells >= 250000 && L.cells <= 600000 && g.nz <= 96;
+        else
+            wanted = L.cells >= (needInfo ? (f16 ? 3000000u : 6700000u) : (f16 ? 1000000u : 1250000u));
     }
     if (const char* e = getenv("PLBAMD_FUSED")) wanted = atoi(e) != 0;
     // 32-bit lane offsets: within a plane, or (reflections) over ten slots

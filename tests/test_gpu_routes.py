@@ -91,3 +91,33 @@ def test_cache_policy_of_small_lattices(gpu, storage, n, policy):
     """Ordinary loads (2) in the last-level cache, except 16-bit lattices of 6 to 19 MB, where they cost time."""
     with plb.Block3D(n, n, n, plb.D3Q19, plb.BGK(1.7), storage=storage, periodic=True) as lat:
         assert lat.runInfo()["cache_policy"] == policy
+
+
+@pytest.mark.parametrize("storage, shape, kind, dynamics, force, taken", [
+    # 16-bit, two cells per thread: FP16 BGK without edges, tags or force, 250,000 to 600,000 cells, rows up to 96
+    ("f16", (32, 32, 32), "periodic", "bgk", False, False), ("f16", (72, 72, 72), "periodic", "bgk", False, True),
+    ("f16", (96, 96, 96), "periodic", "bgk", False, False), ("f16", (44, 93, 128), "periodic", "bgk", False, False),
+    ("f16", (72, 72, 72), "periodic", "rbgk", False, False), ("f16", (72, 72, 72), "periodic", "bgk", True, False),
+    ("f16", (72, 72, 72), "box", "bgk", False, False), ("bf16", (72, 72, 72), "periodic", "bgk", False, False),
+    # 16-bit, one cell per thread (odd nz)
+    ("f16", (83, 85, 87), "periodic", "rbgk", False, False), ("f16", (101, 101, 101), "periodic", "rbgk", False, True),
+    ("f16", (129, 131, 133), "box", "bgk", False, False), ("f16", (149, 151, 153), "box", "bgk", True, True),
+    ("bf16", (101, 101, 101), "periodic", "bgk", False, False), ("bf16", (109, 109, 109), "periodic", "rbgk", False, True),
+    ("bf16", (149, 151, 153), "box", "bgk", False, False), ("bf16", (191, 203, 197), "box", "bgk", False, True),
+    # FP32: regularized BGK or a force from 430,000 cells on; with edges and rows of broken lines from 900,000
+    ("f32", (68, 75, 62), "periodic", "rbgk", False, False), ("f32", (68, 75, 62), "periodic", "bgk", False, True),
+    ("f32", (60, 88, 64), "periodic", "bgk", True, False), ("f32", (80, 80, 80), "periodic", "rbgk", False, True),
+    ("f32", (97, 99, 101), "box", "rbgk", True, True), ("f32", (83, 85, 87), "box", "rbgk", False, False),
+    ("f32", (83, 85, 87), "box", "bgk", False, True),
+    # FP64 with edges or tags: with a force not between 800,000 and 3,000,000 cells (whole lines; the cache otherwise)
+    ("f64", (80, 80, 80), "box", "rbgk", True, True), ("f64", (112, 112, 112), "box", "rbgk", True, False),
+    ("f64", (128, 128, 128), "walls", "rbgk", True, False), ("f64", (112, 112, 112), "box", "rbgk", False, True),
+    ("f64", (112, 112, 112), "periodic", "rbgk", True, True), ("f64", (97, 99, 101), "box", "rbgk", True, False),
+    ("f64", (129, 131, 133), "walls", "rbgk", True, True), ("f64", (160, 160, 160), "walls", "rbgk", True, True)])
+def test_two_steps_where_they_are_the_faster_way(gpu, monkeypatch, storage, shape, kind, dynamics, force, taken):
+    monkeypatch.delenv("PLBAMD_FUSED", raising=False)
+    dyn = plb.BGK(1.7) if dynamics == "bgk" else plb.RegularizedBGK(1.7)
+    lat = plb.Block3D(*shape, plb.D3Q19, dyn, storage=storage, periodic=kind != "box", force=(1e-5, 0.0, 0.0) if force else None)
+    if kind == "walls":
+        lat.defineDynamics((5, 5, 5, 5, 5, 5), plb.WallLink)
+    assert two_step_launches(lat, [5]) == (2 if taken else 0)
