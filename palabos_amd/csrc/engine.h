@@ -71,6 +71,7 @@ struct HostSlots;   // hostio.h
 struct Lattice {
     plbamd_lattice_desc desc;
     std::shared_ptr<HostSlots> hostSlots;   // once a transfer has used them
+    bool noPinned = false;                  // they could not be had: not tried again
     int device = -1;                  // HIP device the lattice lives on
     bool multi = false;
     std::vector<plbamd_box> bulk;     // global bulk box of each block

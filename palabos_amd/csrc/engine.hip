@@ -53,23 +53,29 @@ HostSlots::~HostSlots() {
 std::shared_ptr<HostSlots> hostSlots(Lattice& L) {
     static std::mutex table;
     static std::map<int, std::weak_ptr<HostSlots>> byDevice;
+    // the way without pinned memory, for its test: whatever slots other lattices hold
+    if (L.noPinned || getenv("PLBAMD_NO_PINNED")) return nullptr;
     if (L.hostSlots) return L.hostSlots;
-    std::lock_guard<std::mutex> lock(table);
-    std::shared_ptr<HostSlots> s = byDevice[L.device].lock();
-    if (!s) {
-        s = std::make_shared<HostSlots>();
-        s->device = L.device;
-        bool ok = hipHostMalloc((void**)&s->pinned, HostSlots::kSlots * HostSlots::kBytes, hipHostMallocDefault) == hipSuccess &&
-                  !getenv("PLBAMD_NO_PINNED");   // the way without pinned memory, for its test
-        for (hipStream_t& q : s->stream) ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
-        if (!ok) {
-            (void)hipGetLastError();
-            return nullptr;
+    try {
+        std::lock_guard<std::mutex> lock(table);
+        std::shared_ptr<HostSlots> s = byDevice[L.device].lock();
+        if (!s) {
+            s = std::make_shared<HostSlots>();
+            s->device = L.device;
+            bool ok = hipHostMalloc((void**)&s->pinned, HostSlots::kSlots * HostSlots::kBytes, hipHostMallocDefault) == hipSuccess;
+            for (hipStream_t& q : s->stream) ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
+            if (!ok) {
+                (void)hipGetLastError();
+                L.noPinned = true;
+                return nullptr;
+            }
+            byDevice[L.device] = s;
         }
-        byDevice[L.device] = s;
+        L.hostSlots = s;
+    } catch (const std::bad_alloc&) {
+        return nullptr;
     }
-    L.hostSlots = s;
-    return s;
+    return L.hostSlots;
 }
 
 void releaseSpares() {

@@ -13,6 +13,7 @@
 #define PALABOS_AMD_HOSTIO_H
 
 #include <atomic>
+#include <new>
 #include <thread>
 
 #include "engine.h"
@@ -62,7 +63,7 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     const uint64_t chunks = nX * nY * nZ;
     std::shared_ptr<HostSlots> slots = hostSlots(L);
     std::unique_lock<std::mutex> lock;
-    std::vector<char> pageable;     // without pinned memory: through ordinary memory and a device chunk
+    std::unique_ptr<char[]> pageable;   // without pinned memory: through ordinary memory and a device chunk
     DeviceBuffers buf;
     char* onDevice = nullptr;
     if (slots) {
@@ -70,7 +71,8 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
         ++L.pinnedTransfers;
     } else {
         ++L.pageableTransfers;
-        pageable.resize(chunkBytes);
+        pageable.reset(new (std::nothrow) char[chunkBytes]);
+        if (!pageable) return fail(PLBAMD_ENOMEM, "transfer: out of host memory");
         onDevice = static_cast<char*>(buf.get(chunkBytes));
         if (!onDevice) return fail(PLBAMD_ENOMEM, "transfer: cannot allocate a staging buffer");
     }
@@ -121,7 +123,7 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
         }
     }
     if (slots) work(slots->slot(0), slots->stream[0]);
-    else work(pageable.data(), L.stream);
+    else work(pageable.get(), L.stream);
     for (std::thread& t : helpers) t.join();
     if (error.load() != (int)hipSuccess)
         return fail(PLBAMD_EHIP, std::string("transfer: ") + hipGetErrorString((hipError_t)error.load()));
