@@ -13,7 +13,9 @@
 #define PALABOS_AMD_HOSTIO_H
 
 #include <atomic>
+#include <condition_variable>
 #include <new>
+#include <optional>
 #include <thread>
 
 #include "engine.h"
@@ -21,16 +23,43 @@
 namespace plbamd {
 
 // The slots and streams of one device: shared by its lattices, made by the first
-// transfer, freed with the last lattice. One transfer at a time uses them.
+// transfer, freed with the last lattice. A transfer takes a slot for each of its
+// chunks, and who waits longest gets the next one: a small read does not wait for
+// another lattice's gigabytes, but for one of their chunks.
 struct HostSlots {
     static constexpr int kSlots = 8;
     static constexpr size_t kBytes = 4u << 20;
-    std::mutex use;
     int device = -1;
     char* pinned = nullptr;
     hipStream_t stream[kSlots] = {};
     ~HostSlots();
     char* slot(int k) { return pinned + (size_t)k * kBytes; }
+    // a free slot for one chunk, in the order of asking
+    struct Use {
+        HostSlots& s;
+        int k;
+        explicit Use(HostSlots& slots) : s(slots) {
+            std::unique_lock<std::mutex> lock(s.mutex);
+            const uint64_t ticket = s.asked++;
+            s.freed.wait(lock, [&] { return ticket == s.served && s.nFree > 0; });
+            ++s.served;
+            k = s.freeSlot[--s.nFree];
+            if (s.served != s.asked && s.nFree > 0) s.freed.notify_all();
+        }
+        ~Use() {
+            std::lock_guard<std::mutex> lock(s.mutex);
+            s.freeSlot[s.nFree++] = k;
+            if (s.served != s.asked) s.freed.notify_all();
+        }
+        Use(const Use&) = delete;
+        Use& operator=(const Use&) = delete;
+    };
+
+private:
+    std::mutex mutex;
+    std::condition_variable freed;
+    uint64_t asked = 0, served = 0;
+    int freeSlot[kSlots] = {7, 6, 5, 4, 3, 2, 1, 0}, nFree = kSlots;
 };
 // Null when the pinned memory cannot be had.
 std::shared_ptr<HostSlots> hostSlots(Lattice& L);
@@ -62,12 +91,10 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     const uint64_t nX = (lx + sx - 1) / sx, nY = (ly + sy - 1) / sy, nZ = (lz + sz - 1) / sz;
     const uint64_t chunks = nX * nY * nZ;
     std::shared_ptr<HostSlots> slots = hostSlots(L);
-    std::unique_lock<std::mutex> lock;
     std::unique_ptr<char[]> pageable;   // without pinned memory: through ordinary memory and a device chunk
     DeviceBuffers buf;
     char* onDevice = nullptr;
     if (slots) {
-        lock = std::unique_lock<std::mutex>(slots->use);
         ++L.pinnedTransfers;
     } else {
         ++L.pageableTransfers;
@@ -78,8 +105,12 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     }
     std::atomic<uint64_t> next{0};
     std::atomic<int> error{(int)hipSuccess};
-    auto work = [&](char* slot, hipStream_t stream) {
+    auto work = [&]() {
         for (uint64_t c; error.load() == (int)hipSuccess && (c = next.fetch_add(1)) < chunks;) {
+            std::optional<HostSlots::Use> use;
+            if (slots) use.emplace(*slots);
+            char* const slot = slots ? slots->slot(use->k) : pageable.get();
+            const hipStream_t stream = slots ? slots->stream[use->k] : L.stream;
             const uint64_t ix = c / (nY * nZ), iy = c / nZ % nY, iz = c % nZ;
             plbamd_box k;
             k.x0 = b.x0 + (int)(ix * sx); k.x1 = std::min<int>(b.x1, k.x0 + (int)sx - 1);
@@ -113,17 +144,16 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     const int want = slots ? (int)std::min<uint64_t>(HostSlots::kSlots, chunks) : 1;
     for (int k = 1; k < want; ++k) {
         try {
-            helpers.emplace_back([&, k] {
+            helpers.emplace_back([&] {
                 const hipError_t err = hipSetDevice(L.device);
-                if (err == hipSuccess) work(slots->slot(k), slots->stream[k]);
+                if (err == hipSuccess) work();
                 else error.store((int)err);
             });
         } catch (...) {
             break;   // no more threads to be had: those there are do the work
         }
     }
-    if (slots) work(slots->slot(0), slots->stream[0]);
-    else work(pageable.get(), L.stream);
+    work();
     for (std::thread& t : helpers) t.join();
     if (error.load() != (int)hipSuccess)
         return fail(PLBAMD_EHIP, std::string("transfer: ") + hipGetErrorString((hipError_t)error.load()));

@@ -1,5 +1,7 @@
 """Transfers of host arrays next to each other (csrc/hostio.h): lattices of one
 device share pinned slots."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -31,3 +33,50 @@ def test_without_pinned_memory_beside_a_lattice_that_has_it(gpu, monkeypatch):
         monkeypatch.delenv("PLBAMD_NO_PINNED")
         assert np.array_equal(lat.getPopulations(), 2 * f)
         assert lat.runInfo()["pinned_transfers"] == 2
+
+
+def test_a_small_read_does_not_wait_for_another_lattices_transfer(gpu):
+    """One cell's read waits for a chunk of the other transfer (4 MB), not for its 1.3 GB of populations."""
+    with lattice((204, 204, 204)) as big, lattice((8, 8, 8)) as small:
+        small.macroscopic((1, 1, 1, 1, 1, 1))
+        big.getPopulations((0, 0, 0, 203, 0, 203))
+        done = threading.Event()
+
+        def transfer():
+            try:
+                big.getPopulations()
+            finally:
+                done.set()
+        t = threading.Thread(target=transfer)
+        reads = 0
+        t.start()
+        while not done.is_set():
+            small.macroscopic((1, 1, 1, 1, 1, 1))
+            reads += 1
+        t.join()
+        print(f"[transfers] {reads} reads beside one transfer", flush=True)
+        assert reads >= 10   # some hundred; one or two when they wait for all of it
+
+
+def test_transfers_of_many_threads(gpu):
+    """More transfers at once than there are slots, each of several chunks: every array arrives whole."""
+    shape, n = (40, 64, 96), 12
+    lats = [lattice(shape) for _ in range(n)]
+    try:
+        f = [0.02 * uniform(shape + (19,), 5 + k) for k in range(n)]
+        wrong = []
+
+        def go(k):
+            for _ in range(3):
+                lats[k].setPopulations(f[k])
+                if not np.array_equal(lats[k].getPopulations(), f[k]):
+                    wrong.append(k)
+        threads = [threading.Thread(target=go, args=(k,)) for k in range(n)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert wrong == []
+    finally:
+        for lat in lats:
+            lat.close()
