@@ -4,13 +4,15 @@
 // (up) here: the runtime stages it through its own pinned buffer and copies on one
 // thread, which also takes the page faults of a fresh array. A chunk here is a
 // run of cells whose kernel reads or writes a pinned slot directly over the bus
-// (57 GB/s), and several host threads, each with a slot and a stream, move the
+// (57 GB/s), and several host threads, each chunk with a slot and a stream, move the
 // chunks between slots and the caller's arrays: the populations of 128^3 FP64
 // cells (319 MB) come down in 7.4 ms instead of 34.8 and go up in 6.0 instead of
-// 19.1, their density and velocity (67 MB) in 2.0 instead of 7.8. No staging
-// memory on the device.
+// 19.1, their density and velocity (67 MB) in 2.0 instead of 7.8. Only uploads of
+// 3 to 48 MB take memory on the device (kCopiedUploadMin).
 #ifndef PALABOS_AMD_HOSTIO_H
 #define PALABOS_AMD_HOSTIO_H
+
+#include <emmintrin.h>
 
 #include <atomic>
 #include <condition_variable>
@@ -64,11 +66,43 @@ private:
 // Null when the pinned memory cannot be had.
 std::shared_ptr<HostSlots> hostSlots(Lattice& L);
 
+// Uploads between these sizes go in one pageable copy per array to device memory, and
+// smaller ones in chunks on the calling thread: helper threads take the arrays' lines
+// into other cores' caches, and a program that writes them anew pays for it (density and
+// velocity rewritten, then uploaded, us: 8.4 MB copied 390, by eight threads 520-870; 16.8 MB
+// 690, 1490-1670; 67 MB 4190, 4530-5300; from new arrays each time 2.1 MB 315, 530-800, 16.8
+// MB 2000, 4930). Above, the threads win (populations of 80 / 319 / 638 MB left as they are
+// 3280 -> 1590, 11.3 -> 5.8 ms, 22.0 -> 11.5; rewritten in place 5300 -> 4800-6250, 19.8 -> 17-19
+// ms, 39 -> 33).
+constexpr uint64_t kCopiedUploadMin = 3u << 20, kCopiedUploadMax = 72u << 20;
+
 // One host array over a box, `perCell` bytes a cell in C order (host null: none).
 struct HostPart {
     char* host;
     size_t perCell;
 };
+
+// A copy from another thread's array to a slot that the device reads, leaving neither
+// in the caches of the core that makes it. (With memcpy the owner of the array, writing
+// it anew, fetched its lines back from there: populations of 80 MB rewritten and uploaded
+// 8.1-8.9 ms instead of 4.8-6.3.)
+inline void copyPast(void* to, const void* from, size_t n) {
+    char* d = static_cast<char*>(to);
+    const char* s = static_cast<const char*>(from);
+    for (; n >= 64; n -= 64, d += 64, s += 64) {
+        _mm_prefetch(s + 1024, _MM_HINT_NTA);
+        const __m128i a = _mm_loadu_si128((const __m128i*)s), b = _mm_loadu_si128((const __m128i*)(s + 16)),
+                      c = _mm_loadu_si128((const __m128i*)(s + 32)), e = _mm_loadu_si128((const __m128i*)(s + 48));
+        _mm_stream_si128((__m128i*)d, a);
+        _mm_stream_si128((__m128i*)(d + 16), b);
+        _mm_stream_si128((__m128i*)(d + 32), c);
+        _mm_stream_si128((__m128i*)(d + 48), e);
+    }
+    _mm_sfence();
+    std::memcpy(d, s, n);
+}
+
+inline void copyPlain(void* to, const void* from, size_t n) { std::memcpy(to, from, n); }
 
 // Moves `parts` over box b: launch(chunk, staged, stream) queues the kernels that
 // read (up) or write (down) the chunk's values at staged[part], C order over the
@@ -81,9 +115,32 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     // one plane, else cells of one row
     const uint64_t ly = b.y1 - b.y0 + 1, lz = b.z1 - b.z0 + 1;
     const uint64_t lx = b.x1 - b.x0 + 1;
-    // chunks of an eighth of the whole, between 256 KB (a launch and its wait cost
-    // about 10 us) and a slot
-    const size_t chunkBytes = std::min<uint64_t>(HostSlots::kBytes, std::max<uint64_t>(256u << 10, boxCells(b) * perCell / HostSlots::kSlots + 4096));
+    const uint64_t total = boxCells(b) * perCell;
+    if (up && total > kCopiedUploadMin && total < kCopiedUploadMax) {
+        DeviceBuffers buf;
+        void* dev[4] = {};
+        if (char* at = static_cast<char*>(buf.get(total + 256 * nParts))) {   // one allocation: each costs 30 us and more
+            for (int p = 0; p < nParts; ++p) {
+                if (!parts[p].host) continue;
+                dev[p] = at;
+                at += (boxCells(b) * parts[p].perCell + 255) / 256 * 256;
+            }
+            hipError_t err = hipSuccess;
+            for (int p = 0; p < nParts && err == hipSuccess; ++p)
+                if (parts[p].host)
+                    err = hipMemcpyAsync(dev[p], parts[p].host, boxCells(b) * parts[p].perCell, hipMemcpyHostToDevice, L.stream);
+            if (err == hipSuccess) err = launch(b, dev, L.stream);
+            const hipError_t end = hipStreamSynchronize(L.stream);   // before the buffers go, on every path
+            if (err == hipSuccess) err = end;
+            if (err != hipSuccess) return fail(PLBAMD_EHIP, std::string("transfer: ") + hipGetErrorString(err));
+            ++L.pageableTransfers;
+            return PLBAMD_OK;
+        }
+    }
+    // chunks of an eighth of the whole, between 1 MB (a launch and its wait cost about
+    // 10 us, a thread 20: 623 KB of populations up 79 us in chunks of 256 KB, 46 in one)
+    // and a slot
+    const size_t chunkBytes = std::min<uint64_t>(HostSlots::kBytes, std::max<uint64_t>(1u << 20, total / HostSlots::kSlots + 4096));
     const uint64_t fit = chunkBytes / perCell - 8;    // 8: the parts' alignment
     const uint64_t sx = std::min(lx, std::max<uint64_t>(1, fit / (ly * lz)));
     const uint64_t sy = ly * lz <= fit ? ly : std::min(ly, std::max<uint64_t>(1, fit / lz));
@@ -103,6 +160,7 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
         onDevice = static_cast<char*>(buf.get(chunkBytes));
         if (!onDevice) return fail(PLBAMD_ENOMEM, "transfer: cannot allocate a staging buffer");
     }
+    const int want = !slots || (up && total <= kCopiedUploadMin) ? 1 : (int)std::min<uint64_t>(HostSlots::kSlots, chunks);
     std::atomic<uint64_t> next{0};
     std::atomic<int> error{(int)hipSuccess};
     auto work = [&]() {
@@ -124,7 +182,7 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
                 if (!parts[p].host) continue;
                 staged[p] = slot + at;
                 at = (at + cells * parts[p].perCell + 15) / 16 * 16;
-                if (up) std::memcpy(staged[p], parts[p].host + first * parts[p].perCell, cells * parts[p].perCell);
+                if (up) (want > 1 ? copyPast : copyPlain)(staged[p], parts[p].host + first * parts[p].perCell, cells * parts[p].perCell);
             }
             void* dev[4] = {};
             hipError_t err = hipSuccess;
@@ -141,7 +199,6 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
         }
     };
     std::vector<std::thread> helpers;
-    const int want = slots ? (int)std::min<uint64_t>(HostSlots::kSlots, chunks) : 1;
     for (int k = 1; k < want; ++k) {
         try {
             helpers.emplace_back([&] {

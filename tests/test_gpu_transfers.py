@@ -80,3 +80,25 @@ def test_transfers_of_many_threads(gpu):
     finally:
         for lat in lats:
             lat.close()
+
+
+@pytest.mark.parametrize("shape", [(6, 70, 75), (100, 80, 66), (2, 801, 327), (1, 9, 63000)])
+def test_uploads_by_size(gpu, shape):
+    """Populations of 4.8 MB (one copy to the device) and of 80 to 86 MB, whose chunks in pinned memory are whole
+    x planes, rows of one plane and parts of one row: every value arrives, in a box that starts off the edges too."""
+    with lattice(shape) as lat:
+        f = 0.02 * uniform(shape + (19,), 3)
+        lat.setPopulations(f)
+        pinned = f.nbytes >= 72 * 2 ** 20
+        assert lat.runInfo()["pinned_transfers"] == int(pinned)
+        assert lat.runInfo()["pageable_transfers"] == int(not pinned)
+        assert np.array_equal(lat.getPopulations(), f)
+        x0, y0, z0 = (n // 3 for n in shape)
+        part = 0.02 * uniform(f[x0:, y0:, z0:].shape, 4)
+        f[x0:, y0:, z0:] = part
+        lat.setPopulations(part, (x0, shape[0] - 1, y0, shape[1] - 1, z0, shape[2] - 1))
+        assert np.array_equal(lat.getPopulations(), f)
+        lat.initializeAtEquilibrium(1.0 + 0.01 * uniform(shape, 5), 0.02 * uniform(shape + (3,), 6))
+        rho, u = lat.macroscopic()
+        np.testing.assert_allclose(rho, 1.0 + 0.01 * uniform(shape, 5), rtol=1e-13)
+        np.testing.assert_allclose(u, 0.02 * uniform(shape + (3,), 6), rtol=1e-9, atol=1e-14)
