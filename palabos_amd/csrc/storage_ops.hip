@@ -140,7 +140,11 @@ int checkpointTyped(Lattice& L, const char* path, int elem, bool force, bool enf
     }
     // the reference reads with operator>>, which skips white space (every
     // white-space character is at most ' '; every base64 character above it)
-    if (std::any_of(file.begin(), file.end(), [](char c) { return (unsigned char)c <= ' '; }))
+    // (the least character, 16 at a time: a search that stops at the first one ran at a
+    // byte a cycle or less, whichever way its loop was aligned)
+    unsigned char least = 255;
+    for (size_t k = 0; k < file.size(); ++k) least = std::min(least, (unsigned char)file[k]);
+    if (least <= ' ')
         file.erase(std::remove_if(file.begin(), file.end(), [](char c) { return std::isspace((unsigned char)c) != 0; }),
                    file.end());
     const size_t headChars = enforceUint ? 8 : 12;
