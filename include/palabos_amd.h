@@ -357,12 +357,28 @@ int plbamd_adjoint_gradient(int handle, int nsteps, int checkpoint_every, const 
  * kernels on the same states, so the same records and the same gradient).
  * bytes >= 0: at most that many; -1 (the default): the free device memory at
  * the call beyond a reserve of max(4 GiB, 1/32 of the device); 0: every
- * segment is recomputed. No Palabos counterpart. */
+ * segment is recomputed. The call's buffer is kept for the next one when it is at
+ * most 1/16 of the device and, where a budget was set, at most that
+ * (plbamd_set_kept_bytes bounds it too and gives it back). No Palabos counterpart. */
 int plbamd_set_adjoint_record_bytes(int handle, int64_t bytes);
 
 /* Segments the last plbamd_adjoint_gradient call recorded in its forward
  * sweep, and the device bytes of those records. No Palabos counterpart. */
 int plbamd_get_adjoint_record_info(int handle, int* kept_segments, int64_t* bytes);
+
+/* Device memory the lattice may hold between calls, beyond what it needs, to make
+ * the next calls faster: a second population array with its tables (two steps per
+ * launch; as large as the populations, 4 or 8 bytes a cell more with edges or tags),
+ * and the adjoint's buffer. -1 (the default): a second array of at most an eighth of
+ * the memory that is free when it is first used, and an adjoint buffer as
+ * plbamd_set_adjoint_record_bytes says. bytes >= 0: at most that many; what is held
+ * beyond is given back at once, and steps that had needed it run one at a time, with
+ * the same results. 0 therefore frees all of it (and -1 afterwards lets it come
+ * back). Allocations of this library that run short take the memory of every
+ * lattice back by themselves; those of others (torch, another library in the
+ * process) cannot, so a program that shares the device sets a bound here.
+ * plbamd_get_run_info tells what is held. No Palabos counterpart. */
+int plbamd_set_kept_bytes(int handle, int64_t bytes);
 
 /* How the lattice runs: counts since it was created and what it holds, for
  * tests and benchmarks that say which way a call took (the results do not depend

@@ -90,7 +90,7 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     const uint64_t nAcc = (uint64_t)adjWGs + planeWGs;   // J accumulators: bulk workgroups, then plane ones
     const uint64_t nScale = std::max<uint32_t>(1, L.nSpecial);
     // One buffer holds everything; the lattice keeps it for the next call when it is
-    // at most a sixteenth of the card's memory (thirteen allocations a call came to
+    // at most a sixteenth of the card's memory and the caller's budgets (thirteen allocations a call came to
     // cost 113 ms a call once some fifty calls had been made).
     //   fixed:      working state, adjoint states, gradients, accumulators
     //   recompute:  checkpoints and one segment's records (not when every segment is kept)
@@ -120,12 +120,15 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
             bytes = n;
             return true;
         }
-        // given back to the lattice, or freed
+        // given back to the lattice, or freed: a caller who set a budget for the records
+        // shares the device, so no more than that is kept; nor more than the lattice
+        // may keep at all
         ~Buffer() {
             size_t freeB = 0, totalB = 0;
-            if (p && hipMemGetInfo(&freeB, &totalB) == hipSuccess && bytes <= totalB / 16) {
+            const bool records = L.adjointRecordBytes < 0 || bytes <= (uint64_t)L.adjointRecordBytes;
+            if (p && records && hipMemGetInfo(&freeB, &totalB) == hipSuccess && bytes <= totalB / 16) {
                 std::lock_guard<std::mutex> use(L.spareMutex);
-                if (!L.adjointBuf) {
+                if (!L.adjointBuf && (L.keptBudget < 0 || L.keptBytes() + bytes <= (uint64_t)L.keptBudget)) {
                     L.adjointBuf = p;
                     L.adjointBufBytes = bytes;
                     return;

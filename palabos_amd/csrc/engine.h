@@ -165,22 +165,31 @@ struct Lattice {
     // the adjoint's buffer between its calls (under spareMutex; adjoint.hip)
     char* adjointBuf = nullptr;
     uint64_t adjointBufBytes = 0;
+    int64_t keptBudget = -1;       // plbamd_set_kept_bytes
     bool anySolid = false;         // link-wall solids
     // what ran, for plbamd_get_run_info
     int64_t twoStepLaunches = 0, pinnedTransfers = 0, pageableTransfers = 0;
     bool nodeBesideWall = false;   // and nodes or boundary objects: single steps
 
     // device bytes held by all of these (under spareMutex)
-    uint64_t keptBytes() const {
+    uint64_t twoStepBytes() const {
         return (spare ? 19 * geom[0].slot * elemSize : 0) + (dInfo ? 4 * cells : 0) + (dIndex ? 4 * cells : 0) +
-               (dPre ? 19 * (uint64_t)nSpecial * elemSize : 0) + adjointBufBytes;
+               (dPre ? 19 * (uint64_t)nSpecial * elemSize : 0);
     }
-    void releaseSpare() {
-        hipFree(spare); hipFree(dInfo); hipFree(dIndex); hipFree(dPre); hipFree(adjointBuf);
-        adjointBuf = nullptr;
-        adjointBufBytes = 0;
+    uint64_t keptBytes() const { return twoStepBytes() + adjointBufBytes; }
+    void releaseTwoStep() {
+        hipFree(spare); hipFree(dInfo); hipFree(dIndex); hipFree(dPre);
         spare = dPre = nullptr;
         dInfo = dIndex = nullptr;
+    }
+    void releaseAdjointBuf() {
+        hipFree(adjointBuf);
+        adjointBuf = nullptr;
+        adjointBufBytes = 0;
+    }
+    void releaseSpare() {
+        releaseTwoStep();
+        releaseAdjointBuf();
     }
 
     ~Lattice() {

@@ -922,6 +922,12 @@ static bool fusedReady(Lattice& L) {
     // 32-bit lane offsets: within a plane, or (reflections) over ten slots
     const uint64_t span = (needInfo ? 10 * g.slot : (uint64_t)g.ny * g.nz) * L.elemSize;
     if (!wanted || span > 0xffffffffull) return false;
+    if (L.keptBudget >= 0) {
+        const uint64_t need = bytes + (needInfo ? 4 * L.cells : 0) +
+                              (needInfo && L.nSpecial ? 4 * L.cells + 19 * (uint64_t)L.nSpecial * L.elemSize : 0);
+        if (need > (uint64_t)L.keptBudget) return false;
+        if (need + L.adjointBufBytes > (uint64_t)L.keptBudget) L.releaseAdjointBuf();
+    }
     if (!L.spare) {
         size_t freeB = 0, totalB = 0;
         if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || bytes > freeB / 8 || hipMalloc(&L.spare, bytes) != hipSuccess) {
@@ -939,7 +945,7 @@ static bool fusedReady(Lattice& L) {
         }
         if (!ok) {
             (void)hipGetLastError();
-            L.releaseSpare();
+            L.releaseTwoStep();
             return false;
         }
         L.fused = planFused(g, L.elemSize, needInfo, L.nSpecial != 0);
@@ -1547,6 +1553,18 @@ int plbamd_get_adjoint_record_info(int handle, int* kept_segments, int64_t* byte
     if (!L || !kept_segments || !bytes) return fail(PLBAMD_EINVAL, "get_adjoint_record_info: bad argument");
     *kept_segments = L->adjointKept;
     *bytes = L->adjointKeptBytes;
+    return PLBAMD_OK;
+}
+
+int plbamd_set_kept_bytes(int handle, int64_t bytes) {
+    Lattice* L = find(handle);
+    if (!L || bytes < -1) return fail(PLBAMD_EINVAL, "set_kept_bytes: bad argument");
+    std::lock_guard<std::mutex> use(L->spareMutex);
+    L->keptBudget = bytes;
+    if (bytes < 0 || L->keptBytes() <= (uint64_t)bytes) return PLBAMD_OK;
+    PLBAMD_HIP(hipStreamSynchronize(L->stream));
+    L->releaseAdjointBuf();
+    if (L->keptBytes() > (uint64_t)bytes) L->releaseTwoStep();
     return PLBAMD_OK;
 }
 

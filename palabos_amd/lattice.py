@@ -416,6 +416,14 @@ class Block3D:
         check(lib().plbamd_get_adjoint_record_info(self.handle, ctypes.byref(n), ctypes.byref(b)))
         return n.value, b.value
 
+    def setKeptBytes(self, nbytes):
+        """Device memory the lattice may hold between calls to make the next ones faster
+        (a second population array, adjointGradient's buffer): -1 (default) as much
+        as an eighth of the free memory and a sixteenth of the device, otherwise at
+        most nbytes; what is held beyond is given back at once. Results do not
+        depend on it. For programs that share the device, with torch for example."""
+        check(lib().plbamd_set_kept_bytes(self.handle, int(nbytes)))
+
     def runInfo(self):
         """Which way the lattice's calls took (the results do not depend on it): a dict
         of two_step_launches, kept_bytes (device memory held between calls),

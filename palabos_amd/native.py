@@ -39,7 +39,7 @@ EXPORTS = (
     "plbamd_adjoint_gradient", "plbamd_set_adjoint_record_bytes", "plbamd_get_adjoint_record_info", "plbamd_get_time", "plbamd_save_binary_block", "plbamd_load_binary_block",
     "plbamd_compute_fields", "plbamd_set_solid_density", "plbamd_reduce_moments_noalloc",
     "plbamd_add_velocity_edge", "plbamd_add_velocity_corner", "plbamd_set_boundary_type",
-    "plbamd_execute_processors", "plbamd_get_run_info", "plbamd_bandwidth_probe", "plbamd_multiblock_create_ex",
+    "plbamd_execute_processors", "plbamd_get_run_info", "plbamd_set_kept_bytes", "plbamd_bandwidth_probe", "plbamd_multiblock_create_ex",
     "plbamd_get_block_count", "plbamd_compute_rhobar_j", "plbamd_get_rhobar_j", "plbamd_set_rhobar_j",
     "plbamd_external_collide_and_stream",
 )
@@ -132,6 +132,7 @@ def lib():
         "plbamd_compute_fields": [i32, pbox, vp],
         "plbamd_set_solid_density": [i32, i32, ctypes.c_double],
         "plbamd_get_run_info": [i32, vp],
+        "plbamd_set_kept_bytes": [i32, ctypes.c_int64],
         "plbamd_get_time": [i32, ctypes.POINTER(ctypes.c_int64)],
         "plbamd_adjoint_gradient": [i32, i32, i32, ctypes.POINTER(Objective), vp, vp, vp, vp],
         "plbamd_set_adjoint_record_bytes": [i32, ctypes.c_int64],
