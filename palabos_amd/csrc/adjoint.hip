@@ -146,16 +146,16 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     // (len per segment, one more for f^T) fit the budget: what the caller allows, or
     // the free memory beyond a reserve. Record r of kept segment c is
     // keep[keepFirst * K + r].
-    uint64_t available = 0;
-    if (L.adjointRecordBytes < 0) {
+    auto freeMemory = [&]() -> uint64_t {
         size_t freeB = 0, totalB = 0;
-        if (hipMemGetInfo(&freeB, &totalB) == hipSuccess) {
-            const uint64_t taken = std::max<uint64_t>(4ull << 30, totalB / 32) + fixedBytes;
-            available = freeB + buffer.bytes > taken ? freeB + buffer.bytes - taken : 0;
-        } else {
+        if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) {
             (void)hipGetLastError();
+            return 0;
         }
-    }
+        const uint64_t taken = std::max<uint64_t>(4ull << 30, totalB / 32) + fixedBytes;
+        return freeB + buffer.bytes > taken ? freeB + buffer.bytes - taken : 0;
+    };
+    uint64_t available = L.adjointRecordBytes < 0 ? freeMemory() : 0;
     int nKeep = 0;
     uint64_t keepRecs = 1;
     auto fit = [&](uint64_t budget) {
@@ -174,6 +174,12 @@ int adjointGradient(Lattice& L, int T, int K, const plbamd_objective& obj, doubl
     };
     auto total = [&]() { return fixedBytes + (nKeep == nCk ? 0 : againBytes) + keepBytes(); };
     fit(L.adjointRecordBytes >= 0 ? (uint64_t)L.adjointRecordBytes : available);
+    if (nKeep < nCk && L.adjointRecordBytes < 0) {
+        // records before what lattices hold for later calls
+        releaseSpares();
+        available = freeMemory();
+        fit(available);
+    }
     if (nKeep < nCk && L.adjointRecordBytes < 0) fit(available > againBytes ? available - againBytes : 0);
     bool have = buffer.ensure(total());
     if (!have && nKeep > 0) {

@@ -63,8 +63,8 @@ extern "C" int plbamd_bandwidth_probe(int pattern, uint64_t bytes, int repeats, 
     void* b = nullptr;
     hipStream_t s = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    hipError_t err = hipMalloc(&a, alloc);
-    if (err == hipSuccess && pattern == PLBAMD_PROBE_COPY) err = hipMalloc(&b, alloc);
+    hipError_t err = deviceAlloc(&a, alloc);
+    if (err == hipSuccess && pattern == PLBAMD_PROBE_COPY) err = deviceAlloc(&b, alloc);
     if (err == hipSuccess) err = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
     if (err == hipSuccess) err = hipEventCreate(&e0);
     if (err == hipSuccess) err = hipEventCreate(&e1);

@@ -213,7 +213,8 @@ struct Recording {
 };
 
 // hipMalloc that, short of memory, takes back the second arrays and adjoint buffers
-// of the lattices that no call is using and tries again.
+// of all lattices (once the calls that step with them have queued their steps) and
+// tries again. Not to be called with a lattice's spareMutex held.
 hipError_t deviceAlloc(void** p, size_t bytes);
 void releaseSpares();
 

@@ -82,8 +82,10 @@ void releaseSpares() {
     std::lock_guard<std::mutex> lock(g_mutex);
     for (auto& e : g_lattices) {
         Lattice& L = *e.second;
-        std::unique_lock<std::mutex> use(L.spareMutex, std::try_to_lock);
-        if (!use.owns_lock() || !(L.spare || L.adjointBuf)) continue;
+        // after the call that uses them: no call allocates under its spareMutex, or waits
+        // for g_mutex under it, so this ends
+        std::lock_guard<std::mutex> use(L.spareMutex);
+        if (!(L.spare || L.adjointBuf)) continue;
         (void)hipStreamSynchronize(L.stream);
         L.releaseSpare();
     }
@@ -418,7 +420,7 @@ int setup(Lattice& L) {
     auto uploadSegments = [&](const std::vector<CopySegment>& segs, CopySegment** dSegs, CopyTask** dTasks,
                               uint32_t* nTasks) -> int {
         if (segs.empty()) return PLBAMD_OK;
-        PLBAMD_HIP(hipMalloc(dSegs, segs.size() * sizeof(CopySegment)));
+        PLBAMD_HIP(deviceAlloc((void**)dSegs, segs.size() * sizeof(CopySegment)));
         PLBAMD_HIP(hipMemcpy(*dSegs, segs.data(), segs.size() * sizeof(CopySegment), hipMemcpyHostToDevice));
         std::vector<CopyTask> tasks;
         for (size_t k = 0; k < segs.size(); ++k) {
@@ -426,7 +428,7 @@ int setup(Lattice& L) {
             for (uint64_t f = 0; f < cnt; f += 256) tasks.push_back(CopyTask{(uint32_t)k, (uint32_t)f});
         }
         *nTasks = (uint32_t)tasks.size();
-        PLBAMD_HIP(hipMalloc(dTasks, tasks.size() * sizeof(CopyTask)));
+        PLBAMD_HIP(deviceAlloc((void**)dTasks, tasks.size() * sizeof(CopyTask)));
         PLBAMD_HIP(hipMemcpy(*dTasks, tasks.data(), tasks.size() * sizeof(CopyTask), hipMemcpyHostToDevice));
         return PLBAMD_OK;
     };

@@ -1,7 +1,10 @@
 """Device memory that a lattice holds between calls (plbamd_set_kept_bytes): bounded,
 given back when asked and when an allocation of the library runs short, and
 without an effect on the results."""
+import contextlib
 import ctypes
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -89,3 +92,55 @@ def test_adjoint_buffer_keeps_to_the_budgets(gpu):
         assert lat.runInfo()["kept_bytes"] == held
     with pytest.raises(plb.native.PlbError):
         lattice(8).setKeptBytes(-2)
+
+
+@contextlib.contextmanager
+def filled(leave):
+    """The device's memory taken but for about `leave` bytes: all that is reported free but 2 GB, then pieces of
+    64 MB until there is none (the device has more than it reports), of which `leave` are given back."""
+    rt, taken = hip(), []
+
+    def take(n):
+        p = ctypes.c_void_p()
+        if rt.hipMalloc(ctypes.byref(p), ctypes.c_size_t(n)) != 0:
+            return False
+        taken.append(p)
+        return True
+    try:
+        assert take(free_bytes() - (2 << 30))
+        while take(64 << 20):
+            assert len(taken) < 200
+        for _ in range(leave // (64 << 20)):
+            assert rt.hipFree(taken.pop()) == 0
+        yield
+    finally:
+        rt.hipGetLastError()
+        for p in taken:
+            assert rt.hipFree(p) == 0
+
+
+def test_every_allocation_takes_kept_memory_back(gpu, monkeypatch):
+    """160^3 FP64: 623 MB of populations and as much kept. With 400 MB left, a probe of 700 MB needs it."""
+    monkeypatch.delenv("PLBAMD_FUSED", raising=False)
+    with lattice(160) as lat:
+        lat.collideAndStream(5)
+        assert lat.runInfo()["kept_bytes"] > 590 << 20
+        with filled(400 << 20):
+            ms, moved, gbs = plb.native.bandwidth_probe("slots", 1400 << 20, repeats=1)
+        assert lat.runInfo()["kept_bytes"] == 0
+
+
+def test_an_allocation_waits_for_the_call_that_uses_kept_memory(gpu, monkeypatch):
+    """The same while another thread is in a call of many steps with it: the allocation waits for that call's
+    launches instead of failing."""
+    monkeypatch.delenv("PLBAMD_FUSED", raising=False)
+    with lattice(160) as lat:
+        lat.collideAndStream(5)
+        with filled(400 << 20):
+            t = threading.Thread(target=lat.collideAndStream, args=(12000,))
+            t.start()
+            time.sleep(0.003)
+            with lattice(150) as other:      # 513 MB
+                other.collideAndStream(2)
+            t.join()
+        assert lat.time == 12005
