@@ -975,18 +975,22 @@ int launchStep(Lattice& L, bool odd, bool stats) {
                                          : launchStepTyped<S, 1>(L, odd, stats);
 }
 
-int step(Lattice& L, int nsteps) {
+// Set-up before nsteps steps: tags, and whether steps are taken two at a time (those
+// that need not report statistics, from an odd time on), with what that takes. Then
+// `use` holds spareMutex until the steps are queued.
+static int prepareSteps(Lattice& L, int nsteps, bool& fused, std::unique_lock<std::mutex>& use) {
     PLBAMD_TRY(rebuild(L));
-    // steps that need not report statistics, from an odd time on, two at a time
-    std::unique_lock<std::mutex> use(L.spareMutex, std::defer_lock);
-    bool fused = false;
-    if (nsteps - (L.statsOn ? 1 : 0) - (L.time & 1 ? 0 : 1) >= 2) {
-        use.lock();
-        const bool had = L.spare && (L.dInfo || !(L.dTags || !(L.geom[0].px && L.geom[0].py && L.geom[0].pz)));
-        fused = fusedReady(L);
-        if (fused && !had) PLBAMD_TRY(fusedDispatch(L, FUSED_PREPARE));
-        if (fused) PLBAMD_TRY(fusedDispatch(L, FUSED_BEGIN));
-    }
+    fused = false;
+    if (nsteps - (L.statsOn ? 1 : 0) - (L.time & 1 ? 0 : 1) < 2) return PLBAMD_OK;
+    use = std::unique_lock<std::mutex>(L.spareMutex);
+    const bool had = L.spare && (L.dInfo || !(L.dTags || !(L.geom[0].px && L.geom[0].py && L.geom[0].pz)));
+    fused = fusedReady(L);
+    if (fused && !had) PLBAMD_TRY(fusedDispatch(L, FUSED_PREPARE));
+    return PLBAMD_OK;
+}
+
+static int queueSteps(Lattice& L, int nsteps, bool fused) {
+    if (fused) PLBAMD_TRY(fusedDispatch(L, FUSED_BEGIN));
     for (int s = 0; s < nsteps; ++s) {
         const bool odd = (L.time & 1) != 0;
         if (fused && odd && nsteps - s - (L.statsOn ? 1 : 0) >= 2) {
@@ -1009,6 +1013,13 @@ int step(Lattice& L, int nsteps) {
         if (stats) L.statsValid = true;
     }
     return PLBAMD_OK;
+}
+
+int step(Lattice& L, int nsteps) {
+    std::unique_lock<std::mutex> use;
+    bool fused;
+    PLBAMD_TRY(prepareSteps(L, nsteps, fused, use));
+    return queueSteps(L, nsteps, fused);
 }
 
 // Transfer arguments for block bi and the part of the global box `g` it owns.
@@ -1459,10 +1470,16 @@ int plbamd_collide_and_stream_timed(int handle, int nsteps, double* ms) {
     Lattice* L = find(handle);
     if (!L) return fail(PLBAMD_EINVAL, "collide_and_stream_timed: unknown handle");
     if (nsteps < 0 || !ms) return fail(PLBAMD_EINVAL, "collide_and_stream_timed: bad argument");
-    PLBAMD_TRY(rebuild(*L));
-    PLBAMD_HIP(hipEventRecord(L->ev0, L->stream));
-    PLBAMD_TRY(step(*L, nsteps));
-    PLBAMD_HIP(hipEventRecord(L->ev1, L->stream));
+    {
+        // the set-up before the first event: it is not step time
+        std::unique_lock<std::mutex> use;
+        bool fused;
+        PLBAMD_TRY(prepareSteps(*L, nsteps, fused, use));
+        PLBAMD_HIP(hipStreamSynchronize(L->stream));
+        PLBAMD_HIP(hipEventRecord(L->ev0, L->stream));
+        PLBAMD_TRY(queueSteps(*L, nsteps, fused));
+        PLBAMD_HIP(hipEventRecord(L->ev1, L->stream));
+    }
     PLBAMD_HIP(hipEventSynchronize(L->ev1));
     float elapsed = 0.f;
     PLBAMD_HIP(hipEventElapsedTime(&elapsed, L->ev0, L->ev1));

@@ -28,3 +28,21 @@ def test_tagged_odd_steps_keep_their_loads_together(gpu, monkeypatch):
             us.append(step_us(lat, 50))
     print(f"[step time] plain {us[0]:.1f} us, tagged {us[1]:.1f} us", flush=True)
     assert us[1] < 1.17 * us[0]
+
+
+def test_timed_steps_do_not_include_their_set_up(gpu, monkeypatch):
+    """The first timed call of a lattice allocates the second array and its tables (a millisecond and more) before the
+    clock starts, as any later one finds them."""
+    monkeypatch.delenv("PLBAMD_FUSED", raising=False)
+
+    def first_and_next():
+        with plb.Block3D(128, 128, 128, plb.D3Q19, plb.BGK(1.8), storage="f64") as lat:
+            lat.toggleInternalStatistics(False)
+            lat.collideAndStream(1)
+            first = lat.collideAndStreamTimed(4)
+            assert lat.runInfo()["two_step_launches"] == 2
+            return first, min(lat.collideAndStreamTimed(4) for _ in range(5))
+    first_and_next()     # the kernels' code comes with the first use in a process
+    first, later = first_and_next()
+    print(f"[step time] first call {first * 1e3:.0f} us, later ones {later * 1e3:.0f} us", flush=True)
+    assert first < 1.5 * later
