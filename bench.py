@@ -15,13 +15,15 @@ recomputed.
 value        MLUPS = cells * steps / wall seconds / 1e6 over the timed steps,
              populations resident in HBM before the timed region starts.
 roofline     the collide-and-stream launches: the bytes they have to move / their
-             time, measured with HIP events on the stream the kernels run on. At
-             this size FP64 and FP32 take two steps per launch and so read and
-             write the 19 populations of a cell once per two steps; 16-bit storage
-             takes one step per launch (even and odd steps alternate two kernels).
+             time, measured with HIP events on the stream the kernels run on. How
+             many launches took two steps, reading and writing the 19 populations of
+             a cell once for both, is what the engine counted over the timed steps
+             (at this size FP64 and FP32 do; 16-bit storage takes one step per
+             launch, even and odd steps alternating two kernels).
              "algorithmic_bytes_per_cell" is per step; "traffic" is the HBM bytes
              per launch from rocprofv3 counters
-             (profiles/bulk_step_tg512_counters.txt).
+             (profiles/bulk_step_tg512_counters.txt), null for launches of another
+             kind than those.
 cpu_baseline the compiled Palabos reference (oracle/_ref/ref_driver, serial) on a
              bounded sample (periodic BGK FP64 128^3): "value" is the aggregate
              of one independent serial process per host core of this job's
@@ -47,16 +49,26 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# Bytes a step has to move per cell: 19 populations read and written once per step,
-# or once per two steps where one launch takes both.
-BYTES_PER_CELL = {"f64": 19 * 8, "f32": 19 * 4, "f16": 19 * 2 * 2, "bf16": 19 * 2 * 2}
-# The launches at this workload (the first and the last step of a call with an even
-# number of steps are single ones).
-KERNELS = {"f64": "plbamd::fused_two_steps (two steps)",
-           "f32": "plbamd::fused_two_steps (two steps)",
-           "f16": "plbamd::bulk_even_linear (even) / plbamd::bulk_pairs (odd)",
-           "bf16": "plbamd::bulk_even_linear (even) / plbamd::bulk_pairs (odd)"}
-STEPS_PER_LAUNCH = {"f64": 2, "f32": 2, "f16": 1, "bf16": 1}
+STORAGE_BYTES = {"f64": 8, "f32": 4, "f16": 2, "bf16": 2}
+# Steps per launch in the committed counter profile, which "traffic" is read from.
+PROFILED_STEPS_PER_LAUNCH = {"f64": 2, "f32": 2, "f16": 1}
+
+
+def launches(precision, n, steps, two_step_launches):
+    """What `steps` steps of an n^3 lattice were launched as, of which two_step_launches
+    took two: kernel, steps per launch (of most), launches, and the bytes a step has to
+    move per cell (19 populations read and written once per launch)."""
+    count = steps - two_step_launches
+    if two_step_launches > 0:
+        kernel = "plbamd::fused_two_steps (two steps)"
+    elif STORAGE_BYTES[precision] > 2:
+        kernel = "plbamd::bulk_step (even) / plbamd::bulk_odd_staged (odd)"
+    elif n % 2 == 0:
+        kernel = "plbamd::bulk_even_linear (even) / plbamd::bulk_pairs (odd)"
+    else:
+        kernel = "plbamd::bulk_step"
+    return {"kernel": kernel, "steps_per_launch": 2 if two_step_launches > 0 else 1, "launches": count,
+            "bytes_per_cell": 2 * 19 * STORAGE_BYTES[precision] * count / steps}
 
 
 def taylor_green_init(lat, n, u0):
@@ -84,12 +96,14 @@ def run_precision(precision, n, steps, warmup, omega=1.8, u0=0.04):
         lat.toggleInternalStatistics(False)
         if warmup:
             lat.collideAndStream(warmup)
+        pairs = lat.runInfo()["two_step_launches"]
         t0 = time.perf_counter()
         ms_events = lat.collideAndStreamTimed(steps)  # blocks until the last step has finished
         wall = time.perf_counter() - t0
+        how = launches(precision, n, steps, lat.runInfo()["two_step_launches"] - pairs)
         cells = n ** 3
         kernel_ms = ms_events / steps
-        achieved = BYTES_PER_CELL[precision] * cells / (kernel_ms * 1e-3) / 1e9
+        achieved = how["bytes_per_cell"] * cells / (kernel_ms * 1e-3) / 1e9
         return {
             "dtype": precision,
             "value": cells * steps / wall / 1e6,
@@ -97,6 +111,11 @@ def run_precision(precision, n, steps, warmup, omega=1.8, u0=0.04):
             "event_ms_per_step": kernel_ms,
             "achieved_gbs": achieved,
             "frac": achieved / HBM_PEAK_GBS,
+            "kernel": how["kernel"],
+            "algorithmic_bytes_per_cell": how["bytes_per_cell"],
+            "steps_per_launch": how["steps_per_launch"],
+            "event_ms_per_launch": ms_events / how["launches"],
+            "traffic": traffic_from_profile(precision, n, how["steps_per_launch"]),
         }
     finally:
         lat.close()
@@ -198,9 +217,11 @@ def cpu_baseline():
             "sample": f"oracle restatement, periodic BGK FP64 {n}^3, {steps} steps, {sec:.1f} s", "host": host}
 
 
-def traffic_from_profile(precision, n):
+def traffic_from_profile(precision, n, steps_per_launch):
     """HBM bytes per launch of the bulk kernel from the committed rocprofv3 counter
     summary (profiles/bulk_step_tg512_counters.txt), or None."""
+    if PROFILED_STEPS_PER_LAUNCH.get(precision) != steps_per_launch:
+        return None
     path = os.path.join(ROOT, "profiles", "bulk_step_tg512_counters.txt")
     if not os.path.exists(path):
         return None
@@ -280,10 +301,6 @@ def main():
         for p in ("f64", "f32", "f16"):
             if p != args.precision:
                 variants.append(run_precision(p, args.n, args.steps, args.warmup))
-    for v in variants:
-        v["kernel"] = KERNELS[v["dtype"]]
-        v["traffic"] = traffic_from_profile(v["dtype"], args.n)
-    traffic = traffic_from_profile(args.precision, args.n)
     line = {
         "metric": "D3Q19 MLUPS (FP64/FP32/FP16-store) & % HBM peak; adjoint/forward ratio",
         "value": main_run["value"],
@@ -300,10 +317,9 @@ def main():
         "config": {"workload": f"taylor_green_{args.n}^3_periodic_bgk", "lattice": [args.n] * 3,
                    "omega": 1.8, "u0": 0.04, "precision": args.precision, "statistics": False},
         "roofline": {"bound": "hbm", "achieved": main_run["achieved_gbs"], "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": main_run["frac"], "traffic": traffic,
-                     "kernel": KERNELS[args.precision], "algorithmic_bytes_per_cell": BYTES_PER_CELL[args.precision],
-                     "steps_per_launch": STEPS_PER_LAUNCH[args.precision],
-                     "event_ms_per_launch": main_run["event_ms_per_step"] * STEPS_PER_LAUNCH[args.precision]},
+                     "unit": "GB/s", "frac": main_run["frac"],
+                     **{k: main_run[k] for k in ("traffic", "kernel", "algorithmic_bytes_per_cell", "steps_per_launch",
+                                                 "event_ms_per_launch")}},
         "variants": variants,
     }
     if not args.no_adjoint:
