@@ -821,18 +821,23 @@ int rebuild(Lattice& L) {
 }
 
 // Tile and chunk of the fused steps: the least of
-//   rounds of workgroups * (planes per workgroup + 2.5) * bytes per plane of a tile.
+//   rounds of workgroups * (planes per workgroup + 2.5) * (bytes per plane of a tile + fixed).
 // The 2.5 planes are the two that a chunk's ends repeat and the pipeline's start;
 // the bytes are the lines a row of the tile reads, its rim counted at `rim` (most
 // of it hits in L2), and those it writes; rows that do not start on 64-byte
 // boundaries write lines in parts. Against 900 timed combinations of tile and
 // chunk on eleven lattices (64^3 to 384x256x256, 191x203x197 among them) the
 // choice is 1-5 % from the fastest; the fewest tiles alone chose 18x23 cells at
-// 160^3 (FP64 218 us a step; with 10x40 144 us). With edges or tags, at most 64 cells
-// wide for FP64 (72^3 19.6 -> 16.3 us) and 126 otherwise, as every wavefront of a
-// whole-row tile holds edges (FP32 256x128x128 with edges 105 -> 89, channel 117 -> 110,
-// link walls 256x160x128 154 -> 159); FP64 with special cells, whose tiles take
-// longer, half a round more, which prefers shorter chunks (channel 192x96x96
+// 160^3 (FP64 218 us a step; with 10x40 144 us). `fixed`: with edges or tags, in
+// 32-bit arithmetic, a plane takes its time whatever it moves (a chain of loads, two
+// collisions and two barriers of one workgroup per CU; in the units of the bytes, lines
+// of 128), so that few useful cells in a tile cost more: whole rows of 112-126 FP32 cells leave six of the eight rows
+// of a tile, half rows thirteen of fifteen (256x128x120 with edges 94 -> 85 us, channel
+// 110 -> 105, 160x128x224 106 -> 86). Against 4600 timed combinations with edges, link
+// walls or planes and rows of 80 to 256 cells the choice is 1.3-1.5 % from the fastest in
+// the mean and 10 % at most; without `fixed` 5-7 % and 18-23 %. FP64 with edges or tags: at
+// most 64 cells wide (72^3 19.6 -> 16.3 us); with special cells, whose tiles take longer,
+// half a round more, which prefers shorter chunks (channel 192x96x96
 // 100 -> 90, 256x128x128 194 -> 182, 256x160x160 270 -> 280).
 static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, bool specials) {
     const int threads = fused_threads(std::max<size_t>(4, size));
@@ -841,7 +846,8 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
     Lattice::FusedPlan best;
     double least = 1e300;
     const double waves = specials && size == 8 ? 0.5 : 0.0;
-    for (int width = 8; width <= (info ? (size == 8 ? 64 : 126) : 128); width += 2) {
+    const double fixed = info && size < 8 ? 200.0 : 0.0;
+    for (int width = 8; width <= (info && size == 8 ? 64 : 128); width += 2) {
         const int w = std::min(width, g.nz), tz = (g.nz + w - 1) / w;
         int rows = threads / (w + 2) - 2;
         if (rows < 1) break;
@@ -854,7 +860,7 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
         for (int chunks = 1; chunks <= g.nx; ++chunks) {
             const int len = (g.nx + chunks - 1) / chunks;
             const double wgs = (double)ty * tz * ((g.nx + len - 1) / len);
-            const double cost = (std::ceil(wgs / slots) + waves) * (len + 2.5) * bytes;
+            const double cost = (std::ceil(wgs / slots) + waves) * (len + 2.5) * (bytes + fixed);
             if (cost >= least) continue;
             least = cost;
             best.rows = rows + 2; best.cols = w + 2; best.tilesY = ty; best.tilesZ = tz; best.len = len;
@@ -891,7 +897,7 @@ static Lattice::FusedPlan planFused(const BlockGeom& g, size_t size, bool info, 
 //          cache (6.7 10^6 cells) and 1.0-1.5 beyond (191x203x197 with nodes 218 -> 159)
 //   A force on FP64 with edges or tags (two collisions with it and the cell's word in
 //   178 registers): link walls 80^3 31.3 -> 25.9, 96^3 47.6 -> 47.2, 112^3 69.9 -> 83.7, 128^3 105.9 ->
-//   115.3, 160^3 229 -> 199; 97^3 55.1 -> 56.3, 129^3 159 -> 124
+//   115.3, 362x128x64 153 -> 141, 160^3 229 -> 199, edges 54x137x352 157 -> 132; 97^3 55.1 -> 56.3, 129^3 159 -> 124
 // Planes and momentum-exchange nodes bring two more small launches, which single
 // steps of small lattices do without (bulk_and_special): FP64 channel 128x64x64
 // 31.1 -> 40.2, cavity 96^3 64.4 -> 56.6, channel 192x96x96 107 -> 90; FP32 256x128x128
@@ -908,7 +914,7 @@ static bool fusedReady(Lattice& L) {
     const bool heavy = forced || L.desc.dynamics != PLBAMD_BGK;   // more instructions a cell
     if (L.elemSize == 8) {
         wanted = L.cells >= (L.nSpecial ? 700000u : needInfo ? 370000u : 250000u) &&
-                 !(needInfo && forced && L.cells >= 800000 && (lines ? L.cells < 3000000 : bytes <= kCachedBytes));
+                 !(needInfo && forced && L.cells >= 800000 && (lines ? L.cells < 2300000 : bytes <= kCachedBytes));
     } else if (L.elemSize == 4) {
         wanted = needInfo ? bytes >= 300000000u || (!lines && L.cells >= (heavy ? 900000u : 600000u))
                           : L.cells >= (heavy ? 430000u : lines ? 300000u : 250000u) &&

@@ -109,7 +109,7 @@ def test_cache_policy_of_small_lattices(gpu, storage, n, policy):
     ("f32", (60, 88, 64), "periodic", "bgk", True, False), ("f32", (80, 80, 80), "periodic", "rbgk", False, True),
     ("f32", (97, 99, 101), "box", "rbgk", True, True), ("f32", (83, 85, 87), "box", "rbgk", False, False),
     ("f32", (83, 85, 87), "box", "bgk", False, True),
-    # FP64 with edges or tags: with a force not between 800,000 and 3,000,000 cells (whole lines; the cache otherwise)
+    # FP64 with edges or tags: with a force not between 800,000 and 2,300,000 cells (whole lines; the cache otherwise)
     ("f64", (80, 80, 80), "box", "rbgk", True, True), ("f64", (112, 112, 112), "box", "rbgk", True, False),
     ("f64", (128, 128, 128), "walls", "rbgk", True, False), ("f64", (112, 112, 112), "box", "rbgk", False, True),
     ("f64", (112, 112, 112), "periodic", "rbgk", True, True), ("f64", (97, 99, 101), "box", "rbgk", True, False),

@@ -46,3 +46,15 @@ def test_timed_steps_do_not_include_their_set_up(gpu, monkeypatch):
     first, later = first_and_next()
     print(f"[step time] first call {first * 1e3:.0f} us, later ones {later * 1e3:.0f} us", flush=True)
     assert first < 1.5 * later
+
+
+def test_tiles_of_long_rows_hold_enough_rows(gpu, monkeypatch):
+    """Two-step tiles with edges: a row of 120 or 124 cells taken whole leaves few rows to a tile, and a lattice of such
+    rows took longer than one of 128 (FP32 256x128xnz: 94, 94 and 89 us a step; halved 85, 87 and 89)."""
+    monkeypatch.setenv("PLBAMD_FUSED", "1")
+    us = {}
+    for nz in (120, 124, 128):
+        with plb.Block3D(256, 128, nz, plb.D3Q19, plb.BGK(1.8), storage="f32") as lat:
+            us[nz] = step_us(lat, 40)
+    print(f"[step time] {us}", flush=True)
+    assert max(us[120], us[124]) < 1.03 * us[128]
