@@ -608,10 +608,11 @@ __device__ __forceinline__ void odd_cell_general(const StepArgs& a, const BlockG
 // and one 32-bit lane offset each, computed once: the cell gathers f_i where it later
 // scatters f*_opp(i) (slot opp(i) of x - c_i, or its own slot i where that is beyond an
 // edge or a link wall). Needs the populations within 4 GB (kLinearOddBytes is less).
-template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, int POLICY>
+// Its stores are ordinary ones, whatever the policy: the lines that two lanes' shifted
+// rows write in parts merge in the caches. PLAIN (policy 2): so are its loads.
+template<typename S, int DYN, bool TAGS, bool STATS, bool FORCED, bool PLAIN>
 __global__ void __launch_bounds__(512) bulk_odd_linear(StepArgs a) {
     using T = typename Store<S>::T;
-    constexpr bool PLAIN = POLICY == 2;
     const uint32_t wg = blockIdx.x;
     const int b = a.evenBlock ? (int)a.evenBlock[wg] : 0;
     const BlockGeom g = a.blocks[b];
@@ -670,10 +671,7 @@ __global__ void __launch_bounds__(512) bulk_odd_linear(StepArgs a) {
             for (int i = 0; i < 19; ++i) fc[i] = ld<S, PLAIN>(at(f, off[i]));
             collide_cell<S, DYN, STATS, FORCED, false>(a, g, cell, tag, in_bulk(g, x, y, z), fc, st, wall, wf);
 #pragma unroll
-            for (int i = 0; i < 19; ++i) {
-                if constexpr (POLICY >= 1) Store<S>::store_raw_cached(at(f, off[opp(i)]), Store<S>::to_raw(fc[i]));
-                else Store<S>::store(at(f, off[opp(i)]), fc[i]);
-            }
+            for (int i = 0; i < 19; ++i) Store<S>::store_raw_cached(at(f, off[opp(i)]), Store<S>::to_raw(fc[i]));
         }
     }
     store_bulk_stats<STATS, FORCED>(st, wf, a.partials, wg, a.walls);

@@ -112,8 +112,8 @@ int launchStepTyped(Lattice& L, bool odd, bool stats, const Recording* record) {
             const dim3 eg((unsigned)L.nEven), eb(kEvenThreads);
 #define PLBAMD_OD(TG, ST, FO)                                                                                       \
     do {                                                                                                            \
-        if (L.policy == 2) hipLaunchKernelGGL((bulk_odd_linear<S, DYN, TG, ST, FO, 2>), eg, eb, 0, L.stream, a);    \
-        else hipLaunchKernelGGL((bulk_odd_linear<S, DYN, TG, ST, FO, 1>), eg, eb, 0, L.stream, a);                  \
+        if (L.policy == 2) hipLaunchKernelGGL((bulk_odd_linear<S, DYN, TG, ST, FO, true>), eg, eb, 0, L.stream, a); \
+        else hipLaunchKernelGGL((bulk_odd_linear<S, DYN, TG, ST, FO, false>), eg, eb, 0, L.stream, a);              \
     } while (0)
 #define PLBAMD_OD_F(TG, ST) do { if (forced) PLBAMD_OD(TG, ST, true); else PLBAMD_OD(TG, ST, false); } while (0)
 #define PLBAMD_OD_S(TG) do { if (stats) PLBAMD_OD_F(TG, true); else PLBAMD_OD_F(TG, false); } while (0)
