@@ -62,9 +62,7 @@ std::shared_ptr<HostSlots> hostSlots(Lattice& L) {
         if (!s) {
             s = std::make_shared<HostSlots>();
             s->device = L.device;
-            bool ok = hipHostMalloc((void**)&s->pinned, HostSlots::kSlots * HostSlots::kBytes, hipHostMallocDefault) == hipSuccess;
-            for (hipStream_t& q : s->stream) ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
-            if (!ok) {
+            if (hipHostMalloc((void**)&s->pinned, HostSlots::kSlots * HostSlots::kBytes, hipHostMallocDefault) != hipSuccess) {
                 (void)hipGetLastError();
                 L.noPinned = true;
                 return nullptr;

@@ -8,7 +8,7 @@
 // chunks between slots and the caller's arrays: the populations of 128^3 FP64
 // cells (319 MB) come down in 7.4 ms instead of 34.8 and go up in 6.0 instead of
 // 19.1, their density and velocity (67 MB) in 2.0 instead of 7.8. Only uploads of
-// 3 to 48 MB take memory on the device (kCopiedUploadMin).
+// 0.75 to 72 MB take memory on the device (kCopiedUploadMin).
 #ifndef PALABOS_AMD_HOSTIO_H
 #define PALABOS_AMD_HOSTIO_H
 
@@ -70,11 +70,12 @@ std::shared_ptr<HostSlots> hostSlots(Lattice& L);
 // smaller ones in chunks on the calling thread: helper threads take the arrays' lines
 // into other cores' caches, and a program that writes them anew pays for it (density and
 // velocity rewritten, then uploaded, us: 8.4 MB copied 390, by eight threads 520-870; 16.8 MB
-// 690, 1490-1670; 67 MB 4190, 4530-5300; from new arrays each time 2.1 MB 315, 530-800, 16.8
-// MB 2000, 4930). Above, the threads win (populations of 80 / 319 / 638 MB left as they are
-// 3280 -> 1590, 11.3 -> 5.8 ms, 22.0 -> 11.5; rewritten in place 5300 -> 4800-6250, 19.8 -> 17-19
-// ms, 39 -> 33).
-constexpr uint64_t kCopiedUploadMin = 3u << 20, kCopiedUploadMax = 72u << 20;
+// 690, 1490-1670; 67 MB 4190, 4530-5300; from new arrays each time 2.1 MB 335, 530-800, 16.8
+// MB 2000, 4930). Below, a chunk is the faster way (populations of 0.6 / 1.2 / 2.5 MB
+// copied 51 / 87 / 151, in chunks 46 / 95 / 168). Above, the threads win (populations of 80 /
+// 319 / 638 MB left as they are 3280 -> 1590, 11.3 -> 5.8 ms, 22.0 -> 11.5; rewritten in place
+// 5300 -> 4800-6250, 19.8 -> 17-19 ms, 39 -> 33).
+constexpr uint64_t kCopiedUploadMin = 768u << 10, kCopiedUploadMax = 72u << 20;
 
 // One host array over a box, `perCell` bytes a cell in C order (host null: none).
 struct HostPart {
@@ -119,11 +120,15 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
     if (up && total > kCopiedUploadMin && total < kCopiedUploadMax) {
         DeviceBuffers buf;
         void* dev[4] = {};
-        if (char* at = static_cast<char*>(buf.get(total + 256 * nParts))) {   // one allocation: each costs 30 us and more
+        auto padded = [&](int p) { return parts[p].host ? (boxCells(b) * parts[p].perCell + 15) / 16 * 16 : 0; };
+        size_t bytes = 0;
+        for (int p = 0; p < nParts; ++p) bytes += padded(p);
+        // one allocation (each costs 30 us and more) and no larger than the arrays (64 MiB
+        // and some bytes take 270 us longer than 64 MiB)
+        if (char* at = static_cast<char*>(buf.get(bytes))) {
             for (int p = 0; p < nParts; ++p) {
-                if (!parts[p].host) continue;
-                dev[p] = at;
-                at += (boxCells(b) * parts[p].perCell + 255) / 256 * 256;
+                dev[p] = parts[p].host ? at : nullptr;
+                at += padded(p);
             }
             hipError_t err = hipSuccess;
             for (int p = 0; p < nParts && err == hipSuccess; ++p)
@@ -168,7 +173,14 @@ int hostTransfer(Lattice& L, const plbamd_box& b, const HostPart* parts, int nPa
             std::optional<HostSlots::Use> use;
             if (slots) use.emplace(*slots);
             char* const slot = slots ? slots->slot(use->k) : pageable.get();
-            const hipStream_t stream = slots ? slots->stream[use->k] : L.stream;
+            hipStream_t stream = L.stream;
+            if (slots) {
+                // a slot's stream comes with its first use
+                hipStream_t& own = slots->stream[use->k];
+                const hipError_t made = own ? hipSuccess : hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+                if (made != hipSuccess) { error.store((int)made); return; }
+                stream = own;
+            }
             const uint64_t ix = c / (nY * nZ), iy = c / nZ % nY, iz = c % nZ;
             plbamd_box k;
             k.x0 = b.x0 + (int)(ix * sx); k.x1 = std::min<int>(b.x1, k.x0 + (int)sx - 1);
