@@ -22,9 +22,10 @@ def lattice(n, storage="f64", periodic=True):
 
 
 def hip():
-    """The HIP runtime that the library runs on."""
+    """The HIP runtime that the library runs on: torch brings one of its own, which is another if it came later."""
     with open("/proc/self/maps") as maps:
-        path = next(line.split()[-1] for line in maps if "libamdhip64" in line)
+        paths = {line.split()[-1] for line in maps if "libamdhip64" in line}
+    path = next((p for p in sorted(paths) if "/torch/" not in p), min(paths))
     return ctypes.CDLL(path)
 
 
