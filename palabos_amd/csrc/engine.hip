@@ -989,8 +989,10 @@ static int prepareSteps(Lattice& L, int nsteps, bool& fused, std::unique_lock<st
     use = std::unique_lock<std::mutex>(L.spareMutex);
     const bool had = L.spare && (L.dInfo || !(L.dTags || !(L.geom[0].px && L.geom[0].py && L.geom[0].pz)));
     fused = fusedReady(L);
-    if (fused && !had) PLBAMD_TRY(fusedDispatch(L, FUSED_PREPARE));
-    return PLBAMD_OK;
+    if (!fused || had) return PLBAMD_OK;
+    const int rc = fusedDispatch(L, FUSED_PREPARE);
+    if (rc) L.releaseTwoStep();   // tables that were not filled are not to be found by the next call
+    return rc;
 }
 
 static int queueSteps(Lattice& L, int nsteps, bool fused) {
